@@ -62,8 +62,8 @@ def screen():
 
 def algorithmic_flops_per_sample(A, B, th, chunks, npix_sample=512, seed=0):
     """Counts the per-sample FP64 operations of the kernels' own loops (the
-    walk along the grid with its direct evaluations, split into `chunks`
-    ranges per pixel as the launch does) on a seeded subset of the workload's
+    anchors' direct evaluations and the Taylor series along the grid, each
+    of its blocks in `chunks` parts as the launch has) on a seeded subset of the workload's
     pixels: CPU instantiation of the device source on an op-counting type,
     kgeo_amd/libkgeo_opcount.so."""
     path = os.path.join(ROOT, "kgeo_amd", "libkgeo_opcount.so")
@@ -637,12 +637,12 @@ def main():
     st = status.cpu().numpy()
     nonfinite = int(np.sum(st & 1))
 
-    chunks = int(lib.kgeo_sample_chunks(npix, NGEO))
+    chunks = 1  # parts per block at this size (pick_parts, kg_series_pass.hpp)
     flops_s, flops_setup, ops = algorithmic_flops_per_sample(A, B, th, chunks)
     achieved_tf = flops_s * samples / (samp_ms * 1e-3) / 1e12
     bytes_per_launch = 32.0 * samples
     hbm_gbs = bytes_per_launch / (samp_ms * 1e-3) / 1e9
-    roofline = {"bound": "valu-fp64", "kernel": "sample passes (kg_theta_* + kg_radial_*: heads, far, repair, walk, fixup)", "achieved": achieved_tf, "peak": FP64_PEAK_TFLOPS,
+    roofline = {"bound": "valu-fp64", "kernel": "sample passes (kg_theta_heads, kg_radial_heads, kg_series, kg_fixup)", "achieved": achieved_tf, "peak": FP64_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": achieved_tf / FP64_PEAK_TFLOPS,
                 "traffic": read_profile_value("traffic_bytes_per_launch"),
                 "flops_per_sample": flops_s, "algorithmic_bytes_per_launch": bytes_per_launch,
@@ -671,7 +671,7 @@ def main():
             "vs_baseline": None, "dtype": "f64", "data": "synthetic",
             "config": {"workload": "raytrace_ana 512x512 ngeo=500 (a=0.94, th_o=17 deg, r_o=1e4, "
                                    "alpha,beta in [-8,8]); writes r, theta, phi, t",
-                       "npix": npix, "ngeo": NGEO, "parallelism": "single GPU, pixels x sample chunks"},
+                       "npix": npix, "ngeo": NGEO, "parallelism": "single GPU, pixels x sample blocks"},
             "roofline": roofline, "cpu_baseline": cpu,
             "gpu_vs_cpu": (value / cpu["value"]) if cpu else None, "grad_images": grad, "polarized_image": image,
             "batch": batch,

@@ -247,7 +247,12 @@ template <class T> KG_INLINE T ellip_pi_amp(const LegendreBase<T>& L, const T& n
 template <class T, int NP> struct LegendreFam {
   T F, EmF;
   T Pi[NP];
+  T rho[NP];  // 1 - n sn^2, as the Pi took it
 };
+
+// A pole factor 1 - n sn^2 below this is worth forming without cancellation
+// (legendre_family, radial_state): at 1/64 the plain form has lost six bits.
+constexpr double kPoleNear = 1.0 / 64.0;
 
 template <class T, int NP>
 KG_INLINE void legendre_family(const Amp<T>& A, const T& m, const T& Kc, const T& EmKc, const T (&n)[NP],
@@ -260,7 +265,13 @@ KG_INLINE void legendre_family(const Amp<T>& A, const T& m, const T& Kc, const T
   L.y = 1.0 - m * s2;
   T rho[NP];
 #pragma unroll
-  for (int i = 0; i < NP; ++i) rho[i] = 1.0 - n[i] * s2;
+  for (int i = 0; i < NP; ++i) {
+    rho[i] = 1.0 - n[i] * s2;
+    // the polar integral next to the axis (n near 1, sn near +-1): 1 - n is
+    // exact there and n cn^2 small, so no digits cancel
+    if (NP == 1 && kfabs(val(rho[i])) < kPoleNear) rho[i] = (1.0 - n[i]) + n[i] * L.x;
+    out.rho[i] = rho[i];
+  }
   CarlsonSet<T, NP> cs;
   carlson_family(L.x, L.y, rho, want_rd, cs);
   L.rf = cs.rf;
@@ -336,6 +347,7 @@ enum : int { THK_NONE = 0, THK_ORD = 1, THK_ORD_K0 = 2, THK_VORT = 3 };
 
 template <class T> struct ThetaConsts {
   T v[TH_NSLOT];
+  T u0;          // d cos(theta)/dtau at the observer (the series' start, kg_series.hpp)
   int kind;
   int eta_zero;  // eta == 0: ordinary branch only if some eta>0 in the image
 };
@@ -346,6 +358,7 @@ KG_INLINE void theta_consts(const RayScalars<T>& c, const PixelSetup<T>& px, boo
 #pragma clang fp contract(off)
 #endif
   for (int i = 0; i < TH_NSLOT; ++i) tc.v[i] = T(0.0);
+  tc.u0 = T(0.0);
   tc.kind = THK_NONE;
   tc.eta_zero = (val(px.eta) == 0.0);
   const T& up = px.up;
@@ -380,6 +393,8 @@ KG_INLINE void theta_consts(const RayScalars<T>& c, const PixelSetup<T>& px, boo
     tc.v[TH_B] = 2.0 * up * pref;   // G_t prefactor
     tc.v[TH_C] = -tc.v[TH_B] / (2.0 * k);  // G_t = TH_C (E - F) - sGt for k != 0
     tc.kind = (val(k) == 0.0) ? THK_ORD_K0 : THK_ORD;
+    // cos(theta) = TH_A sn: from the same rounded amplitude as sG
+    tc.u0 = (s * ksqrt(up)) * w * (Ao.c * ksqrt(Lo.y));
     if (do_phi_t) {
       T EmKk = ellip_EmK(k);
       T Pic = ellip_pi_complete(up, k, Kk);
@@ -423,6 +438,7 @@ KG_INLINE void theta_consts(const RayScalars<T>& c, const PixelSetup<T>& px, boo
     tc.v[TH_C] = prefC;
     tc.v[TH_h] = T(c.h);
     tc.kind = THK_VORT;
+    tc.u0 = s * tc.v[TH_w] * (up - um) * (Ao.s * Ao.c * ksqrt(Lo.y)) / kfabs(c.cos_th);
     if (do_phi_t) {
       T EmKk = ellip_EmK(k);
       T Pic = ellip_pi_complete(upm, k, Kk);
@@ -878,6 +894,17 @@ template <class T> KG_INLINE T log_ratio(const T& a, const T& b) {
   return klog1p(arg);
 }
 
+// log_ratio(a, b) where D = b^2 - a^2 is known better than b - |a|: next to
+// a removable singularity of a block, whose log and third-kind integral
+// cancel, both from the same D.
+template <class T> KG_INLINE T log_ratio_near(const T& a, const T& b, const T& D) {
+  const bool flip = val(a) * val(b) < 0.0;
+  const T a1 = flip ? -a : a;
+  const T diff = D / (b + a1);  // b - a1
+  const T lg = klog1p(val(diff) * val(b) > 0.0 ? 2.0 * a1 / diff : -(2.0 * b / diff));
+  return flip ? -lg : lg;
+}
+
 template <class T> KG_INLINE T radial_arg(const RadialConsts<T>& rc, const T& tau) {
   return rc.v[R_U0] - rc.v[R_Xs] * tau;
 }
@@ -939,6 +966,17 @@ KG_INLINE void radial_state(const RadialConsts<T>& rc, const JacobiLadder<T>& la
       if (rcase == 3) block_log_args<T, 3>(rc, i, st.s, st.d, a, b);
       else block_log_args<T, 4>(rc, i, st.s, st.d, a, b);
       st.lg[i] = log_ratio(a, b);
+      // R1's 1 + al cn (S1's cn + g sn) has its pole on one of the two sides
+      // where 1 - n sn^2 vanishes (r at a horizon or at infinity); on the
+      // other the block is regular and the log and Pi cancel (up to 4e-10
+      // lost at a sample next to it before D was taken from Pi's own factor)
+      if (kfabs(val(fam.rho[i])) < kPoleNear) {
+        const T& p1 = v[(rcase == 3 ? C3_p0 : C4_q0) + i];
+        const T D = rcase == 3 ? p1 * p1 * fam.rho[i] : -(k * p1 * p1 / nn[i]) * fam.rho[i];
+        const double side = rcase == 3 ? val(v[C3_al0 + i]) * val(st.c)
+                                       : val(v[C4_g0 + i]) * val(st.s) * val(st.c);
+        if (side > 0.0) st.lg[i] = log_ratio_near(a, b, D);
+      }
     }
   }
 }
@@ -1201,6 +1239,10 @@ enum PlanSlot : int {
   PL_THK,    // theta kind
   PL_ETA0,   // eta == 0
   PL_RCASE,  // r_integrate case
+  PL_QA,     // the radial quartic r^4 + A r^2 + B r + C (the series, kg_series.hpp)
+  PL_QB,
+  PL_QC,
+  PL_U0,     // d cos(theta)/dtau at the observer
   PL_N
 };
 
@@ -1212,11 +1254,30 @@ template <class T> struct PixelConsts {
   T stop;
 };
 
+// The radial quartic r^4 + A r^2 + B r + C = (r^2 + 2 z r + p)(r^2 - 2 z r + q)
+// of the rounded roots r = -z -+ .., z -+ ..: the resolvent loses digits
+// where its cubic's linear term vanishes, and every sample of the reference
+// inherits the roots' rounding, so the series does too.
+template <class T> KG_INLINE void radial_quartic(const PixelSetup<T>& px, T& A, T& B, T& C) {
+#if defined(__clang__)
+#pragma clang fp contract(off)
+#endif
+  const T z = 0.5 * (px.rr[2] + px.rr[3]);
+  const T p = px.rr[0] * px.rr[1] - px.ri[0] * px.ri[1];
+  const T q = px.rr[2] * px.rr[3] - px.ri[2] * px.ri[3];
+  A = p + q - 4.0 * (z * z);
+  B = 2.0 * z * (q - p);
+  C = p * q;
+}
+
 // The plan in two parts: theta, lambda and the grid stop; the radial
 // constants (PL_R .. PL_R + R_NSLOT - 1 and PL_RCASE).
-KG_INLINE void plan_pack_theta(const ThetaConsts<double>& tc, double lam, double stop, double* plan) {
+KG_INLINE void plan_pack_theta(const ThetaConsts<double>& tc, const PixelSetup<double>& px, double stop,
+                               double* plan) {
   for (int i = 0; i < TH_NSLOT; ++i) plan[PL_TH + i] = tc.v[i];
-  plan[PL_LAM] = lam;
+  plan[PL_LAM] = px.lam;
+  radial_quartic(px, plan[PL_QA], plan[PL_QB], plan[PL_QC]);
+  plan[PL_U0] = tc.u0;
   plan[PL_STOP] = stop;
   plan[PL_THK] = static_cast<double>(tc.kind);
   plan[PL_ETA0] = static_cast<double>(tc.eta_zero);
@@ -1229,9 +1290,9 @@ KG_INLINE void plan_pack_radial(const RadialConsts<double>& rc, double* plan) {
 
 KG_INLINE bool plan_slot_radial(int s) { return (s >= PL_R && s < PL_R + R_NSLOT) || s == PL_RCASE; }
 
-KG_INLINE void plan_pack(const ThetaConsts<double>& tc, const RadialConsts<double>& rc, double lam, double stop,
-                         double* plan) {
-  plan_pack_theta(tc, lam, stop, plan);
+KG_INLINE void plan_pack(const ThetaConsts<double>& tc, const RadialConsts<double>& rc, const PixelSetup<double>& px,
+                         double stop, double* plan) {
+  plan_pack_theta(tc, px, stop, plan);
   plan_pack_radial(rc, plan);
 }
 
@@ -1275,7 +1336,7 @@ KG_INLINE PixelSetup<double> plan_pixel(const RayScalars<double>& c, double alph
   RadialConsts<double> rc;
   theta_consts(c, px, do_phi_t, tc);
   radial_consts(c, px, do_phi_t, rc);
-  plan_pack(tc, rc, px.lam, c.maxtaufrac * px.tau_tot, plan);
+  plan_pack(tc, rc, px, c.maxtaufrac * px.tau_tot, plan);
   return px;
 }
 
@@ -1286,7 +1347,7 @@ KG_INLINE PixelSetup<double> plan_pixel_theta(const RayScalars<double>& c, doubl
   pixel_setup(c, alpha, beta, px);
   ThetaConsts<double> tc;
   theta_consts(c, px, do_phi_t, tc);
-  plan_pack_theta(tc, px.lam, c.maxtaufrac * px.tau_tot, plan);
+  plan_pack_theta(tc, px, c.maxtaufrac * px.tau_tot, plan);
   return px;
 }
 

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "kg_sample.hpp"
+#include "kg_series_pass.hpp"
 
 namespace kg {
 
@@ -96,6 +97,44 @@ void three_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, c
     for (int64_t sg = 0; sg < kFixupSpan; ++sg)
       st[i] |= radial_fixup_sample<DO_PHI_T, T>(c, plan, npix, i, gflags, o, i, j, w, sg);
   }
+}
+
+// The series passes over all pixels, in the kernels' order: heads of both
+// coordinates, the blocks in `parts` parts each, then the fixups of theta and r over one queue.
+// nfix[0] receives the queue's length (-1 past the kernels' capacity).
+template <class T>
+void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, const SampleOut& o, int64_t parts,
+                   uint32_t* st, int64_t* nfix) {
+  const int64_t npix = o.npix, G = o.ngeo, nb = series_blocks(G);
+  std::vector<double> trec(static_cast<size_t>(nb) * kThSFields * npix), rrec(static_cast<size_t>(nb) * kRSFields * npix);
+  const Records rth{trec.data(), npix, 0}, rr{rrec.data(), npix, 0};
+  std::vector<uint64_t> items;
+  HostPush push{&items};
+  for (int64_t i = 0; i < npix; ++i)
+    for (int64_t hd = 0; hd < nb; ++hd) {
+      st[i] |= series_theta_head_pixel<T>(plan, npix, i, gflags, o, i, hd, nb, rth);
+      st[i] |= series_radial_head_pixel<T>(plan, npix, i, gflags, o, i, hd, nb, val(c.r_o), rr);
+    }
+  for (int64_t i = 0; i < npix; ++i)
+    for (int64_t u = 0; u < nb * parts; ++u) {
+      const int64_t b = u / parts, q = u % parts;
+      LocalSlots<T> slots;
+      st[i] |= o.sig ? series_block_pixel<true, false, LocalSlots<T>, HostPush, T>(c, plan, npix, i, gflags, o, i, true, b, nb, q, parts, rth, rr, slots, push)
+                     : series_block_pixel<false, false, LocalSlots<T>, HostPush, T>(c, plan, npix, i, gflags, o, i, true, b, nb, q, parts, rth, rr, slots, push);
+    }
+  const size_t cap = static_cast<size_t>(npix) * static_cast<size_t>(fixup_items(G));
+  nfix[0] = items.size() <= cap ? static_cast<int64_t>(items.size()) : -1;
+  nfix[1] = nfix[0];
+  nfix[2] = 0;
+  for (int part = 0; part < 2; ++part)
+    for (uint64_t e : items) {
+      int64_t i, j;
+      bool w;
+      unpack_host_item(e, i, j, w);
+      for (int64_t sg = 0; sg < kFixupSpan; ++sg)
+        st[i] |= part == 0 ? theta_fixup_sample<true, T>(plan, npix, i, gflags, o, i, j, w, sg)
+                           : radial_fixup_sample<true, T>(c, plan, npix, i, gflags, o, i, j, w, sg);
+    }
 }
 
 }  // namespace kg

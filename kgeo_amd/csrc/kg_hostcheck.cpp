@@ -112,8 +112,11 @@ void kgh_setup(const double* sc, const double* alpha, const double* beta, int64_
 // ([PL_N][npix] slot-major), image-wide flags and per-pixel sample code
 // (kg_sample.hpp) as kg_setup and the sample kernels, with ngeo split into
 // `chunks` contiguous ranges per pixel as the kernels' grid does.
-//   passes = 3: the anchor / walk / fixup passes (the kernels' path for the
-//               linspace grid with ngeo > 2); nfix[3] (optional) receives the
+//   passes = 4: the heads / series / fixup passes with each block in `chunks` parts,
+//               per ray (the kernels' path for the linspace grid with ngeo >
+//               2); nfix (optional) receives the fixup queue's length;
+//   passes = 3: the anchor / walk / fixup passes (the same samples by the
+//               addition theorems); nfix[3] (optional) receives the
 //               theta and radial fixup-queue lengths and the radial repair
 //               items;
 //   passes = 1: one combined loop per coordinate (theta_pixel, radial_pixel:
@@ -147,9 +150,10 @@ void kgh_raytrace_passes(const double* sc, const double* alpha, const double* be
     o.t = nullptr;
     o.ph = nullptr;
   }
-  if (passes == 3 && !tau_in && G > 2) {
+  if ((passes == 3 || (passes == 4 && do_phi_t)) && !tau_in && G > 2) {
     int64_t nf[3] = {0, 0, 0};
-    if (do_phi_t) three_passes<true, double>(c, plan.data(), gflags, o, chunks, st.data(), nf);
+    if (passes == 4) series_passes<double>(c, plan.data(), gflags, o, chunks, st.data(), nf);
+    else if (do_phi_t) three_passes<true, double>(c, plan.data(), gflags, o, chunks, st.data(), nf);
     else three_passes<false, double>(c, plan.data(), gflags, o, chunks, st.data(), nf);
     if (nfix) {
       nfix[0] = nf[0];

@@ -71,10 +71,11 @@ extern "C" {
 int kgc_num_ops(void) { return kgcount::NOPS; }
 
 // Per-sample op counts summed over npix pixels x ngeo linspace samples, as
-// the sample kernels execute them: the anchor / walk / fixup passes
-// (kg_host_passes.hpp: direct evaluations at the step, the segment starts,
-// the last sample and from each refused step on; the walk elsewhere) with
-// ngeo split into `chunks` ranges per pixel as the kernels' grid does.
+// the sample kernels execute them: the heads / series / fixup passes
+// (kg_host_passes.hpp: direct evaluations at the block starts, the last
+// sample and where the series is refused; expansions and polynomials
+// elsewhere) with each block in `chunks` parts as the kernels' grid has.  Each ray takes its own steps here; a wave's 64 rays take the
+// smallest of theirs, so the kernels run more expansions than are counted.
 // Separately, the per-pixel setup counts.  sc as in kg_hostcheck.cpp.
 void kgc_count(const double* sc, const double* alpha, const double* beta, int64_t npix, int64_t ngeo, int chunks,
                uint64_t* per_sample_ops, uint64_t* setup_ops) {
@@ -111,7 +112,7 @@ void kgc_count(const double* sc, const double* alpha, const double* beta, int64_
   std::memset(kgcount::g_ops, 0, sizeof(kgcount::g_ops));
   std::vector<uint32_t> st(static_cast<size_t>(npix), 0u);
   int64_t nfix[3];
-  three_passes<true, CD>(cc, plan.data(), gflags, o, chunks, st.data(), nfix);
+  series_passes<CD>(cc, plan.data(), gflags, o, chunks, st.data(), nfix);
   for (int q = 0; q < kgcount::NOPS; ++q) samp_acc[q] += kgcount::g_ops[q];
   for (int q = 0; q < kgcount::NOPS; ++q) {
     per_sample_ops[q] = samp_acc[q];

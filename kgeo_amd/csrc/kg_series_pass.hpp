@@ -1,0 +1,432 @@
+// The sample passes of the linspace grid by Taylor series (kg_series.hpp),
+// shared by the plain kernels (kgeo_raytrace.hip) and the batched survey
+// (kgeo_batch.hip).
+//
+// A ray's grid is split into two blocks of consecutive samples.  The first
+// starts from the observer, whose state is known in closed form, the second
+// from an anchor, a direct evaluation (Landen ladder, Carlson duplications)
+// of its first sample:
+//   heads   one lane per (pixel, head): the anchors, and the last grid sample
+//           (at 1e-10 of the horizon for captured rays, where only the
+//           direct formulas reproduce the reference's rounding);
+//   series  one lane per (pixel, block, part): samples of the block;
+//   fixup   one lane per (queued range, sample): direct evaluation of what
+//           the series leaves (kg_sample.hpp).
+// The anchor keeps every sample within half a ray of the reference's own
+// arithmetic: near the critical curve a difference in the last bit grows
+// along the ray (by 1/d over a ray at distance d from the curve, 1/sqrt(d)
+// over half of one), in the series and in the closed formulas alike.
+//
+// Where the rays are too few to fill the chip, the samples of a block are
+// split into parts, one lane each, which all run the block's expansions up to
+// their own samples' end: the results do not depend on the parts, nor on how
+// many rays are sampled together.  (More blocks instead of parts would run
+// fewer expansions per lane, but more anchors, and would let near-critical
+// rays change by 1e-9 with the number of pixels.)
+//
+// The lanes of a wave take their steps together (the smallest any lane
+// needs), so a sample index is uniform across the wave and every store is
+// one contiguous row; a lane that would hold the others to steps below
+// 1/kSeriesMinStep of its block leaves the rest of it to the fixup pass.
+// Blocks start at multiples of kFixupSpan, so a queued range lies in one.
+
+#pragma once
+
+#include "kg_sample.hpp"
+#include "kg_series.hpp"
+
+namespace kg {
+
+constexpr int kSeriesBlocks = 2;
+constexpr int kSeriesMaxParts = 8;
+constexpr double kSeriesMinStep = 128.0;
+
+#if defined(__HIPCC__)
+// A lane's column of its wave's LDS (LocalSlots).  fresh() keeps the loads
+// that follow it in their loop iteration: hoisted, the constants would hold
+// registers through the sample loops.
+struct LdsSlots {
+  double (*s)[64];
+  int lane;
+  __device__ void set(int q, double x) { s[q][lane] = x; }
+  __device__ double operator()(int q) const { return s[q][lane]; }
+  __device__ void fresh() const { asm volatile("" ::: "memory"); }
+};
+#endif
+
+// First sample of block b of nb (nb: the end, the last grid sample).
+KG_INLINE int64_t series_start(int64_t ngeo, int64_t b, int64_t nb) {
+  const int64_t last = ngeo - 1;
+  return b >= nb ? last : last * b / nb / kFixupSpan * kFixupSpan;
+}
+
+// Blocks per ray: two, as long as each holds kFixupSpan samples.  (One block
+// over a whole ray near the critical curve: 1.2e-10 of r at 0.94, 17 deg, 500
+// samples, against 6e-12 in two.)
+KG_INLINE int64_t series_blocks(int64_t ngeo) { return ngeo - 1 >= kSeriesBlocks * kFixupSpan ? kSeriesBlocks : 1; }
+
+// First sample of part q of `parts` of a block's samples js .. je - 1.
+KG_INLINE int64_t series_part(int64_t js, int64_t je, int64_t q, int64_t parts) {
+  return q <= 0 ? js : (q >= parts ? je : (js + (je - js) * q / parts) / kFixupSpan * kFixupSpan);
+}
+
+// Parts per block for npix rays (all images') sampled together on grids of
+// ngeo samples: enough that 2^17 (ray, part) lanes fill the chip's 2048 places
+// at two waves per SIMD.  More cost their expansions again.  Measured with 1,
+// 2, 4 and 8 parts (ms): 1000 rays x 250 samples 0.477, 0.409, 0.374, 0.361;
+// 64 x 64 x 100 0.456, 0.430, 0.425, 0.420; 217 x 301 x 333 0.94, 0.81, 0.86,
+// 1.04; 512 x 512 x 500 2.28, 2.44, 2.97, 3.97; a survey of 16 images of
+// 192 x 192 rays and 128 .. 512 samples 9.7, 10.4, 10.4, 10.4.
+inline int64_t pick_parts(int64_t npix, int64_t ngeo) {
+  int64_t want = npix > 0 ? (1LL << 17) / npix : 1;
+  const int64_t most = ngeo / series_blocks(ngeo) / kFixupSpan;
+  if (want > kSeriesMaxParts) want = kSeriesMaxParts;
+  if (want > most) want = most;
+  return want < 1 ? 1 : want;
+}
+
+// Anchor records: theta (c, dc/dtau, G_phi, G_t), radial (r, I_+, I_-, I_1, I_2, dw/dtau);
+// record 0 the last sample, record b the first sample of block b.
+constexpr int kThSFields = 4;
+constexpr int kRSFields = 6;
+
+// Smallest x over the wave's lanes (all 64 must call), x >= 0.
+KG_INLINE float wave_min(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  int v = __float_as_int(x);  // ordered as integers for x >= 0
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) {
+    const int o = __shfl_xor(v, s);
+    v = o < v ? o : v;
+  }
+  return __int_as_float(__builtin_amdgcn_readfirstlane(v));
+#else
+  return x;
+#endif
+}
+
+// d cos(theta)/dtau from the Jacobi state at a sample (theta_out's cos theta).
+template <class T, int KIND>
+KG_INLINE void theta_motion(const ThetaConsts<T>& tc, const ThState<T>& st, T& c, T& u) {
+  const T* v = tc.v;
+  if (KIND == THK_VORT) {
+    c = v[TH_h] * ksqrt(v[TH_A] + v[TH_B] * (st.s * st.s));
+    u = -(v[TH_w] * v[TH_B]) * (st.s * st.c * st.d) / c;
+  } else {
+    c = v[TH_A] * st.s;
+    u = -(v[TH_w] * v[TH_A]) * (st.c * st.d);
+  }
+}
+
+// d(1/r)/dtau from the Jacobi state at a sample (radial_out's r).
+template <class T, int CASE> KG_INLINE T radial_motion(const RadialConsts<T>& rc, const RState<T>& st) {
+  const T* v = rc.v;
+  const T& Xs = v[R_Xs];
+  if (CASE == 4) {
+    const T& g0 = v[C4_g0];
+    const T den = st.c + g0 * st.s;
+    const T num = -v[C4_a2] * (g0 * st.c - st.s) - v[C4_b1] * den;  // r den
+    return v[C4_a2] * Xs * st.d * (1.0 + g0 * g0) / (num * num);
+  }
+  if (CASE == 3) {
+    const T &AA = v[C3_AA], &BB = v[C3_BB], &r1 = v[C3_rr1], &r2 = v[C3_rr2];
+    const T num = (BB * r2 - AA * r1) + (BB * r2 + AA * r1) * st.c;
+    return 2.0 * AA * BB * (r2 - r1) * Xs * (st.s * st.d) / (num * num);
+  }
+  const T num = v[C2_rr4] * v[C2_rr31] - v[C2_rr3] * v[C2_rr41] * (st.s * st.s);
+  return 2.0 * Xs * v[C2_rr41] * v[C2_rr31] * v[C2_rr43] * (st.s * st.c * st.d) / (num * num);
+}
+
+// Theta head hd (0 the last sample, b the anchor of block b) of output pixel
+// i: theta and the parked G_phi, G_t of its sample, and an anchor's motion.
+template <class T, int KIND>
+KG_INLINE bool series_theta_head(const SampleOut& o, const ThetaConsts<T>& tc, const JacobiLadder<T>& lad, int64_t i,
+                                 int64_t hd, int64_t nb, double stop, const Records& rt, int64_t col) {
+  const int64_t j = hd == 0 ? o.ngeo - 1 : series_start(o.ngeo, hd, nb);
+  WalkStep<T, 1> w;
+  theta_init(tc, w);
+  const double tau = mino_tau(j, o.ngeo, stop, false);
+  const T arg = theta_arg(tc, T(tau));
+  ThState<T> ts;
+  WalkState<T, 1> st;
+  theta_direct<T, KIND, true>(tc, lad, w, arg, ts, st);
+  T th = T(0.0), Gph = T(0.0), Gt = T(0.0);
+  theta_out<T, KIND>(tc, arg, ts, true, th, Gph, Gt);
+  if (hd > 0) {
+    T c, u;
+    theta_motion<T, KIND>(tc, ts, c, u);
+    // next to a singularity of Pi (walk_enter) the anchor is not used
+    if (!kfinite(val(st.P[0]))) c = T(NAN);
+    *rt.at(hd, kThSFields, 0, col) = val(c);
+    *rt.at(hd, kThSFields, 1, col) = val(u);
+    *rt.at(hd, kThSFields, 2, col) = val(Gph);
+    *rt.at(hd, kThSFields, 3, col) = val(Gt);
+  }
+  return theta_store<T, true>(o, j * o.npix + i, tau, th, Gph, Gt);
+}
+
+template <class T = double>
+KG_INLINE uint32_t series_theta_head_pixel(const double* __restrict__ plan, int64_t stride, int64_t p, uint32_t gflags,
+                                           const SampleOut& o, int64_t i, int64_t hd, int64_t nb, const Records& rt) {
+  ThetaConsts<T> tc;
+  const ThetaPick tp = theta_pick(plan, stride, p, gflags, o, tc);
+  if (!tp.walk) return 0u;
+  JacobiLadder<T> lad;
+  jacobi_ladder(tc.v[TH_mp], lad);
+  bool bad;
+  switch (tp.kind) {
+    case THK_ORD: bad = series_theta_head<T, THK_ORD>(o, tc, lad, i, hd, nb, tp.stop, rt, p); break;
+    case THK_ORD_K0: bad = series_theta_head<T, THK_ORD_K0>(o, tc, lad, i, hd, nb, tp.stop, rt, p); break;
+    default: bad = series_theta_head<T, THK_VORT>(o, tc, lad, i, hd, nb, tp.stop, rt, p); break;
+  }
+  return loop_status(bad, lad);
+}
+
+// Radial head hd: the sample's r and radial integrals, and an anchor's motion.
+// Head 0 also stores r at sample 0, from the closed form (an ulp of its
+// argument is up to 6e-11 of r_o for rays near the critical curve, where the
+// plan's rounded roots place the observer; the closed form keeps sample 0
+// with the samples it gives next to it).
+template <class T, int CASE>
+KG_INLINE uint32_t series_radial_head(const double* __restrict__ plan, int64_t stride, int64_t p, const SampleOut& o,
+                                      int64_t i, int64_t hd, int64_t nb, const Records& rt) {
+  RadialConsts<T> rc;
+  T lam;
+  double stop;
+  radial_pick(plan, stride, p, rc, lam, stop);
+  JacobiLadder<T> lad;
+  jacobi_ladder(rc.v[R_k], lad);
+  const int64_t j = hd == 0 ? o.ngeo - 1 : series_start(o.ngeo, hd, nb);
+  WalkStep<T, 3> w;
+  radial_init<T, CASE>(rc, w);
+  const double tau = mino_tau(j, o.ngeo, stop, false);
+  const T dv = rc.v[R_Xs] * tau;
+  const T X = rc.v[R_U0] - dv;
+  RState<T> rs;
+  WalkState<T, 3> st;
+  T lb[3];
+  radial_direct<T, CASE, true>(rc, lad, w, X, dv, rs, st, lb);
+  const RadialOut<T> ro = radial_out<T, CASE>(rc, T(tau), rs, true);
+  T v = T(0.0);
+  if (hd == 0 && o.r && o.ngeo > 1) {
+    RState<T> r0;
+    r0.s = rc.v[R_sn0];
+    r0.c = rc.v[R_cn0];
+    r0.d = rc.v[R_dn0];
+    o.r[i] = val(radial_out<T, CASE>(rc, T(0.0), r0, false).r);
+  }
+  if (hd > 0) {
+    v = radial_motion<T, CASE>(rc, rs);
+    // next to a singularity of an integral (walk_enter, block_log_enter)
+    // the closed formulas lose digits: the anchor is not used
+    bool ok = kfinite(val(v));
+    // below MINSPIN case 3 has no third-kind part of I_-
+    const int np = (CASE == 3 && val(rc.v[C3_hasm]) == 0.0) ? 2 : 3;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) ok = ok & ((q >= np) | (kfinite(val(st.P[q])) & kfinite(val(lb[q]))));
+    if (!ok) v = T(NAN);
+  }
+  *rt.at(hd, kRSFields, 0, p) = val(ro.r);
+  *rt.at(hd, kRSFields, 1, p) = val(ro.Ip);
+  *rt.at(hd, kRSFields, 2, p) = val(ro.Im);
+  *rt.at(hd, kRSFields, 3, p) = val(ro.I1);
+  *rt.at(hd, kRSFields, 4, p) = val(ro.I2);
+  *rt.at(hd, kRSFields, 5, p) = val(v);
+  return loop_status(false, lad);
+}
+
+template <class T = double>
+KG_INLINE uint32_t series_radial_head_pixel(const double* __restrict__ plan, int64_t stride, int64_t p,
+                                            uint32_t gflags, const SampleOut& o, int64_t i, int64_t hd,
+                                            int64_t nb, double r_o, const Records& rt) {
+  const int rcase = static_cast<int>(plan[static_cast<int64_t>(PL_RCASE) * stride + p]);
+  const double m = plan[static_cast<int64_t>(PL_R + R_k) * stride + p];
+  if (!radial_walks(o, gflags, m)) {
+    // its blocks leave every sample to the fixup pass, but an early block 0
+    // (series_block_pixel), which cannot know, still writes its own
+    if (hd == 0 && o.r) o.r[i] = r_o;
+    return 0u;
+  }
+  switch (rcase) {
+    case 4: return series_radial_head<T, 4>(plan, stride, p, o, i, hd, nb, rt);
+    case 3: return series_radial_head<T, 3>(plan, stride, p, o, i, hd, nb, rt);
+    default: return series_radial_head<T, 2>(plan, stride, p, o, i, hd, nb, rt);
+  }
+}
+
+// A head's sample: r and the combination of its radial record with the
+// theta pass's parked G_phi, G_t (as radial_store).
+template <class T>
+KG_INLINE bool series_head_store(const SampleOut& o, const CombineConsts<T>& cmb, int64_t idx, double tau,
+                                 const Records& rr, int64_t hd, int64_t col) {
+  RadialOut<T> ro;
+  ro.r = T(*rr.at(hd, kRSFields, 0, col));
+  ro.Ip = T(*rr.at(hd, kRSFields, 1, col));
+  ro.Im = T(*rr.at(hd, kRSFields, 2, col));
+  ro.I1 = T(*rr.at(hd, kRSFields, 3, col));
+  ro.I2 = T(*rr.at(hd, kRSFields, 4, col));
+  return radial_store_g<T, true>(o, cmb, idx, tau, ro, T(o.ph[idx]), T(o.t[idx]));
+}
+
+// Part q of `parts` of block b of output pixel i (plan column p) by the
+// series.  All lanes of a wave call together; `in` is false for a lane without a pixel
+// (its i and p must be valid).  EARLY: block 0 of several, which reads nothing
+// of the plan's radial constants (kg_setup_radial may still be writing them)
+// and no record; not below MINSPIN.  Returns the status bits.
+template <bool SIG, bool EARLY, class Slots, class Push, class T = double>
+KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __restrict__ plan, int64_t stride,
+                                      int64_t p, uint32_t gflags, const SampleOut& o, int64_t i, bool in, int64_t b,
+                                      int64_t nb, int64_t q, int64_t parts, const Records& rth, const Records& rr,
+                                      Slots& k, Push& push) {
+  constexpr int P = kSeriesOrder;
+  const int64_t last = o.ngeo - 1;
+  const int64_t js = series_start(o.ngeo, b, nb), je = series_start(o.ngeo, b + 1, nb);
+  if (js >= je) {  // a grid of one sample; series_blocks gives blocks of others kFixupSpan samples
+    if (in && q + 1 == parts) push(i, js, false);
+    return 0u;
+  }
+  const int64_t ps = series_part(js, je, q, parts), pe = series_part(js, je, q + 1, parts);
+  const bool ends = b + 1 == nb && q + 1 == parts;  // the last sample is this part's too
+  if (ps >= pe) return 0u;  // never the block's last part
+  SeriesState<T> st;
+  double stop;
+  bool live = in;
+  bool bad = false;
+  {
+    ThetaConsts<T> tc;
+    const ThetaPick tp = theta_pick(plan, stride, p, gflags, o, tc);
+    stop = tp.stop;
+    const T lam = T(plan[static_cast<int64_t>(PL_LAM) * stride + p]);
+    // EARLY: the plan's radial constants may still be being written
+    const bool walks =
+        tp.walk && (EARLY || radial_walks(o, gflags, plan[static_cast<int64_t>(PL_R + R_k) * stride + p]));
+    if (live && !walks) {
+      // no heads for this pixel either: every sample, the last included
+      for (int64_t j = ps; j < (ends ? o.ngeo : pe); j += kFixupSpan) push(i, j, false);
+      live = false;
+    }
+    const T h = T(stop / static_cast<double>(o.ngeo - 1));
+    series_ray(c, tc, tp.kind == THK_VORT, lam, T(plan[static_cast<int64_t>(PL_QA) * stride + p]),
+               T(plan[static_cast<int64_t>(PL_QB) * stride + p]), T(plan[static_cast<int64_t>(PL_QC) * stride + p]), h, k);
+    if (!EARLY && c.minspin && plan[static_cast<int64_t>(PL_RCASE) * stride + p] == 3.0) {
+      // below MINSPIN the reference leaves the third-kind part of I_- out in
+      // this case (kerr_raytracing_ana.py:529): 1/(r - r_-) is a constant
+      const double* r0 = plan + static_cast<int64_t>(PL_R) * stride + p;
+      const T kc = -(T(r0[C3_AA * stride]) + T(r0[C3_BB * stride])) * T(r0[C3_iImd * stride]);
+      const T m0 = 1.0 + T(c.rminus) * kc;
+      k.set(SR_am, k(SR_am) * m0);
+      k.set(SR_bm, k(SR_bm) * m0);
+      k.set(SR_rm, T(0.0));
+    }
+    const CombineConsts<T> cmb = combine_consts(c, lam);
+    if (!EARLY && live && ends) bad = series_head_store<T>(o, cmb, last * o.npix + i, stop, rr, 0, p) || bad;
+    const int64_t idx = js * o.npix + i;
+    if (EARLY || b == 0) {
+      const T w0 = 1.0 / T(c.r_o);
+      st.w = w0;
+      st.v = ksqrt(1.0 + w0 * w0 * (k(SR_A) + w0 * (k(SR_B) + w0 * k(SR_C))));
+      st.c = c.cos_th;
+      st.u = T(plan[static_cast<int64_t>(PL_U0) * stride + p]);
+      st.t = T(0.0);
+      st.f = T(0.0);
+      st.s = T(0.0);
+    } else {
+      const double tau = mino_tau(js, o.ngeo, stop, false);
+      st.c = T(*rth.at(b, kThSFields, 0, p));
+      st.u = T(*rth.at(b, kThSFields, 1, p));
+      st.w = 1.0 / T(*rr.at(b, kRSFields, 0, p));
+      st.v = T(*rr.at(b, kRSFields, 5, p));
+      if (live) {
+        RadialOut<T> ro;
+        ro.r = T(*rr.at(b, kRSFields, 0, p));
+        ro.Ip = T(*rr.at(b, kRSFields, 1, p));
+        ro.Im = T(*rr.at(b, kRSFields, 2, p));
+        ro.I1 = T(*rr.at(b, kRSFields, 3, p));
+        ro.I2 = T(*rr.at(b, kRSFields, 4, p));
+        Sample<T> s;
+        combine(cmb, T(tau), ro, T(0.0), T(*rth.at(b, kThSFields, 2, p)), T(*rth.at(b, kThSFields, 3, p)), s);
+        st.t = -s.t;
+        st.f = -s.ph;
+        st.s = -s.sig;
+      }
+    }
+    // the series needs a pole at the axis (lam != 0), a bounded observer and
+    // a finite start
+    const bool ok = kfinite(val(st.w)) & kfinite(val(st.v)) & kfinite(val(st.c)) & kfinite(val(st.u)) &
+                    kfinite(val(st.t)) & kfinite(val(st.f)) & (val(k(SR_l2)) > 0.0) & (val(lam) != 0.0) &
+                    (val(st.w) > 0.0) & kfinite(val(k(SR_E))) & kfinite(val(h));
+    if (live && !ok) {
+      push_range(push, i, ps, pe, last);
+      live = false;
+    }
+    if (live && ps == js) {
+      // the block's first sample
+      const double tau = mino_tau(js, o.ngeo, stop, false);
+      const T th = acos_poly(st.c);
+      if (o.tau_out) o.tau_out[idx] = tau;
+      if (o.th && b == 0) o.th[idx] = val(th);  // the anchor's head wrote it
+      if (o.r && b > 0) o.r[idx] = *rr.at(b, kRSFields, 0, p);  // sample 0: radial head 0
+      o.t[idx] = val(-st.t);
+      o.ph[idx] = val(-st.f);
+      if (SIG) o.sig[idx] = val(-st.s);
+    }
+    if (!live) {
+      // a harmless motion for the lane's share of the wave's steps
+      st.w = T(1.0e-3);
+      st.v = T(0.0);
+      st.c = T(0.0);
+      st.u = T(0.0);
+    }
+  }
+  const float floor_x = static_cast<float>(je - js) / static_cast<float>(kSeriesMinStep);
+  // the position, in samples from js (exact: steps end on multiples of 2^-10)
+  double x0 = 0.0;
+  int64_t j = js + 1;
+  const double xe = static_cast<double>(je - js);
+  while (j < pe) {
+    Series<T, P, SIG> S;
+    k.fresh();
+    float x = series_expand<T, P, SIG>(c, k, st, S);
+    if (!(x >= floor_x)) {  // also NaN
+      if (live) push_range(push, i, j < ps ? ps : j, pe, last);
+      live = false;
+    }
+    if (!live) x = 1.0e30f;
+    x = wave_min(x);
+    if (x == 1.0e30f) break;  // no lane is left
+    double x1 = x0 + static_cast<double>(x);
+    if (x1 > xe) x1 = xe;
+    x1 = kfloor(x1 * 1024.0) * (1.0 / 1024.0);
+    const int64_t jn = js + static_cast<int64_t>(kfloor(x1)) + 1;  // the first sample after the step
+    const int64_t jm = jn < pe ? jn : pe;
+    if (j < ps) j = ps < jm ? ps : jm;
+    double xj = static_cast<double>(j - js) - x0;
+    for (; j < jm; ++j) {
+      SeriesState<T> s;
+      T r;
+      k.fresh();
+      series_at<T, P, SIG, false>(k, S, T(xj), s, r);
+      xj += 1.0;
+      const T th = acos_fast(s.c);
+      if (live) {
+        const int64_t idx = j * o.npix + i;
+        if (o.tau_out) o.tau_out[idx] = mino_tau(j, o.ngeo, stop, false);
+        if (o.th) o.th[idx] = val(th);
+        if (o.r) o.r[idx] = val(r);
+        o.t[idx] = val(-s.t);
+        o.ph[idx] = val(-s.f);
+        if (SIG) o.sig[idx] = val(-s.s);
+        bad = bad | !(kfabs(val(r)) + kfabs(val(th)) + kfabs(val(s.t)) + kfabs(val(s.f)) < INFINITY);
+      }
+    }
+    if (j >= pe) break;
+    SeriesState<T> e;
+    T r;
+    series_at<T, P, SIG, true>(k, S, T(x1 - x0), e, r);
+    st = e;
+    x0 = x1;
+  }
+  return bad ? ST_NONFINITE : 0u;
+}
+
+}  // namespace kg

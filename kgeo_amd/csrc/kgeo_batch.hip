@@ -10,17 +10,15 @@
 //                        straddles two images and the image-wide predicates
 //                        (any eta > 0, any zero grid step) are per-image
 //                        wave ballots.
-//   kg_batch_pass<P>     for theta then r, the heads, far and walk passes of
-//                        the plain kernels (kg_sample.hpp), each a fixed grid
-//                        of waves taking work items (image, 64-pixel tile,
-//                        head / block / Mino-time chunk) from its own atomic
-//                        counter until the pass is empty; every wave leaves
-//                        once the counter passes the pass's item total, so
-//                        the grid always drains;
-//   kg_batch_repair      after the radial far pass: the blocks whose long
-//                        step was refused, one lane per (block, segment),
-//                        by direct evaluation (grid-stride);
-//   kg_batch_fixup<R>    the queued ranges of all images, one lane per
+//   kg_batch_heads<P>    the theta, then the radial heads of the plain kernels
+//                        (kg_series_pass.hpp): a fixed grid of waves taking
+//                        work items (image, 64-pixel tile, head) from an
+//                        atomic counter until the pass is empty; every wave
+//                        leaves once the counter passes the pass's item
+//                        total, so the grid always drains;
+//   kg_batch_series      the rays' blocks, items (image, tile, block,
+//                        part), in the same way;
+//   kg_batch_fixup       the queued ranges of all images, one lane per
 //                        (range, sample), by direct evaluation (grid-stride).
 // Outputs go to caller arenas: image k's [ngeo_k][npix_k] block of r, theta,
 // phi, t starts at element out_off[k] (sum of npix*ngeo of the images before
@@ -33,7 +31,7 @@
 #include <vector>
 
 #include "../../include/kgeo.h"
-#include "kg_sample.hpp"
+#include "kg_series_pass.hpp"
 
 using namespace kg;
 
@@ -62,13 +60,9 @@ constexpr int64_t kMaxItems = (1LL << 31) - (1LL << 24);  // leaves room for one
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 // pass kinds and their per-tile work units
-enum : int { K_HEAD = 0, K_FAR = 1, K_WALK = 2, K_N = 3 };
-// pass counters: theta heads, far, walk, then r heads, far, walk; then the
-// theta and radial fixup-queue counters
-constexpr int kPassCounters = 2 * K_N;
-constexpr int kQueueCounter = kPassCounters;  // + 0 theta, + 1 r
-constexpr int kRepairCounter = kPassCounters + 2;  // the radial far pass's repair items
-constexpr int kCounters = kPassCounters + 3;
+enum : int { K_HEAD = 0, K_SERIES = 1, K_N = 2 };
+// counters: theta heads, radial heads, series, then the fixup queue
+enum : int { CT_THETA = 0, CT_RADIAL, CT_SERIES, CT_QUEUE, kCounters };
 
 struct BatchImage {
   RayScalars<double> c;
@@ -79,7 +73,7 @@ struct BatchImage {
   int64_t out_off;   // first element of the image's [ngeo][npix] block
   int64_t item_off[K_N];  // first work item of each pass kind
   int64_t th_rec, r_rec;  // first element of the image's record tables
-  int32_t units[K_N];     // heads, anchor blocks, Mino-time chunks per tile
+  int32_t units[K_N];     // per tile: heads (one per block); parts of all blocks
   int32_t do_phi_t;
 };
 
@@ -170,16 +164,6 @@ struct BatchPush {
   }
 };
 
-// The radial far pass hands a block with a lost long step to kg_batch_repair
-// through the queue storage (the theta fixups are done with it; the radial
-// walk's pushes come after the repair pass): at most one item per block and
-// pixel slot, within the queue's capacity.
-struct BatchRepair {
-  static constexpr bool kOn = true;
-  BatchPush push;
-  __device__ void operator()(int64_t i, int64_t j, bool walked) const { push(i, j, walked); }
-};
-
 __device__ inline SampleOut image_out(const BatchDev& d, const BatchImage& B) {
   return SampleOut{nullptr, nullptr, d.t + B.out_off, d.r + B.out_off, d.th + B.out_off, d.ph + B.out_off, nullptr,
                    B.npix, B.ngeo};
@@ -189,37 +173,10 @@ __device__ inline Records image_records(const BatchDev& d, const BatchImage& B, 
   return Records{d.rec + (theta ? B.th_rec : B.r_rec), B.slots, B.slot_off};
 }
 
-// One unit of pass KIND (theta if THETA) for pixel i of image B.  Every
-// image samples t, phi and sigma (the plan rejects images without
-// KGEO_DO_PHI_T), so PHI_T is true throughout.
-template <int KIND, bool THETA>
-__device__ inline uint32_t batch_unit(const BatchDev& d, const BatchImage& B, int im, int64_t i, int64_t u) {
-  const int64_t s = B.slot_off + i;
-  const uint32_t fl = d.flags[im];
-  const SampleOut o = image_out(d, B);
-  const Records rt = image_records(d, B, THETA);
-  constexpr bool PHI_T = true;
-  if (KIND == K_HEAD) {
-    return THETA ? theta_head_pixel<PHI_T>(d.plan, d.total_slots, s, fl, o, i, u, rt)
-                 : radial_head_pixel<PHI_T>(B.c, d.plan, d.total_slots, s, fl, o, i, u, rt);
-  }
-  if (KIND == K_FAR) {
-    const BatchRepair repair{
-        BatchPush{d.queue, d.counter + kRepairCounter, d.qcap, static_cast<unsigned long long>(im)}};
-    return THETA ? theta_far_pixel<PHI_T>(d.plan, d.total_slots, s, fl, o, i, u, rt)
-                 : radial_far_pixel<PHI_T>(B.c, d.plan, d.total_slots, s, fl, o, i, u, rt, repair);
-  }
-  const int64_t j0 = chunk_start(B.ngeo, u, B.units[K_WALK]);
-  const int64_t j1 = chunk_start(B.ngeo, u + 1, B.units[K_WALK]);
-  BatchPush push{d.queue, d.counter + kQueueCounter + (THETA ? 0 : 1), d.qcap, static_cast<unsigned long long>(im)};
-  return THETA ? theta_walk_pixel<PHI_T>(d.plan, d.total_slots, s, fl, o, i, j0, j1, rt, push)
-               : radial_walk_pixel<PHI_T>(B.c, d.plan, d.total_slots, s, fl, o, i, j0, j1, rt, push);
-}
-
-template <int KIND, bool THETA>
-__device__ inline void batch_pass(const BatchDev& d) {
+// Items (image, tile, unit) of pass KIND from `counter` until none is left;
+// f(image, its index, its pixel on this lane, whether there is one, unit).
+template <int KIND, class F> __device__ inline void batch_items(const BatchDev& d, uint32_t* counter, F f) {
   const int lane = __lane_id();
-  uint32_t* counter = d.counter + (THETA ? 0 : K_N) + KIND;
   for (;;) {
     const uint32_t item = fetch_item(counter, lane);
     if (item >= d.total_items[KIND]) break;  // scalar branch: the whole wave leaves once the pass is empty
@@ -228,31 +185,47 @@ __device__ inline void batch_pass(const BatchDev& d) {
     const int64_t li = static_cast<int64_t>(item) - B.item_off[KIND];
     const int64_t units = B.units[KIND];
     const int64_t i = (li / units) * kWave + lane;
-    const int64_t u = li % units;
-    if (i < B.npix) {
-      const uint32_t st = batch_unit<KIND, THETA>(d, B, im, i, u);
-      if (d.status && st) atomicOr(&d.status[B.pix_off + i], st);
-    }
+    const bool in = i < B.npix;
+    const uint32_t st = f(B, im, in ? i : B.npix - 1, in, li % units);
+    if (in && d.status && st) atomicOr(&d.status[B.pix_off + i], st);
     atomicAdd(&d.done[im], lane == 0 ? 1u : 0u);
   }
 }
 
-template <int KIND, bool THETA>
-__global__ __launch_bounds__(kBlock) void kg_batch_pass(BatchDev d) {
-  batch_pass<KIND, THETA>(d);
+template <bool THETA> __global__ __launch_bounds__(kBlock) void kg_batch_heads(BatchDev d) {
+  batch_items<K_HEAD>(d, d.counter + (THETA ? CT_THETA : CT_RADIAL),
+                      [&](const BatchImage& B, int im, int64_t i, bool in, int64_t hd) {
+                        if (!in) return 0u;
+                        const int64_t s = B.slot_off + i;
+                        const SampleOut o = image_out(d, B);
+                        const Records rt = image_records(d, B, THETA);
+                        return THETA ? series_theta_head_pixel(d.plan, d.total_slots, s, d.flags[im], o, i, hd,
+                                                               B.units[K_HEAD], rt)
+                                     : series_radial_head_pixel(d.plan, d.total_slots, s, d.flags[im], o, i, hd,
+                                                                B.units[K_HEAD], B.c.r_o, rt);
+                      });
 }
 
-// the walk pass held to two waves per SIMD, as kg_radial_walk
-template <bool THETA>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_batch_walk(BatchDev d) {
-  batch_pass<K_WALK, THETA>(d);
+// kg_series (kgeo_raytrace.hip) over all images, two waves per SIMD as there.
+// A survey of 16 images (64 .. 512 pixels a side, 50 .. 400 samples; 58 million
+// samples) takes 9.7 ms, where the walk by addition theorems took 21.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_batch_series(BatchDev d) {
+  __shared__ double sl[kBlock / kWave][SERIES_SLOTS][kWave];
+  LdsSlots slots{sl[threadIdx.x / kWave], static_cast<int>(threadIdx.x % kWave)};
+  batch_items<K_SERIES>(d, d.counter + CT_SERIES, [&](const BatchImage& B, int im, int64_t i, bool in, int64_t u) {
+    BatchPush push{d.queue, d.counter + CT_QUEUE, d.qcap, static_cast<unsigned long long>(im)};
+    const SampleOut o = image_out(d, B);
+    const Records rth = image_records(d, B, true), rr = image_records(d, B, false);
+    const int64_t nb = B.units[K_HEAD], parts = B.units[K_SERIES] / nb;
+    return series_block_pixel<false, false>(B.c, d.plan, d.total_slots, B.slot_off + i, d.flags[im], o, i, in, u % nb,
+                                            nb, parts - 1 - u / nb, parts, rth, rr, slots, push);
+  });
 }
 
 // one lane per (queued range, sample of the range) (grid-stride), each
-// sample by direct evaluation, as the plain kg_theta_fixup / kg_radial_fixup
-template <bool THETA>
+// sample by direct evaluation, as the plain kg_fixup
 __global__ __launch_bounds__(kBlock) void kg_batch_fixup(BatchDev d) {
-  const unsigned long long c = d.counter[kQueueCounter + (THETA ? 0 : 1)];
+  const unsigned long long c = d.counter[CT_QUEUE];
   const unsigned long long n = (c < d.qcap ? c : d.qcap) * kFixupSpan;
   for (unsigned long long e = static_cast<unsigned long long>(blockIdx.x) * kBlock + threadIdx.x; e < n;
        e += static_cast<unsigned long long>(gridDim.x) * kBlock) {
@@ -266,32 +239,8 @@ __global__ __launch_bounds__(kBlock) void kg_batch_fixup(BatchDev d) {
     const int64_t s = B.slot_off + i;
     const uint32_t fl = d.flags[im];
     const SampleOut o = image_out(d, B);
-    const uint32_t st = THETA ? theta_fixup_sample<true>(d.plan, d.total_slots, s, fl, o, i, j, walked, sg)
-                              : radial_fixup_sample<true>(B.c, d.plan, d.total_slots, s, fl, o, i, j, walked, sg);
-    if (d.status && st) atomicOr(&d.status[B.pix_off + i], st);
-  }
-}
-
-// one lane per (repair item, segment of its block) (grid-stride), as the
-// plain kg_radial_repair
-constexpr int kRepairSegments = static_cast<int>(kAnchorBlock / kAnchorEvery);
-
-__global__ __launch_bounds__(kBlock) void kg_batch_repair(BatchDev d) {
-  const unsigned long long c = d.counter[kRepairCounter];
-  const unsigned long long n = (c < d.qcap ? c : d.qcap) * kRepairSegments;
-  for (unsigned long long e = static_cast<unsigned long long>(blockIdx.x) * kBlock + threadIdx.x; e < n;
-       e += static_cast<unsigned long long>(gridDim.x) * kBlock) {
-    const unsigned long long q = d.queue[e / kRepairSegments];
-    const int64_t sg = static_cast<int64_t>(e % kRepairSegments);
-    const int im = static_cast<int>((q >> 51) & 0xfffull);
-    const int64_t j = static_cast<int64_t>((q >> 31) & 0xfffffull);
-    const int64_t i = static_cast<int64_t>(q & 0x7fffffffull);
-    const BatchImage& B = d.imgs[im];
-    const int64_t s = B.slot_off + i;
-    const uint32_t fl = d.flags[im];
-    const SampleOut o = image_out(d, B);
-    const Records rt = image_records(d, B, false);
-    const uint32_t st = radial_repair_pixel<true>(B.c, d.plan, d.total_slots, s, fl, o, i, j, sg, rt);
+    uint32_t st = theta_fixup_sample<true>(d.plan, d.total_slots, s, fl, o, i, j, walked, sg);
+    st |= radial_fixup_sample<true>(B.c, d.plan, d.total_slots, s, fl, o, i, j, walked, sg);
     if (d.status && st) atomicOr(&d.status[B.pix_off + i], st);
   }
 }
@@ -330,13 +279,16 @@ int64_t total_slots_of(const kgeo_ray_params* imgs, int32_t nimg) {
 }
 
 // Elements of image k's theta and radial record tables (a walked grid needs
-// ngeo > 2; smaller images keep none) and its fixup-queue share.
+// ngeo > 2; smaller images keep none) and its fixup-queue share.  The sizes
+// are the interface's; the anchor records take a part of each table.
 int64_t theta_rec_elems(const kgeo_ray_params& p) {
   return p.ngeo > 2 ? theta_records(p.ngeo) * kThFields * slots_of(p) : 0;
 }
 int64_t radial_rec_elems(const kgeo_ray_params& p) {
   return p.ngeo > 2 ? radial_records(p.ngeo) * kRFields * slots_of(p) : 0;
 }
+static_assert(kSeriesBlocks * kThSFields <= 4 * kThFields && kSeriesBlocks * kRSFields <= 4 * kRFields,
+              "the records fit the smallest tables");
 int64_t queue_elems(const kgeo_ray_params& p) { return fixup_items(p.ngeo) * slots_of(p); }
 
 struct BatchSizes {
@@ -414,10 +366,13 @@ int kgeo_batch_plan(const kgeo_ray_params* imgs, int32_t nimg, const kgeo_batch_
   std::vector<BatchImage> host(nimg);
   std::vector<uint32_t> per(nimg);
   int64_t pix = 0, slots = 0, outo = 0, rec = 0;
-  int64_t items[K_N] = {0, 0, 0};
-  // walk items hold whole segments (chunk starts are multiples of kAnchorEveryLong)
+  int64_t items[K_N] = {0, 0};
+  // the survey's size as its caller cut it: an item holds samples_per_item
+  // samples, rounded up to whole segments
+  int64_t asked = 0;
   const int64_t spi =
       (static_cast<int64_t>(tn.samples_per_item) + kAnchorEveryLong - 1) / kAnchorEveryLong * kAnchorEveryLong;
+  const int64_t all_slots = total_slots_of(imgs, nimg);
   for (int32_t k = 0; k < nimg; ++k) {
     const kgeo_ray_params& p = imgs[k];
     BatchImage& B = host[k];
@@ -428,9 +383,13 @@ int kgeo_batch_plan(const kgeo_ray_params* imgs, int32_t nimg, const kgeo_batch_
     B.slot_off = slots;
     B.slots = slots_of(p);
     B.out_off = outo;
-    B.units[K_HEAD] = static_cast<int32_t>(anchor_heads(p.ngeo));
-    B.units[K_FAR] = static_cast<int32_t>(anchor_blocks(p.ngeo));
-    B.units[K_WALK] = static_cast<int32_t>((p.ngeo + spi - 1) / spi);
+    // an item of the series is 64 rays' part of a block: as many parts as
+    // the tuning asks for, while they help to fill the chip (the results are
+    // the same bits for any)
+    const int64_t nb = series_blocks(p.ngeo);
+    const int64_t fill = pick_parts(all_slots, p.ngeo), asks = (p.ngeo / nb + spi - 1) / spi;
+    B.units[K_HEAD] = static_cast<int32_t>(nb);
+    B.units[K_SERIES] = static_cast<int32_t>(nb * (asks < 1 ? 1 : (asks < fill ? asks : fill)));
     B.th_rec = rec;
     rec += theta_rec_elems(p);
     B.r_rec = rec;
@@ -442,12 +401,14 @@ int kgeo_batch_plan(const kgeo_ray_params* imgs, int32_t nimg, const kgeo_batch_
       B.item_off[q] = items[q];
       items[q] += tiles * B.units[q];
       mine += tiles * B.units[q];
-      if (items[q] > kMaxItems) return bfail(KGEO_E_ARG, "too many work items (%lld); raise samples_per_item", items[q]);
     }
+    asked += tiles * ((p.ngeo + spi - 1) / spi);
+    if (asked > kMaxItems || items[K_HEAD] > kMaxItems)
+      return bfail(KGEO_E_ARG, "too many work items (%lld); raise samples_per_item", asked);
     pix += p.npix;
     slots += B.slots;
     outo += p.npix * p.ngeo;
-    per[k] = static_cast<uint32_t>(2 * mine);  // theta and radial passes
+    per[k] = static_cast<uint32_t>(mine + tiles * B.units[K_HEAD]);  // theta and radial heads
   }
   if (!t || !ph) return bfail(KGEO_E_ARG, "t and ph are required");
 
@@ -508,15 +469,10 @@ int kgeo_batch_plan(const kgeo_ray_params* imgs, int32_t nimg, const kgeo_batch_
   }
   hipLaunchKernelGGL(kg_batch_clear, dim3(1), dim3(kBlock), 0, st, d);
   hipLaunchKernelGGL(kg_batch_setup, dim3(setup_blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL((kg_batch_pass<K_HEAD, true>), dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL((kg_batch_pass<K_FAR, true>), dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL(kg_batch_walk<true>, dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL(kg_batch_fixup<true>, dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL((kg_batch_pass<K_HEAD, false>), dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL((kg_batch_pass<K_FAR, false>), dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL(kg_batch_repair, dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL(kg_batch_walk<false>, dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL(kg_batch_fixup<false>, dim3(blocks), dim3(kBlock), 0, st, d);
+  hipLaunchKernelGGL(kg_batch_heads<true>, dim3(blocks), dim3(kBlock), 0, st, d);
+  hipLaunchKernelGGL(kg_batch_heads<false>, dim3(blocks), dim3(kBlock), 0, st, d);
+  hipLaunchKernelGGL(kg_batch_series, dim3(blocks), dim3(kBlock), 0, st, d);
+  hipLaunchKernelGGL(kg_batch_fixup, dim3(blocks), dim3(kBlock), 0, st, d);
   const int lrc = blaunch("batch kernel launch (capture)");
   hipGraph_t g = nullptr;
   const hipError_t ce = hipStreamEndCapture(st, &g);
@@ -544,9 +500,7 @@ int kgeo_batch_run(kgeo_batch* b, void* stream) {
 
 int64_t kgeo_batch_items(const kgeo_batch* b) {
   if (!b) return -1;
-  int64_t n = 0;
-  for (int q = 0; q < K_N; ++q) n += 2 * static_cast<int64_t>(b->d.total_items[q]);
-  return n;
+  return 2 * static_cast<int64_t>(b->d.total_items[K_HEAD]) + static_cast<int64_t>(b->d.total_items[K_SERIES]);
 }
 
 int kgeo_batch_progress(const kgeo_batch* b, uint32_t* done_items, uint32_t* total_items) {

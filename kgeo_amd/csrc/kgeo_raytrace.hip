@@ -1,10 +1,7 @@
 // HIP kernels (gfx950) and the C-ABI of include/kgeo.h for the analytic
 // Kerr raytracer.
 //
-// Pipeline of one kgeo_raytrace_ana call, on the caller's stream except the
-// plan's radial constants and the radial heads, far and repair passes, which
-// run on a per-device side stream beside the theta work and are joined
-// before the radial walk:
+// Pipeline of one kgeo_raytrace_ana call:
 //   kg_clear_flags   one wave: zero the flag page of the workspace
 //   kg_setup         one lane per pixel: lambda, eta, u_+-, roots, labels,
 //                    tau_tot, nmax_eq and the per-pixel constants of the
@@ -13,23 +10,18 @@
 //                    numpy code decides globally (any eta > 0, any zero step);
 //                    with a side stream, as kg_setup_theta (all but the
 //                    radial constants) and kg_setup_radial (side stream)
-// then, on the linspace grid, per coordinate (theta first: its G_phi, G_t
-// are parked in the phi and t outputs; the radial stores combine them):
+// then, on the linspace grid (kg_series_pass.hpp):
 //   kg_*_heads       one lane per (pixel, head): direct evaluations (Landen
-//                    ladder, Carlson duplication) at the steps h and L h, the
-//                    last sample and each block's first sample -> records
-//   kg_*_far         one lane per (pixel, block): the block's other segment
-//                    starts by long addition steps -> records; a radial
-//                    block whose long step is refused (a pole of a
-//                    third-kind integral inside it) is queued for
-//   kg_radial_repair one lane per (queued block, segment): the block's
-//                    remaining segment starts by direct evaluation -> records
-//   kg_*_walk        one lane per (pixel, sample chunk): every other sample
-//                    by the addition theorems from the records; 64 lanes
-//                    write 512 contiguous bytes per output and sample
-//   kg_*_fixup       one lane per (queued range, sample): direct evaluation
-//                    of the samples where the walk refused a step
-// (kg_sample.hpp).  Caller-given Mino times and grids of at most two samples
+//                    ladder, Carlson duplication) of the last sample and of
+//                    each block's first -> records
+//   kg_series        one lane per (pixel, block of samples): Taylor series
+//                    along the ray; 64 lanes write 512 contiguous bytes per
+//                    output and sample
+//   kg_fixup         one lane per (queued range, sample): direct evaluation
+//                    of what the series leaves
+// A ray's first block starts from the observer and runs on the caller's
+// stream, while the per-device side stream evaluates the heads and then runs
+// the other blocks.  Caller-given Mino times and grids of at most two samples
 // take kg_theta / kg_radial, one combined loop per coordinate.  The work is
 // FP64 VALU (no MFMA).
 
@@ -43,7 +35,7 @@
 
 #include "../../include/kgeo.h"
 #include "kg_counts.hpp"
-#include "kg_sample.hpp"
+#include "kg_series_pass.hpp"
 
 using namespace kg;
 
@@ -71,9 +63,21 @@ constexpr int kBlock = 256;
 // The sample passes run one wave per workgroup: their waves differ widely in
 // cost (radial case, refused steps), and a CU's slot is freed per workgroup,
 // so a multi-wave workgroup would hold its SIMDs until its slowest wave ends.
-// (The theta walk, whose waves cost alike, keeps kBlock.)
 constexpr int kPassBlock = 64;
 constexpr size_t kFlagBytes = 256;
+
+// The tile (pixels 64 t ..) of workgroup b of n along x.  From the image's
+// middle outwards: the rays near the shadow take the most steps, and the long
+// waves are to start first.  Workgroups go to the chip's 8 XCDs in turn and
+// an image is often a multiple of 8 tiles wide, so each group of 8 is turned
+// by one more place, lest an XCD hold the same columns of every row.  (512 x 512 x 500 samples:
+// 2.28 ms, 2.35 in the order of the pixels.)
+__device__ inline int64_t tile_of(unsigned b, unsigned n) {
+  const unsigned g = b >> 3;
+  const unsigned k = (g << 3) + 8 <= n ? (g << 3) + ((b + g) & 7u) : b;
+  const int64_t mid = n / 2;
+  return (k & 1u) ? mid - static_cast<int64_t>((k + 1) / 2) : mid + static_cast<int64_t>(k / 2);
+}
 
 struct DevParams {
   RayScalars<double> c;
@@ -103,19 +107,12 @@ __global__ void kg_clear_flags(uint32_t* flags) {
   if (threadIdx.x < kFlagBytes / sizeof(uint32_t)) flags[threadIdx.x] = 0u;
 }
 
-// Word 0 of the flag page holds the image-wide flags (kg_setup); words 1 and
-// 2 count the theta and radial fixup items of one sample pass, word 3 the
-// radial repair items.
-constexpr int kThetaCount = 1;
-constexpr int kRadialCount = 2;
-constexpr int kRepairCount = 3;  // the radial far pass's repair items
+// Word 0 of the flag page holds the image-wide flags (kg_setup); word 1
+// counts the fixup items of one sample pass.
+constexpr int kFixupCount = 1;
 
 __global__ void kg_clear_counters(uint32_t* flags) {
-  if (threadIdx.x == 0) {
-    flags[kThetaCount] = 0u;
-    flags[kRadialCount] = 0u;
-    flags[kRepairCount] = 0u;
-  }
+  if (threadIdx.x == 0) flags[kFixupCount] = 0u;
 }
 
 // Two waves per SIMD: unbounded the set-up needs about 300 VGPR+AGPR (one
@@ -124,7 +121,7 @@ __global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2)))
     DevParams p, const double* __restrict__ alpha, const double* __restrict__ beta, double* __restrict__ plan,
     uint32_t* __restrict__ gflags, int8_t* __restrict__ rclass, int8_t* __restrict__ thclass,
     int32_t* __restrict__ nmax_eq, double* __restrict__ tau_tot, uint32_t* __restrict__ status) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
+  const int64_t i = tile_of(blockIdx.x, gridDim.x) * kPassBlock + threadIdx.x;
   SetupOut so{false, false};
   if (i < p.npix)
     so = setup_pixel(p.c, p.ngeo, p.do_phi_t != 0, alpha[i], beta[i], plan, p.npix, i, rclass, thclass, nmax_eq,
@@ -141,7 +138,7 @@ __global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2)))
     DevParams p, const double* __restrict__ alpha, const double* __restrict__ beta, double* __restrict__ plan,
     uint32_t* __restrict__ gflags, int8_t* __restrict__ rclass, int8_t* __restrict__ thclass,
     int32_t* __restrict__ nmax_eq, double* __restrict__ tau_tot, uint32_t* __restrict__ status) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
+  const int64_t i = tile_of(blockIdx.x, gridDim.x) * kPassBlock + threadIdx.x;
   SetupOut so{false, false};
   if (i < p.npix)
     so = setup_pixel<true>(p.c, p.ngeo, p.do_phi_t != 0, alpha[i], beta[i], plan, p.npix, i, rclass, thclass,
@@ -152,7 +149,7 @@ __global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2)))
 
 __global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_setup_radial(
     DevParams p, const double* __restrict__ alpha, const double* __restrict__ beta, double* __restrict__ plan) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
+  const int64_t i = tile_of(blockIdx.x, gridDim.x) * kPassBlock + threadIdx.x;
   if (i < p.npix) setup_radial_pixel(p.c, p.do_phi_t != 0, alpha[i], beta[i], plan, p.npix, i);
 }
 
@@ -190,10 +187,8 @@ __global__ __launch_bounds__(kBlock) void kg_radial(DevParams p, SampleArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// The walk in three passes per coordinate (kg_sample.hpp): anchor -> walk ->
-// fixup for theta, then the same for r (whose stores combine phi, t, sigma
-// with the theta parts).  The fixup queue holds one 64-bit item per queued
-// range: walked << 63 | first sample << 32 | pixel.
+// The linspace grid's passes.  The fixup queue holds one 64-bit item per
+// queued range: walked << 63 | first sample << 32 | pixel.
 // ---------------------------------------------------------------------------
 struct FixupQueue {
   unsigned long long* items;
@@ -211,69 +206,56 @@ struct DevPush {
   }
 };
 
-// The radial far pass hands a block with a lost long step to the repair
-// pass through the same queue storage (the theta fixups are done with it, and
-// the radial walk's pushes come after the repair pass).  At most one item per
-// block and pixel: within the queue's npix * ceil(ngeo / 8) items.
-struct DevRepair {
-  static constexpr bool kOn = true;
-  FixupQueue q;
-  __device__ void operator()(int64_t i, int64_t j, bool walked) const { DevPush{q}(i, j, walked); }
-};
-
 __device__ inline void unpack_item(unsigned long long e, int64_t& i, int64_t& j, bool& walked) {
   i = static_cast<int64_t>(e & 0xffffffffull);
   j = static_cast<int64_t>((e >> 32) & 0x7fffffffull);
   walked = (e >> 63) != 0ull;
 }
 
-// grid (pixel blocks, heads): the direct evaluations of the anchor pass
-template <bool DO_PHI_T>
-// last = false: every head but the last sample's (head 2), which the theta
-// far and walk passes do not read; last = true: head 2 alone (grid y = 1),
-// which the side stream takes (it emits the last sample for the radial walk)
-__global__ __launch_bounds__(kPassBlock) void kg_theta_heads(DevParams p, SampleArgs a, Records rt, int64_t nhead,
-                                                             int last) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
+// grid (pixel blocks, heads): the direct evaluations (head 0 the last
+// sample, head b the first sample of block b)
+__global__ __launch_bounds__(kPassBlock) void kg_theta_heads(DevParams p, SampleArgs a, Records rt, int64_t nb) {
+  const int64_t i = tile_of(blockIdx.x, gridDim.x) * kPassBlock + threadIdx.x;
   if (i >= p.npix) return;
-  uint32_t st = 0u;
-  if (last) {
-    st = theta_head_pixel<DO_PHI_T>(a.plan, p.npix, i, a.gflags[0], a.out, i, 2, rt);
-  } else {
-    for (int64_t y = blockIdx.y; y < nhead - 1; y += gridDim.y)
-      st |= theta_head_pixel<DO_PHI_T>(a.plan, p.npix, i, a.gflags[0], a.out, i, y < 2 ? y : y + 1, rt);
-  }
+  const uint32_t st = series_theta_head_pixel(a.plan, p.npix, i, a.gflags[0], a.out, i, blockIdx.y, nb, rt);
   if (a.status && st) atomicOr(&a.status[i], st);
 }
 
-// grid (pixel blocks, anchor blocks): the long steps of the anchor pass
-template <bool DO_PHI_T>
-__global__ __launch_bounds__(kPassBlock) void kg_theta_far(DevParams p, SampleArgs a, Records rt, int64_t nblk) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
+__global__ __launch_bounds__(kPassBlock) void kg_radial_heads(DevParams p, SampleArgs a, Records rt, int64_t nb) {
+  const int64_t i = tile_of(blockIdx.x, gridDim.x) * kPassBlock + threadIdx.x;
   if (i >= p.npix) return;
-  uint32_t st = 0u;
-  for (int64_t b = blockIdx.y; b < nblk; b += gridDim.y)
-    st |= theta_far_pixel<DO_PHI_T>(a.plan, p.npix, i, a.gflags[0], a.out, i, b, rt);
+  const uint32_t st = series_radial_head_pixel(a.plan, p.npix, i, a.gflags[0], a.out, i, blockIdx.y, nb, p.c.r_o, rt);
   if (a.status && st) atomicOr(&a.status[i], st);
 }
 
-template <bool DO_PHI_T>
-// Four waves per SIMD (128 VGPR, a few spills): 1.31 against 1.40 ms at
-// three (512^2 x 500).
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void kg_theta_walk(DevParams p,
-    SampleArgs a, Records rt, FixupQueue q) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= p.npix) return;
-  const int64_t j0 = chunk_start(p.ngeo, blockIdx.y, a.chunks);
-  const int64_t j1 = chunk_start(p.ngeo, blockIdx.y + 1, a.chunks);
+// grid (pixel blocks, parts): one wave per workgroup, 64 neighbouring pixels
+// at one part of block b of their grids (the last part, the longest, first).
+// Bound by FP64 issue: a sample takes 235 vector instructions (84
+// multiply-adds of six polynomials, a logarithm, an arctangent, an arccosine,
+// a reciprocal), an expansion about 2300, and a ray about 12 of them.  At 512 x
+// 512 x 500 samples (t, r, theta, phi written) one block of all rays takes
+// 1.14 ms at 65 % VALU busy; the whole call 2.28 ms, where the walk by
+// addition theorems (up to three Carlson R_J per sample) took 4.95; 217 x 301 x
+// 333 0.82 for 1.29, 64 x 64 x 100 0.42 for 0.54, 1000 x 250 0.36 for 0.55.
+// Two waves per SIMD: one alone (512 registers) is slower from 217 x 301 on
+// (0.98 and 3.0 ms).
+template <bool SIG, bool EARLY>
+__global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_series(
+    DevParams p, SampleArgs a, Records rth, Records rr, int64_t b, int64_t nb, FixupQueue q) {
+  const int64_t lane = tile_of(blockIdx.x, gridDim.x) * kPassBlock + threadIdx.x;
+  const bool in = lane < p.npix;
+  const int64_t i = in ? lane : p.npix - 1;
+  __shared__ double sl[SERIES_SLOTS][kPassBlock];
+  LdsSlots slots{sl, static_cast<int>(threadIdx.x)};
   DevPush push{q};
-  const uint32_t st = theta_walk_pixel<DO_PHI_T>(a.plan, p.npix, i, a.gflags[0], a.out, i, j0, j1, rt, push);
+  const uint32_t st = series_block_pixel<SIG, EARLY>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, in, b, nb,
+                                                     gridDim.y - 1 - blockIdx.y, gridDim.y, rth, rr, slots, push);
   if (a.status && st) atomicOr(&a.status[i], st);
 }
 
-template <bool DO_PHI_T>
-// one lane per (queued range, sample of the range) (grid-stride)
-__global__ __launch_bounds__(kPassBlock) void kg_theta_fixup(DevParams p, SampleArgs a, FixupQueue q) {
+// one lane per (queued range, sample of the range) (grid-stride): theta, then
+// r and the combination, by direct evaluation
+__global__ __launch_bounds__(kPassBlock) void kg_fixup(DevParams p, SampleArgs a, FixupQueue q) {
   const unsigned long long c = *q.count;
   const unsigned long long n = (c < q.cap ? c : q.cap) * kFixupSpan;
   for (unsigned long long e = static_cast<unsigned long long>(blockIdx.x) * kPassBlock + threadIdx.x; e < n;
@@ -282,80 +264,8 @@ __global__ __launch_bounds__(kPassBlock) void kg_theta_fixup(DevParams p, Sample
     bool walked;
     unpack_item(q.items[e / kFixupSpan], i, j, walked);
     const int64_t sg = static_cast<int64_t>(e % kFixupSpan);
-    const uint32_t st = theta_fixup_sample<DO_PHI_T>(a.plan, p.npix, i, a.gflags[0], a.out, i, j, walked, sg);
-    if (a.status && st) atomicOr(&a.status[i], st);
-  }
-}
-
-template <bool DO_PHI_T>
-__global__ __launch_bounds__(kPassBlock) void kg_radial_heads(DevParams p, SampleArgs a, Records rt, int64_t nhead) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
-  if (i >= p.npix) return;
-  uint32_t st = 0u;
-  for (int64_t hd = blockIdx.y; hd < nhead; hd += gridDim.y)
-    st |= radial_head_pixel<DO_PHI_T>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, hd, rt);
-  if (a.status && st) atomicOr(&a.status[i], st);
-}
-
-// Two waves per SIMD: the far pass needs about 268 VGPR+AGPR, one wave per
-// SIMD unbounded; held to 256 with a few spills it runs about a quarter
-// faster (0.32 against 0.44 ms at 512^2 x 500).
-template <bool DO_PHI_T>
-__global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_radial_far(
-    DevParams p, SampleArgs a, Records rt, int64_t nblk, FixupQueue qrep) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
-  if (i >= p.npix) return;
-  const DevRepair repair{qrep};
-  uint32_t st = 0u;
-  for (int64_t b = blockIdx.y; b < nblk; b += gridDim.y)
-    st |= radial_far_pixel<DO_PHI_T>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, b, rt, repair);
-  if (a.status && st) atomicOr(&a.status[i], st);
-}
-
-// one lane per (repair item, segment of its block) (grid-stride): each of
-// a block's segment starts from the lost one on, by direct evaluation
-constexpr int kRepairSegments = static_cast<int>(kAnchorBlock / kAnchorEvery);
-
-template <bool DO_PHI_T>
-__global__ __launch_bounds__(kPassBlock) void kg_radial_repair(DevParams p, SampleArgs a, Records rt,
-                                                              FixupQueue qrep) {
-  const unsigned long long c = *qrep.count;
-  const unsigned long long n = (c < qrep.cap ? c : qrep.cap) * kRepairSegments;
-  for (unsigned long long e = static_cast<unsigned long long>(blockIdx.x) * kPassBlock + threadIdx.x; e < n;
-       e += static_cast<unsigned long long>(gridDim.x) * kPassBlock) {
-    int64_t i, j;
-    bool walked;
-    unpack_item(qrep.items[e / kRepairSegments], i, j, walked);
-    const int64_t sg = static_cast<int64_t>(e % kRepairSegments);
-    const uint32_t st = radial_repair_pixel<DO_PHI_T>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, j, sg, rt);
-    if (a.status && st) atomicOr(&a.status[i], st);
-  }
-}
-
-template <bool DO_PHI_T>
-__global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_radial_walk(DevParams p, SampleArgs a, Records rt, FixupQueue q) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
-  if (i >= p.npix) return;
-  const int64_t j0 = chunk_start(p.ngeo, blockIdx.y, a.chunks);
-  const int64_t j1 = chunk_start(p.ngeo, blockIdx.y + 1, a.chunks);
-  DevPush push{q};
-  const uint32_t st = radial_walk_pixel<DO_PHI_T>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, j0, j1, rt, push);
-  if (a.status && st) atomicOr(&a.status[i], st);
-}
-
-template <bool DO_PHI_T>
-// one lane per (queued range, sample of the range) (grid-stride)
-__global__ __launch_bounds__(kPassBlock) void kg_radial_fixup(DevParams p, SampleArgs a, FixupQueue q) {
-  const unsigned long long c = *q.count;
-  const unsigned long long n = (c < q.cap ? c : q.cap) * kFixupSpan;
-  for (unsigned long long e = static_cast<unsigned long long>(blockIdx.x) * kPassBlock + threadIdx.x; e < n;
-       e += static_cast<unsigned long long>(gridDim.x) * kPassBlock) {
-    int64_t i, j;
-    bool walked;
-    unpack_item(q.items[e / kFixupSpan], i, j, walked);
-    const int64_t sg = static_cast<int64_t>(e % kFixupSpan);
-    const uint32_t st =
-        radial_fixup_sample<DO_PHI_T>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, j, walked, sg);
+    uint32_t st = theta_fixup_sample<true>(a.plan, p.npix, i, a.gflags[0], a.out, i, j, walked, sg);
+    st |= radial_fixup_sample<true>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, j, walked, sg);
     if (a.status && st) atomicOr(&a.status[i], st);
   }
 }
@@ -442,13 +352,14 @@ int env_chunks() {
   return s ? std::atoi(s) : 0;
 }
 
-// Workspace: the flag page, the plan [PL_N][npix] and, for a walked grid
-// (ngeo > 2), the theta and radial record tables and the fixup queue (one
-// item per kFixupSpan samples and pixel bounds every pass's pushes).
+// Workspace: the flag page, the plan [PL_N][npix] and, for a grid of more
+// than two samples, the theta and radial anchor records and the fixup queue
+// (one item per kFixupSpan samples and pixel bounds the series' pushes).  The
+// size is the interface's (kgeo.h), of which the records take a part: per
+// pixel at least 76 doubles, of which they take 2 (kThSFields + kRSFields).
 struct WsLayout {
-  size_t plan, threc, rrec, queue, rqueue, total;
-  int64_t nth, nr;
-  unsigned long long qcap, rcap;
+  size_t plan, threc, rrec, queue, total;
+  unsigned long long qcap;
 };
 
 WsLayout ws_layout(int64_t npix, int64_t ngeo) {
@@ -457,25 +368,19 @@ WsLayout ws_layout(int64_t npix, int64_t ngeo) {
   L.plan = kFlagBytes;
   size_t off = kFlagBytes + np * PL_N * sizeof(double);
   if (ngeo > 2) {
-    L.nth = theta_records(ngeo);
-    L.nr = radial_records(ngeo);
-    L.threc = off;
-    off += static_cast<size_t>(L.nth) * kThFields * np * sizeof(double);
-    L.rrec = off;
-    off += static_cast<size_t>(L.nr) * kRFields * np * sizeof(double);
+    const size_t tables = static_cast<size_t>(theta_records(ngeo)) * kThFields +
+                          static_cast<size_t>(radial_records(ngeo)) * kRFields;
     L.qcap = static_cast<unsigned long long>(np) * static_cast<unsigned long long>(fixup_items(ngeo));
     L.queue = off;
-    off += static_cast<size_t>(L.qcap) * sizeof(unsigned long long);
-    // the radial far pass's repair items, at most one per (pixel, block):
-    // their own storage, as the radial anchor passes run beside the theta
-    // passes, whose fixups use the queue above
-    L.rcap = static_cast<unsigned long long>(np) * static_cast<unsigned long long>(anchor_blocks(ngeo));
-    L.rqueue = off;
-    off += static_cast<size_t>(L.rcap) * sizeof(unsigned long long);
+    L.threc = off + static_cast<size_t>(L.qcap) * sizeof(unsigned long long);
+    L.rrec = L.threc + static_cast<size_t>(kSeriesBlocks) * kThSFields * np * sizeof(double);
+    off += np * sizeof(double) * (static_cast<size_t>(fixup_items(ngeo)) + tables + static_cast<size_t>(anchor_blocks(ngeo)));
   }
   L.total = off;
   return L;
 }
+static_assert(kSeriesBlocks * (kThSFields + kRSFields) <= 4 * kThFields + 4 * kRFields,
+              "the records fit the tables' part of the workspace");
 
 // The kernels always sample t, phi and sigma (as the reference's
 // raytrace_ana does, kerr_raytracing_ana.py:97): the theta pass parks G_phi,
@@ -516,13 +421,12 @@ int validate(const kgeo_ray_params* p, const double* alpha, const double* beta, 
 }
 
 
-// A second stream per device for the radial anchor passes, which depend
-// only on the plan and so run beside the theta passes (two latency-bound
-// kernels interleave on the SIMDs); created once per device, with the fork
-// and join events.  The fork, the side stream's work and the join are
+// A second stream per device for the plan's radial constants, the heads and
+// the blocks that start from them, beside the first blocks (which need only
+// the plan's other part) on the caller's; created once per device, with the
+// fork and join events.  The fork, the side stream's work and the join are
 // enqueued under one lock, so calls from several host threads keep their
-// own dependencies (their radial anchor passes take turns on the side
-// stream).  Streams keep the default priority.
+// own dependencies (their side work takes turns on the side stream).  Streams keep the default priority.
 struct SideStream {
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
@@ -593,29 +497,30 @@ int run_plan(const kgeo_ray_params* p, const double* alpha, const double* beta, 
   return KGEO_OK;
 }
 
-template <bool DO_PHI_T>
-int run_walk(const DevParams& d, const SampleArgs& a, void* ws, dim3 grid, hipStream_t st) {
+int run_series(const DevParams& d, const SampleArgs& a, void* ws, hipStream_t st) {
   const WsLayout L = ws_layout(d.npix, d.ngeo);
   char* base = static_cast<char*>(ws);
   uint32_t* flags = static_cast<uint32_t*>(ws);
   const Records rth{reinterpret_cast<double*>(base + L.threc), d.npix, 0};
   const Records rr{reinterpret_cast<double*>(base + L.rrec), d.npix, 0};
   unsigned long long* items = reinterpret_cast<unsigned long long*>(base + L.queue);
-  unsigned long long* ritems = reinterpret_cast<unsigned long long*>(base + L.rqueue);
-  const FixupQueue qth{items, flags + kThetaCount, L.qcap};
-  const FixupQueue qr{items, flags + kRadialCount, L.qcap};
-  const FixupQueue qrep{ritems, flags + kRepairCount, L.rcap};
-  const unsigned nb = static_cast<unsigned>((d.npix + kPassBlock - 1) / kPassBlock);
-  const dim3 wgrid(nb, grid.y);
-  const unsigned long long fb = (L.qcap + kPassBlock - 1) / kPassBlock;
+  const FixupQueue q{items, flags + kFixupCount, L.qcap};
+  const unsigned np = static_cast<unsigned>((d.npix + kPassBlock - 1) / kPassBlock);
+  const int64_t nb = series_blocks(d.ngeo);
+  const unsigned parts = static_cast<unsigned>(pick_parts(d.npix, d.ngeo));
+  const unsigned nbu = static_cast<unsigned>(nb);
+  const unsigned long long fb = (L.qcap * kFixupSpan + kPassBlock - 1) / kPassBlock;
   const dim3 fgrid(static_cast<unsigned>(fb < 4096ull ? fb : 4096ull));
-  const unsigned long long rb = (L.rcap * kRepairSegments + kPassBlock - 1) / kPassBlock;
-  const dim3 rgrid(static_cast<unsigned>(rb < 4096ull ? (rb > 0 ? rb : 1ull) : 4096ull));
-  auto recs = [](int64_t n) { return static_cast<unsigned>(n < 65535 ? n : 65535); };
+  // block 0 starts from the observer: with further blocks (which take the
+  // last sample) it waits for no head, nor, above MINSPIN, for the radial plan
+  const bool early = nb > 1 && !d.c.minspin;
+  auto series = [&](auto kernel, hipStream_t on, int64_t b) {
+    hipLaunchKernelGGL(kernel, dim3(np, parts), dim3(kPassBlock), 0, on, d, a, rth, rr, b, nb, q);
+    return check_launch("kg_series");
+  };
   hipLaunchKernelGGL(kg_clear_counters, dim3(1), dim3(64), 0, st, flags);
   int rc = check_launch("kg_clear_counters");
   if (rc) return rc;
-  const int64_t nblk = anchor_blocks(d.ngeo), nhead = anchor_heads(d.ngeo);
   {
     std::lock_guard<std::mutex> lock(g_side_mu);
     SideStream* ss = side_stream(st);
@@ -624,36 +529,20 @@ int run_walk(const DevParams& d, const SampleArgs& a, void* ws, dim3 grid, hipSt
       if (hipEventRecord(ss->fork, st) != hipSuccess || hipStreamWaitEvent(rs, ss->fork, 0) != hipSuccess)
         return fail_msg(KGEO_E_HIP, "fork to the side stream failed");
     }
-    // radial heads, far and repair: records only (the walk emits the samples)
-    hipLaunchKernelGGL(kg_radial_heads<DO_PHI_T>, dim3(nb, recs(nhead)), dim3(kPassBlock), 0, rs, d, a, rr, nhead);
-    if ((rc = check_launch("kg_radial_heads"))) return rc;
-    hipLaunchKernelGGL(kg_radial_far<DO_PHI_T>, dim3(nb, recs(nblk)), dim3(kPassBlock), 0, rs, d, a, rr, nblk,
-                       qrep);
-    if ((rc = check_launch("kg_radial_far"))) return rc;
-    hipLaunchKernelGGL(kg_radial_repair<DO_PHI_T>, rgrid, dim3(kPassBlock), 0, rs, d, a, rr, qrep);
-    if ((rc = check_launch("kg_radial_repair"))) return rc;
-    // theta's last-sample head: read by the radial walk only
-    hipLaunchKernelGGL(kg_theta_heads<DO_PHI_T>, dim3(nb, 1), dim3(kPassBlock), 0, rs, d, a, rth, nhead, 1);
-    if ((rc = check_launch("kg_theta_heads (last sample)"))) return rc;
-    if (ss && hipEventRecord(ss->join, rs) != hipSuccess) return fail_msg(KGEO_E_HIP, "join event failed");
-    // theta passes on the caller's stream meanwhile
-    hipLaunchKernelGGL(kg_theta_heads<DO_PHI_T>, dim3(nb, recs(nhead - 1)), dim3(kPassBlock), 0, st, d, a, rth, nhead,
-                       0);
+    // the heads and the blocks that start from them, beside block 0
+    hipLaunchKernelGGL(kg_theta_heads, dim3(np, nbu), dim3(kPassBlock), 0, rs, d, a, rth, nb);
     if ((rc = check_launch("kg_theta_heads"))) return rc;
-    hipLaunchKernelGGL(kg_theta_far<DO_PHI_T>, dim3(nb, recs(nblk)), dim3(kPassBlock), 0, st, d, a, rth, nblk);
-    if ((rc = check_launch("kg_theta_far"))) return rc;
-    hipLaunchKernelGGL(kg_theta_walk<DO_PHI_T>, grid, dim3(kBlock), 0, st, d, a, rth, qth);
-    if ((rc = check_launch("kg_theta_walk"))) return rc;
-    hipLaunchKernelGGL(kg_theta_fixup<DO_PHI_T>, fgrid, dim3(kPassBlock), 0, st, d, a, qth);
-    if ((rc = check_launch("kg_theta_fixup"))) return rc;
+    hipLaunchKernelGGL(kg_radial_heads, dim3(np, nbu), dim3(kPassBlock), 0, rs, d, a, rr, nb);
+    if ((rc = check_launch("kg_radial_heads"))) return rc;
+    for (int64_t b = early ? 1 : 0; b < nb; ++b)
+      if ((rc = a.out.sig ? series(kg_series<true, false>, rs, b) : series(kg_series<false, false>, rs, b))) return rc;
+    if (ss && hipEventRecord(ss->join, rs) != hipSuccess) return fail_msg(KGEO_E_HIP, "join event failed");
+    if (early && (rc = a.out.sig ? series(kg_series<true, true>, st, 0) : series(kg_series<false, true>, st, 0)))
+      return rc;
     if (ss && hipStreamWaitEvent(st, ss->join, 0) != hipSuccess) return fail_msg(KGEO_E_HIP, "join failed");
   }
-  // the radial walk emits every radial sample it walks and every segment
-  // start from its record, combining with the theta pass's G_phi, G_t
-  hipLaunchKernelGGL(kg_radial_walk<DO_PHI_T>, wgrid, dim3(kPassBlock), 0, st, d, a, rr, qr);
-  if ((rc = check_launch("kg_radial_walk"))) return rc;
-  hipLaunchKernelGGL(kg_radial_fixup<DO_PHI_T>, fgrid, dim3(kPassBlock), 0, st, d, a, qr);
-  return check_launch("kg_radial_fixup");
+  hipLaunchKernelGGL(kg_fixup, fgrid, dim3(kPassBlock), 0, st, d, a, q);
+  return check_launch("kg_fixup");
 }
 
 int run_sample(const kgeo_ray_params* p, int64_t ngeo, const double* tau_in, double* tau, double* t, double* r,
@@ -667,9 +556,9 @@ int run_sample(const kgeo_ray_params* p, int64_t ngeo, const double* tau_in, dou
   const int chunks = kgeo_sample_chunks(d.npix, ngeo);
   dim3 grid(nb, static_cast<unsigned>(chunks));
   SampleArgs a{plan, gflags, SampleOut{tau_in, tau, t, r, th, ph, sig, d.npix, ngeo}, status, chunks};
-  // the linspace grid walks (heads, far, walk, fixup passes); caller-given
+  // the linspace grid takes the series (heads, series, fixup); caller-given
   // Mino times and grids of at most two samples are evaluated directly
-  if (!tau_in && ngeo > 2) return run_walk<true>(d, a, ws, grid, st);
+  if (!tau_in && ngeo > 2) return run_series(d, a, ws, st);
   {
     // the plan's radial constants come from the side stream (run_plan)
     std::lock_guard<std::mutex> lock(g_side_mu);
