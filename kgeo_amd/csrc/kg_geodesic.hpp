@@ -653,6 +653,11 @@ template <class T> KG_INLINE void atan_sum_sc(const T& x, const T& g, bool x_inf
   cb = (1.0 - x * g) / d;
 }
 
+// The radial constants, in three stages: each case's modulus, amplitude and
+// characteristics; the elliptic integrals of all cases in one place; what each
+// case makes of them.  (A wave holds rays of all cases: with the integrals
+// inside the cases it ran them three times, and the kernels' first pass over
+// that code, fetched cold by every CU, was most of a small image's set-up.)
 template <class T>
 KG_INLINE void radial_consts(const RayScalars<T>& c, const PixelSetup<T>& px, bool do_phi_t, RadialConsts<T>& rc) {
 #if defined(__clang__)
@@ -664,49 +669,119 @@ KG_INLINE void radial_consts(const RayScalars<T>& c, const PixelSetup<T>& px, bo
   const T& rplus = c.rplus;
   const T& rminus = c.rminus;
   const double r_o = c.r_o;
+  T k, sb, cb;                           // parameter, sin and cos of the observer's amplitude
+  T n0 = T(0.0), np = T(0.0), nm = T(0.0);  // the characteristics of the third-kind integrals
+  T a2 = T(0.0), b1 = T(0.0), g0 = T(0.0), gp = T(0.0), gm = T(0.0), x4rp = T(0.0), x4rm = T(0.0), pref = T(0.0);
+  T AA = T(0.0), BB = T(0.0), al0 = T(0.0), alp = T(0.0), alm = T(0.0);
   if (px.rcase == 4) {
-    T a1 = px.ri[3], b1 = px.rr[3], a2 = px.ri[1], b2 = px.rr[1];
+    T a1 = px.ri[3], b2 = px.rr[1];
+    b1 = px.rr[3];
+    a2 = px.ri[1];
     T CC = ksqrt(sq(a1 - a2) + sq(b1 - b2));
     T DD = ksqrt(sq(a1 + a2) + sq(b1 - b2));
-    T k4 = (4.0 * CC * DD) / sq(CC + DD);
-    T x4rp = (rplus + b1) / a2;
-    T x4rm = (rminus + b1) / a2;
-    T g0 = ksqrt((4.0 * a2 * a2 - sq(CC - DD)) / (sq(CC + DD) - 4.0 * a2 * a2));
-    T gp = (g0 * x4rp - 1.0) / (g0 + x4rp);
-    T gm = (g0 * x4rm - 1.0) / (g0 + x4rm);
-    T sb, cb;
+    k = (4.0 * CC * DD) / sq(CC + DD);
+    x4rp = (rplus + b1) / a2;
+    x4rm = (rminus + b1) / a2;
+    g0 = ksqrt((4.0 * a2 * a2 - sq(CC - DD)) / (sq(CC + DD) - 4.0 * a2 * a2));
+    gp = (g0 * x4rp - 1.0) / (g0 + x4rp);
+    gm = (g0 * x4rm - 1.0) / (g0 + x4rm);
     atan_sum_sc(c.r_o_inf ? T(0.0) : (r_o + b1) / a2, g0, c.r_o_inf, sb, cb);
-    T pref = 2.0 / (CC + DD);
-    T K = ellip_K(k4);
-    Amp<T> Ab = amp_from_sc(sb, cb);
-    LegendreBase<T> Lb = legendre_base(Ab, k4);
-    T Fb = legendre_F(Lb, K);
-    T s2b = ksqrt(1.0 - k4 * (sb * sb));
-    v[R_k] = k4;
-    v[R_K] = K;
+    pref = 2.0 / (CC + DD);
     v[R_Xs] = 1.0 / pref;
-    v[R_U0] = Fb;
-    v[R_sn0] = sb;
-    v[R_cn0] = cb;
-    v[R_dn0] = s2b;
+    n0 = 1.0 + g0 * g0;
+    np = 1.0 + gp * gp;
+    nm = 1.0 + gm * gm;
+  } else if (px.rcase == 3) {
+    T a1 = px.ri[3];
+    b1 = px.rr[3];
+    T rr1 = px.rr[0], rr2 = px.rr[1];
+    T rr21 = rr2 - rr1;
+    T rrp1 = rplus - rr1, rrp2 = rplus - rr2;
+    T rrm1 = rminus - rr1, rrm2 = rminus - rr2;
+    AA = ksqrt(a1 * a1 + sq(b1 - rr2));
+    BB = ksqrt(a1 * a1 + sq(b1 - rr1));
+    k = (sq(AA + BB) - rr21 * rr21) / (4.0 * AA * BB);
+    T x3ro;
+    if (c.r_o_inf) {
+      x3ro = (AA - BB) / (AA + BB);
+    } else {
+      T rro1 = r_o - rr1, rro2 = r_o - rr2;
+      x3ro = (AA * rro1 - BB * rro2) / (AA * rro1 + BB * rro2);
+    }
+    pref = 1.0 / ksqrt(AA * BB);
+    sb = ksqrt((1.0 - x3ro) * (1.0 + x3ro));  // sin(arccos x3ro)
+    cb = x3ro;
+    v[R_Xs] = 1.0 / pref;
+    T x3rp = (AA * rrp1 - BB * rrp2) / (AA * rrp1 + BB * rrp2);
+    T x3rm = (AA * rrm1 - BB * rrm2) / (AA * rrm1 + BB * rrm2);
+    alp = -1.0 / x3rp;
+    alm = -1.0 / x3rm;
+    al0 = (BB + AA) / (BB - AA);
+    n0 = (al0 * al0) / (al0 * al0 - 1.0);
+    np = (alp * alp) / (alp * alp - 1.0);
+    nm = (alm * alm) / (alm * alm - 1.0);
+  } else {
+    T rr1 = px.rr[0], rr2 = px.rr[1], rr3 = px.rr[2], rr4 = px.rr[3];
+    T rr31 = rr3 - rr1, rr32 = rr3 - rr2, rr41 = rr4 - rr1, rr42 = rr4 - rr2;
+    T rrp3 = rplus - rr3, rrm3 = rminus - rr3, rrp4 = rplus - rr4, rrm4 = rminus - rr4;
+    k = (rr32 * rr41) / (rr31 * rr42);
+    T x2ro = c.r_o_inf ? ksqrt(rr31 / rr41) : ksqrt((rr31 * (r_o - rr4)) / (rr41 * (r_o - rr3)));
+    sb = x2ro;
+    cb = ksqrt((1.0 - x2ro) * (1.0 + x2ro));
+    v[R_Xs] = 0.5 * ksqrt(rr31 * rr42);
+    n0 = rr41 / rr31;
+    np = (rrp3 * rr41) / (rrp4 * rr31);
+    nm = (rrm3 * rr41) / (rrm4 * rr31);
+  }
+  // the integrals at the observer's amplitude, and the complete ones
+  const T K = ellip_K(k);
+  const LegendreBase<T> Lb = legendre_base(amp_from_sc(sb, cb), k);
+  const T Fb = legendre_F(Lb, K);
+  const T s2b = ksqrt(1.0 - k * (sb * sb));
+  v[R_k] = k;
+  v[R_K] = K;
+  v[R_U0] = Fb;
+  v[R_sn0] = sb;
+  v[R_cn0] = cb;
+  v[R_dn0] = s2b;
+  T Pc0 = T(0.0), Pcp = T(0.0), Pcm = T(0.0), Pb0 = T(0.0), Pbp = T(0.0), Pbm = T(0.0), Eb = T(0.0);
+  if (do_phi_t) {
+    const T EmK = ellip_EmK(k);
+    v[R_EmK] = EmK;
+    Eb = Fb + legendre_EmF(Lb, k, EmK);
+#if defined(__clang__)
+#pragma clang loop unroll(disable)
+#endif
+    for (int i = 0; i < 3; ++i) {
+      const T n = i == 0 ? n0 : (i == 1 ? np : nm);
+      const T pc = ellip_pi_complete(n, k, K);
+      const T pb = ellip_pi_amp(Lb, n, k, pc);
+      if (i == 0) {
+        Pc0 = pc;
+        Pb0 = pb;
+      } else if (i == 1) {
+        Pcp = pc;
+        Pbp = pb;
+      } else {
+        Pcm = pc;
+        Pbm = pb;
+      }
+    }
+  }
+  if (px.rcase == 4) {
     v[C4_a2] = a2;
     v[C4_b1] = b1;
     v[C4_g0] = g0;
     if (do_phi_t) {
-      T EmK = ellip_EmK(k4);
-      v[R_EmK] = EmK;
-      T n0 = 1.0 + g0 * g0, np = 1.0 + gp * gp, nm = 1.0 + gm * gm;
-      T Pc0 = ellip_pi_complete(n0, k4, K), Pcp = ellip_pi_complete(np, k4, K), Pcm = ellip_pi_complete(nm, k4, K);
       v[C4_gp] = gp; v[C4_gm] = gm;
       v[C4_n0] = n0; v[C4_np] = np; v[C4_nm] = nm;
       v[C4_Pc0] = Pc0; v[C4_Pcp] = Pcp; v[C4_Pcm] = Pcm;
-      T Eb = Fb + legendre_EmF(Lb, k4, EmK);
-      T S1b0 = S1_block(g0, ellip_pi_amp(Lb, n0, k4, Pc0), Fb, s2b, k4);
+      T S1b0 = S1_block(g0, Pb0, Fb, s2b, k);
       v[C4_S1b0] = S1b0;
-      v[C4_S2b0] = S2_block(g0, S1b0, Fb, Eb, sb, cb, s2b, k4);
-      v[C4_S1bp] = S1_block(gp, ellip_pi_amp(Lb, np, k4, Pcp), Fb, s2b, k4);
-      v[C4_S1bm] = S1_block(gm, ellip_pi_amp(Lb, nm, k4, Pcm), Fb, s2b, k4);
-      const T q0 = S1_p(g0, k4), qp = S1_p(gp, k4), qm = S1_p(gm, k4);
+      v[C4_S2b0] = S2_block(g0, S1b0, Fb, Eb, sb, cb, s2b, k);
+      v[C4_S1bp] = S1_block(gp, Pbp, Fb, s2b, k);
+      v[C4_S1bm] = S1_block(gm, Pbm, Fb, s2b, k);
+      const T q0 = S1_p(g0, k), qp = S1_p(gp, k), qm = S1_p(gm, k);
       v[C4_q0] = q0; v[C4_qp] = qp; v[C4_qm] = qm;
       v[C4_l0] = klog(kfabs((1.0 - q0) / (1.0 + q0)));
       v[C4_lp] = klog(kfabs((1.0 - qp) / (1.0 + qp)));
@@ -724,66 +799,28 @@ KG_INLINE void radial_consts(const RayScalars<T>& c, const PixelSetup<T>& px, bo
       v[C4_Imf] = g0 / (a2 - a2 * g0 * x4rm);
     }
   } else if (px.rcase == 3) {
-    T a1 = px.ri[3], b1 = px.rr[3];
     T rr1 = px.rr[0], rr2 = px.rr[1];
-    T rr21 = rr2 - rr1;
-    T rrp1 = rplus - rr1, rrp2 = rplus - rr2;
-    T rrm1 = rminus - rr1, rrm2 = rminus - rr2;
-    T AA = ksqrt(a1 * a1 + sq(b1 - rr2));
-    T BB = ksqrt(a1 * a1 + sq(b1 - rr1));
-    T k3 = (sq(AA + BB) - rr21 * rr21) / (4.0 * AA * BB);
-    T x3ro;
-    if (c.r_o_inf) {
-      x3ro = (AA - BB) / (AA + BB);
-    } else {
-      T rro1 = r_o - rr1, rro2 = r_o - rr2;
-      x3ro = (AA * rro1 - BB * rro2) / (AA * rro1 + BB * rro2);
-    }
-    T pref = 1.0 / ksqrt(AA * BB);
-    T K = ellip_K(k3);
-    T sb = ksqrt((1.0 - x3ro) * (1.0 + x3ro));  // sin(arccos x3ro)
-    T cb = x3ro;
-    Amp<T> Ab = amp_from_sc(sb, cb);
-    LegendreBase<T> Lb = legendre_base(Ab, k3);
-    T Fb = legendre_F(Lb, K);
-    T s2b = ksqrt(1.0 - k3 * (sb * sb));
-    v[R_k] = k3;
-    v[R_K] = K;
-    v[R_Xs] = 1.0 / pref;
-    v[R_U0] = Fb;
-    v[R_sn0] = sb;
-    v[R_cn0] = cb;
-    v[R_dn0] = s2b;
     v[C3_AA] = AA;
     v[C3_BB] = BB;
     v[C3_rr1] = rr1;
     v[C3_rr2] = rr2;
     if (do_phi_t) {
-      T x3rp = (AA * rrp1 - BB * rrp2) / (AA * rrp1 + BB * rrp2);
-      T x3rm = (AA * rrm1 - BB * rrm2) / (AA * rrm1 + BB * rrm2);
-      T alp = -1.0 / x3rp;
-      T alm = -1.0 / x3rm;
-      T al0 = (BB + AA) / (BB - AA);
-      T EmK = ellip_EmK(k3);
-      v[R_EmK] = EmK;
-      T nn0 = (al0 * al0) / (al0 * al0 - 1.0);
-      T nnp = (alp * alp) / (alp * alp - 1.0);
-      T nnm = (alm * alm) / (alm * alm - 1.0);
-      T Pc0 = ellip_pi_complete(nn0, k3, K), Pcp = ellip_pi_complete(nnp, k3, K);
-      T Pcm = c.spin_gt_min ? ellip_pi_complete(nnm, k3, K) : T(0.0);
+      T rr21 = rr2 - rr1;
+      T rrp1 = rplus - rr1, rrp2 = rplus - rr2;
+      T rrm1 = rminus - rr1, rrm2 = rminus - rr2;
       v[C3_al0] = al0; v[C3_alp] = alp; v[C3_alm] = alm;
-      v[C3_nn0] = nn0; v[C3_nnp] = nnp; v[C3_nnm] = nnm;
-      v[C3_Pc0] = Pc0; v[C3_Pcp] = Pcp; v[C3_Pcm] = Pcm;
-      T Eb = Fb + legendre_EmF(Lb, k3, EmK);
-      T R1b0 = R1_block(al0, ellip_pi_amp(Lb, nn0, k3, Pc0), sb, s2b, k3);
+      v[C3_nn0] = n0; v[C3_nnp] = np; v[C3_nnm] = nm;
+      v[C3_Pc0] = Pc0; v[C3_Pcp] = Pcp;
+      v[C3_Pcm] = c.spin_gt_min ? Pcm : T(0.0);
+      T R1b0 = R1_block(al0, Pb0, sb, s2b, k);
       v[C3_R1b0] = R1b0;
-      v[C3_R2b0] = R2_block(al0, nn0, R1b0, Fb, Eb, sb, cb, s2b, k3);
-      v[C3_R1bp] = R1_block(alp, ellip_pi_amp(Lb, nnp, k3, Pcp), sb, s2b, k3);
-      v[C3_R1bm] = c.spin_gt_min ? R1_block(alm, ellip_pi_amp(Lb, nnm, k3, Pcm), sb, s2b, k3) : T(0.0);
+      v[C3_R2b0] = R2_block(al0, n0, R1b0, Fb, Eb, sb, cb, s2b, k);
+      v[C3_R1bp] = R1_block(alp, Pbp, sb, s2b, k);
+      v[C3_R1bm] = c.spin_gt_min ? R1_block(alm, Pbm, sb, s2b, k) : T(0.0);
       v[C3_hasm] = c.spin_gt_min ? T(1.0) : T(0.0);
-      v[C3_p0] = R1_p(al0, k3);
-      v[C3_pp] = R1_p(alp, k3);
-      v[C3_pm] = R1_p(alm, k3);
+      v[C3_p0] = R1_p(al0, k);
+      v[C3_pp] = R1_p(alp, k);
+      v[C3_pm] = R1_p(alm, k);
       v[C3_i0] = 1.0 / (1.0 - al0 * al0);
       v[C3_ip] = 1.0 / (1.0 - alp * alp);
       v[C3_im] = 1.0 / (1.0 - alm * alm);
@@ -800,48 +837,27 @@ KG_INLINE void radial_consts(const RayScalars<T>& c, const PixelSetup<T>& px, bo
       v[C3_iImd] = 1.0 / v[C3_Imd];
       {
         const T al2 = al0 * al0;
-        const T den = k3 + (1.0 - k3) * al2;
+        const T den = k + (1.0 - k) * al2;
         v[C3_r2a] = al2 / den;
         v[C3_r2b] = 1.0 / (al2 - 1.0);
-        v[C3_r2c] = (2.0 * k3 - nn0) / den;
+        v[C3_r2c] = (2.0 * k - n0) / den;
       }
     }
   } else {
     T rr1 = px.rr[0], rr2 = px.rr[1], rr3 = px.rr[2], rr4 = px.rr[3];
-    T rr31 = rr3 - rr1, rr32 = rr3 - rr2, rr41 = rr4 - rr1, rr42 = rr4 - rr2, rr43 = rr4 - rr3;
+    T rr31 = rr3 - rr1, rr41 = rr4 - rr1, rr42 = rr4 - rr2, rr43 = rr4 - rr3;
     T rrp3 = rplus - rr3, rrm3 = rminus - rr3, rrp4 = rplus - rr4, rrm4 = rminus - rr4;
-    T k2 = (rr32 * rr41) / (rr31 * rr42);
-    T x2ro = c.r_o_inf ? ksqrt(rr31 / rr41) : ksqrt((rr31 * (r_o - rr4)) / (rr41 * (r_o - rr3)));
-    T K = ellip_K(k2);
-    T sb = x2ro;
-    T cb = ksqrt((1.0 - x2ro) * (1.0 + x2ro));
-    Amp<T> Ab = amp_from_sc(sb, cb);
-    LegendreBase<T> Lb = legendre_base(Ab, k2);
-    T Fb = legendre_F(Lb, K);
     T sq3142 = ksqrt(rr31 * rr42);
-    v[R_k] = k2;
-    v[R_K] = K;
-    v[R_Xs] = 0.5 * sq3142;
-    v[R_U0] = Fb;
-    v[R_sn0] = sb;
-    v[R_cn0] = cb;
-    v[R_dn0] = ksqrt(1.0 - k2 * (sb * sb));
     v[C2_rr1] = rr1; v[C2_rr2] = rr2; v[C2_rr3] = rr3; v[C2_rr4] = rr4;
     v[C2_rr31] = rr31; v[C2_rr41] = rr41; v[C2_rr43] = rr43;
     if (do_phi_t) {
-      T EmK = ellip_EmK(k2);
-      v[R_EmK] = EmK;
       v[C2_rrp3] = rrp3; v[C2_rrm3] = rrm3;
-      T n1 = rr41 / rr31;
-      T np = (rrp3 * rr41) / (rrp4 * rr31);
-      T nm = (rrm3 * rr41) / (rrm4 * rr31);
-      v[C2_n1] = n1; v[C2_np] = np; v[C2_nm] = nm;
-      T Pc1 = ellip_pi_complete(n1, k2, K), Pcp = ellip_pi_complete(np, k2, K), Pcm = ellip_pi_complete(nm, k2, K);
-      v[C2_Pc1] = Pc1; v[C2_Pcp] = Pcp; v[C2_Pcm] = Pcm;
-      v[C2_Eb] = Fb + legendre_EmF(Lb, k2, EmK);
-      v[C2_Pb1] = ellip_pi_amp(Lb, n1, k2, Pc1);
-      v[C2_Pbp] = ellip_pi_amp(Lb, np, k2, Pcp);
-      v[C2_Pbm] = ellip_pi_amp(Lb, nm, k2, Pcm);
+      v[C2_n1] = n0; v[C2_np] = np; v[C2_nm] = nm;
+      v[C2_Pc1] = Pc0; v[C2_Pcp] = Pcp; v[C2_Pcm] = Pcm;
+      v[C2_Eb] = Eb;
+      v[C2_Pb1] = Pb0;
+      v[C2_Pbp] = Pbp;
+      v[C2_Pbm] = Pbm;
       T cfac = 2.0 / sq3142;
       v[C2_c] = cfac;
       v[C2_fp] = cfac * (rr43 / (rrp3 * rrp4));
@@ -1082,6 +1098,7 @@ KG_INLINE RadialOut<T> radial_eval(const RadialConsts<T>& rc, const JacobiLadder
 // total Mino time (kerr_raytracing_utils.py:382-548); assignments are made in
 // the reference's order so overlapping masks resolve the same way.
 // ---------------------------------------------------------------------------
+// The integrals of all cases in one place, as in radial_consts.
 template <class T> KG_INLINE T mino_total(const RayScalars<T>& c, const PixelSetup<T>& px) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
@@ -1090,31 +1107,41 @@ template <class T> KG_INLINE T mino_total(const RayScalars<T>& c, const PixelSet
   const bool im3 = !(val(px.ri[2]) == 0.0);
   const T& rplus = c.rplus;
   const double r_o = c.r_o;
-  T out = T(0.0);
-  if (iv) {
+  const bool reg2 = !im3 && val(px.rr[2]) < val(rplus);
+  const bool reg1 = !im3 && val(px.rr[2]) > val(rplus);
+  if (!(reg2 || reg1 || iv || im3)) return T(0.0);
+  T k, pref;
+  Amp<T> Ao, Ah;  // the observer's and the horizon's amplitudes
+  if (reg2 || reg1) {
+    T rr1 = px.rr[0], rr2 = px.rr[1], rr3 = px.rr[2], rr4 = px.rr[3];
+    T rr31 = rr3 - rr1, rr32 = rr3 - rr2, rr41 = rr4 - rr1, rr42 = rr4 - rr2;
+    k = (rr32 * rr41) / (rr31 * rr42);
+    T x2ro = c.r_o_inf ? ksqrt(rr31 / rr41) : ksqrt((rr31 * (r_o - rr4)) / (rr41 * (r_o - rr3)));
+    pref = 2.0 / ksqrt(rr31 * rr42);
+    Ao = amp_from_sc(x2ro, ksqrt((1.0 - x2ro) * (1.0 + x2ro)));
+    Ah = Ao;
+    if (reg2) Ah = amp_from_sin(ksqrt((rr31 * (rplus - rr4)) / (rr41 * (rplus - rr3))));
+  } else if (iv) {
     T a1 = px.ri[3], b1 = px.rr[3], a2 = px.ri[1], b2 = px.rr[1];
     T CC = ksqrt(sq(a1 - a2) + sq(b1 - b2));
     T DD = ksqrt(sq(a1 + a2) + sq(b1 - b2));
-    T k4 = (4.0 * CC * DD) / sq(CC + DD);
+    k = (4.0 * CC * DD) / sq(CC + DD);
     T g0 = ksqrt((4.0 * a2 * a2 - sq(CC - DD)) / (sq(CC + DD) - 4.0 * a2 * a2));
     T x4rp = (rplus + b1) / a2;
-    T pref = 2.0 / (CC + DD);
-    T K = ellip_K(k4);
+    pref = 2.0 / (CC + DD);
     T sh, ch, so, co;
     atan_sum_sc(x4rp, g0, false, sh, ch);
     atan_sum_sc(c.r_o_inf ? T(0.0) : (r_o + b1) / a2, g0, c.r_o_inf, so, co);
-    T Ihor = pref * legendre_F(legendre_base(amp_from_sc(sh, ch), k4), K);
-    T Iobs = pref * legendre_F(legendre_base(amp_from_sc(so, co), k4), K);
-    out = Iobs - Ihor;
-  }
-  if (im3 && !iv) {
+    Ah = amp_from_sc(sh, ch);
+    Ao = amp_from_sc(so, co);
+  } else {
     T a1 = px.ri[3], b1 = px.rr[3];
     T rr1 = px.rr[0], rr2 = px.rr[1];
     T rr21 = rr2 - rr1;
     T rrp1 = rplus - rr1, rrp2 = rplus - rr2;
     T AA = ksqrt(a1 * a1 + sq(b1 - rr2));
     T BB = ksqrt(a1 * a1 + sq(b1 - rr1));
-    T k3 = (sq(AA + BB) - rr21 * rr21) / (4.0 * AA * BB);
+    k = (sq(AA + BB) - rr21 * rr21) / (4.0 * AA * BB);
     T x3rp = (AA * rrp1 - BB * rrp2) / (AA * rrp1 + BB * rrp2);
     T x3ro;
     if (c.r_o_inf) {
@@ -1123,33 +1150,14 @@ template <class T> KG_INLINE T mino_total(const RayScalars<T>& c, const PixelSet
       T rro1 = r_o - rr1, rro2 = r_o - rr2;
       x3ro = (AA * rro1 - BB * rro2) / (AA * rro1 + BB * rro2);
     }
-    T pref = 1.0 / ksqrt(AA * BB);
-    T K = ellip_K(k3);
-    T Ihor = pref * legendre_F(legendre_base(amp_from_cos(x3rp), k3), K);
-    T Iobs = pref * legendre_F(legendre_base(amp_from_sc(ksqrt((1.0 - x3ro) * (1.0 + x3ro)), x3ro), k3), K);
-    out = Iobs - Ihor;
+    pref = 1.0 / ksqrt(AA * BB);
+    Ah = amp_from_cos(x3rp);
+    Ao = amp_from_sc(ksqrt((1.0 - x3ro) * (1.0 + x3ro)), x3ro);
   }
-  if (!im3) {
-    const bool reg2 = val(px.rr[2]) < val(rplus);
-    const bool reg1 = val(px.rr[2]) > val(rplus);
-    if (reg2 || reg1) {
-      T rr1 = px.rr[0], rr2 = px.rr[1], rr3 = px.rr[2], rr4 = px.rr[3];
-      T rr31 = rr3 - rr1, rr32 = rr3 - rr2, rr41 = rr4 - rr1, rr42 = rr4 - rr2;
-      T k2 = (rr32 * rr41) / (rr31 * rr42);
-      T x2ro = c.r_o_inf ? ksqrt(rr31 / rr41) : ksqrt((rr31 * (r_o - rr4)) / (rr41 * (r_o - rr3)));
-      T pref = 2.0 / ksqrt(rr31 * rr42);
-      T K = ellip_K(k2);
-      T Iobs = pref * legendre_F(legendre_base(amp_from_sc(x2ro, ksqrt((1.0 - x2ro) * (1.0 + x2ro))), k2), K);
-      if (reg2) {
-        T x2rp = ksqrt((rr31 * (rplus - rr4)) / (rr41 * (rplus - rr3)));
-        T Ihor = pref * legendre_F(legendre_base(amp_from_sin(x2rp), k2), K);
-        out = Iobs - Ihor;
-      } else {
-        out = 2.0 * Iobs;
-      }
-    }
-  }
-  return out;
+  const T K = ellip_K(k);
+  const T Iobs = pref * legendre_F(legendre_base(Ao, k), K);
+  if (reg1) return 2.0 * Iobs;
+  return Iobs - pref * legendre_F(legendre_base(Ah, k), K);
 }
 
 // Full pixel setup: conserved quantities (with the spin-zero eta fix),

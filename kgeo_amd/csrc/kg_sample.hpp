@@ -337,6 +337,13 @@ KG_INLINE uint32_t theta_pixel(const double* __restrict__ plan, int64_t stride, 
   jacobi_ladder(tc.v[TH_mp], lad);
   const bool walk = WALK && walk_ok(o, any_step_zero);
   bool bad;
+  if constexpr (!WALK) {
+    tc.kind = k;
+    // one loop for all kinds, whose integrals a mixed wave then runs once
+    bad = k == THK_NONE ? theta_loop<T, THK_NONE, DO_PHI_T>(o, tc, lad, i, j0, j1, stop, any_step_zero)
+                        : theta_loop<T, -1, DO_PHI_T>(o, tc, lad, i, j0, j1, stop, any_step_zero);
+    return loop_status(bad, lad);
+  }
   switch (k) {
     case THK_ORD:
       bad = walk ? theta_loop_walk<T, THK_ORD, DO_PHI_T>(o, tc, lad, i, j0, j1, stop)
@@ -368,6 +375,10 @@ KG_INLINE uint32_t radial_pixel(const RayScalars<T>& c, const double* __restrict
   jacobi_ladder(rc.v[R_k], lad);
   const bool walk = WALK && walk_ok(o, any_step_zero) && lad.n >= 0;
   bool bad;
+  if constexpr (!WALK) {
+    bad = radial_loop<T, -1, DO_PHI_T>(o, rc, lad, cmb, i, j0, j1, stop, any_step_zero);
+    return loop_status(bad, lad);
+  }
   switch (rc.rcase) {
     case 4:
       bad = walk ? radial_loop_walk<T, 4, DO_PHI_T>(o, rc, lad, cmb, i, j0, j1, stop)

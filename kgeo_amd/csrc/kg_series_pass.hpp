@@ -106,10 +106,10 @@ KG_INLINE float wave_min(float x) {
 }
 
 // d cos(theta)/dtau from the Jacobi state at a sample (theta_out's cos theta).
-template <class T, int KIND>
+template <class T>
 KG_INLINE void theta_motion(const ThetaConsts<T>& tc, const ThState<T>& st, T& c, T& u) {
   const T* v = tc.v;
-  if (KIND == THK_VORT) {
+  if (tc.kind == THK_VORT) {
     c = v[TH_h] * ksqrt(v[TH_A] + v[TH_B] * (st.s * st.s));
     u = -(v[TH_w] * v[TH_B]) * (st.s * st.c * st.d) / c;
   } else {
@@ -119,16 +119,16 @@ KG_INLINE void theta_motion(const ThetaConsts<T>& tc, const ThState<T>& st, T& c
 }
 
 // d(1/r)/dtau from the Jacobi state at a sample (radial_out's r).
-template <class T, int CASE> KG_INLINE T radial_motion(const RadialConsts<T>& rc, const RState<T>& st) {
+template <class T> KG_INLINE T radial_motion(const RadialConsts<T>& rc, const RState<T>& st) {
   const T* v = rc.v;
   const T& Xs = v[R_Xs];
-  if (CASE == 4) {
+  if (rc.rcase == 4) {
     const T& g0 = v[C4_g0];
     const T den = st.c + g0 * st.s;
     const T num = -v[C4_a2] * (g0 * st.c - st.s) - v[C4_b1] * den;  // r den
     return v[C4_a2] * Xs * st.d * (1.0 + g0 * g0) / (num * num);
   }
-  if (CASE == 3) {
+  if (rc.rcase == 3) {
     const T &AA = v[C3_AA], &BB = v[C3_BB], &r1 = v[C3_rr1], &r2 = v[C3_rr2];
     const T num = (BB * r2 - AA * r1) + (BB * r2 + AA * r1) * st.c;
     return 2.0 * AA * BB * (r2 - r1) * Xs * (st.s * st.d) / (num * num);
@@ -139,47 +139,36 @@ template <class T, int CASE> KG_INLINE T radial_motion(const RadialConsts<T>& rc
 
 // Theta head hd (0 the last sample, b the anchor of block b) of output pixel
 // i: theta and the parked G_phi, G_t of its sample, and an anchor's motion.
-template <class T, int KIND>
-KG_INLINE bool series_theta_head(const SampleOut& o, const ThetaConsts<T>& tc, const JacobiLadder<T>& lad, int64_t i,
-                                 int64_t hd, int64_t nb, double stop, const Records& rt, int64_t col) {
-  const int64_t j = hd == 0 ? o.ngeo - 1 : series_start(o.ngeo, hd, nb);
-  WalkStep<T, 1> w;
-  theta_init(tc, w);
-  const double tau = mino_tau(j, o.ngeo, stop, false);
-  const T arg = theta_arg(tc, T(tau));
-  ThState<T> ts;
-  WalkState<T, 1> st;
-  theta_direct<T, KIND, true>(tc, lad, w, arg, ts, st);
-  T th = T(0.0), Gph = T(0.0), Gt = T(0.0);
-  theta_out<T, KIND>(tc, arg, ts, true, th, Gph, Gt);
-  if (hd > 0) {
-    T c, u;
-    theta_motion<T, KIND>(tc, ts, c, u);
-    // next to a singularity of Pi (walk_enter) the anchor is not used
-    if (!kfinite(val(st.P[0]))) c = T(NAN);
-    *rt.at(hd, kThSFields, 0, col) = val(c);
-    *rt.at(hd, kThSFields, 1, col) = val(u);
-    *rt.at(hd, kThSFields, 2, col) = val(Gph);
-    *rt.at(hd, kThSFields, 3, col) = val(Gt);
-  }
-  return theta_store<T, true>(o, j * o.npix + i, tau, th, Gph, Gt);
-}
-
 template <class T = double>
 KG_INLINE uint32_t series_theta_head_pixel(const double* __restrict__ plan, int64_t stride, int64_t p, uint32_t gflags,
                                            const SampleOut& o, int64_t i, int64_t hd, int64_t nb, const Records& rt) {
   ThetaConsts<T> tc;
   const ThetaPick tp = theta_pick(plan, stride, p, gflags, o, tc);
   if (!tp.walk) return 0u;
+  tc.kind = tp.kind;
   JacobiLadder<T> lad;
   jacobi_ladder(tc.v[TH_mp], lad);
-  bool bad;
-  switch (tp.kind) {
-    case THK_ORD: bad = series_theta_head<T, THK_ORD>(o, tc, lad, i, hd, nb, tp.stop, rt, p); break;
-    case THK_ORD_K0: bad = series_theta_head<T, THK_ORD_K0>(o, tc, lad, i, hd, nb, tp.stop, rt, p); break;
-    default: bad = series_theta_head<T, THK_VORT>(o, tc, lad, i, hd, nb, tp.stop, rt, p); break;
+  const int64_t j = hd == 0 ? o.ngeo - 1 : series_start(o.ngeo, hd, nb);
+  WalkStep<T, 1> w;
+  theta_init(tc, w);
+  const double tau = mino_tau(j, o.ngeo, tp.stop, false);
+  const T arg = theta_arg(tc, T(tau));
+  ThState<T> ts;
+  WalkState<T, 1> st;
+  theta_direct<T, -1, true>(tc, lad, w, arg, ts, st);
+  T th = T(0.0), Gph = T(0.0), Gt = T(0.0);
+  theta_out<T, -1>(tc, arg, ts, true, th, Gph, Gt);
+  if (hd > 0) {
+    T c, u;
+    theta_motion<T>(tc, ts, c, u);
+    // next to a singularity of Pi (walk_enter) the anchor is not used
+    if (!kfinite(val(st.P[0]))) c = T(NAN);
+    *rt.at(hd, kThSFields, 0, p) = val(c);
+    *rt.at(hd, kThSFields, 1, p) = val(u);
+    *rt.at(hd, kThSFields, 2, p) = val(Gph);
+    *rt.at(hd, kThSFields, 3, p) = val(Gt);
   }
-  return loop_status(bad, lad);
+  return loop_status(theta_store<T, true>(o, j * o.npix + i, tau, th, Gph, Gt), lad);
 }
 
 // Radial head hd: the sample's r and radial integrals, and an anchor's motion.
@@ -187,9 +176,16 @@ KG_INLINE uint32_t series_theta_head_pixel(const double* __restrict__ plan, int6
 // argument is up to 6e-11 of r_o for rays near the critical curve, where the
 // plan's rounded roots place the observer; the closed form keeps sample 0
 // with the samples it gives next to it).
-template <class T, int CASE>
-KG_INLINE uint32_t series_radial_head(const double* __restrict__ plan, int64_t stride, int64_t p, const SampleOut& o,
-                                      int64_t i, int64_t hd, int64_t nb, const Records& rt) {
+template <class T = double>
+KG_INLINE uint32_t series_radial_head_pixel(const double* __restrict__ plan, int64_t stride, int64_t p,
+                                            uint32_t gflags, const SampleOut& o, int64_t i, int64_t hd, int64_t nb,
+                                            double r_o, const Records& rt) {
+  if (!radial_walks(o, gflags, plan[static_cast<int64_t>(PL_R + R_k) * stride + p])) {
+    // its blocks leave every sample to the fixup pass, but an early block 0
+    // (series_block_pixel), which cannot know, still writes its own
+    if (hd == 0 && o.r) o.r[i] = r_o;
+    return 0u;
+  }
   RadialConsts<T> rc;
   T lam;
   double stop;
@@ -197,33 +193,37 @@ KG_INLINE uint32_t series_radial_head(const double* __restrict__ plan, int64_t s
   JacobiLadder<T> lad;
   jacobi_ladder(rc.v[R_k], lad);
   const int64_t j = hd == 0 ? o.ngeo - 1 : series_start(o.ngeo, hd, nb);
-  WalkStep<T, 3> w;
-  radial_init<T, CASE>(rc, w);
   const double tau = mino_tau(j, o.ngeo, stop, false);
   const T dv = rc.v[R_Xs] * tau;
   const T X = rc.v[R_U0] - dv;
   RState<T> rs;
-  WalkState<T, 3> st;
-  T lb[3];
-  radial_direct<T, CASE, true>(rc, lad, w, X, dv, rs, st, lb);
-  const RadialOut<T> ro = radial_out<T, CASE>(rc, T(tau), rs, true);
+  radial_state<T, -1>(rc, lad, X, dv, true, rs);
+  const RadialOut<T> ro = radial_out<T, -1>(rc, T(tau), rs, true);
   T v = T(0.0);
   if (hd == 0 && o.r && o.ngeo > 1) {
     RState<T> r0;
     r0.s = rc.v[R_sn0];
     r0.c = rc.v[R_cn0];
     r0.d = rc.v[R_dn0];
-    o.r[i] = val(radial_out<T, CASE>(rc, T(0.0), r0, false).r);
+    o.r[i] = val(radial_out<T, -1>(rc, T(0.0), r0, false).r);
   }
   if (hd > 0) {
-    v = radial_motion<T, CASE>(rc, rs);
+    v = radial_motion<T>(rc, rs);
     // next to a singularity of an integral (walk_enter, block_log_enter)
     // the closed formulas lose digits: the anchor is not used
     bool ok = kfinite(val(v));
+    WalkStep<T, 3> w;
+    radial_init<T, -1>(rc, w);
+    const bool blocks = rc.rcase == 3 || rc.rcase == 4;
     // below MINSPIN case 3 has no third-kind part of I_-
-    const int np = (CASE == 3 && val(rc.v[C3_hasm]) == 0.0) ? 2 : 3;
+    const int np = (rc.rcase == 3 && val(rc.v[C3_hasm]) == 0.0) ? 2 : 3;
 #pragma unroll
-    for (int q = 0; q < 3; ++q) ok = ok & ((q >= np) | (kfinite(val(st.P[q])) & kfinite(val(lb[q]))));
+    for (int q = 0; q < 3; ++q) {
+      WalkState<T, 3> st;
+      walk_enter(w, q, rs.Pi[q], X, rs.s, rs.c, rs.d, st);
+      const bool fine = kfinite(val(st.P[q])) & (!blocks | kfinite(val(block_log_enter(rs.lg[q]))));
+      ok = ok & ((q >= np) | fine);
+    }
     if (!ok) v = T(NAN);
   }
   *rt.at(hd, kRSFields, 0, p) = val(ro.r);
@@ -233,25 +233,6 @@ KG_INLINE uint32_t series_radial_head(const double* __restrict__ plan, int64_t s
   *rt.at(hd, kRSFields, 4, p) = val(ro.I2);
   *rt.at(hd, kRSFields, 5, p) = val(v);
   return loop_status(false, lad);
-}
-
-template <class T = double>
-KG_INLINE uint32_t series_radial_head_pixel(const double* __restrict__ plan, int64_t stride, int64_t p,
-                                            uint32_t gflags, const SampleOut& o, int64_t i, int64_t hd,
-                                            int64_t nb, double r_o, const Records& rt) {
-  const int rcase = static_cast<int>(plan[static_cast<int64_t>(PL_RCASE) * stride + p]);
-  const double m = plan[static_cast<int64_t>(PL_R + R_k) * stride + p];
-  if (!radial_walks(o, gflags, m)) {
-    // its blocks leave every sample to the fixup pass, but an early block 0
-    // (series_block_pixel), which cannot know, still writes its own
-    if (hd == 0 && o.r) o.r[i] = r_o;
-    return 0u;
-  }
-  switch (rcase) {
-    case 4: return series_radial_head<T, 4>(plan, stride, p, o, i, hd, nb, rt);
-    case 3: return series_radial_head<T, 3>(plan, stride, p, o, i, hd, nb, rt);
-    default: return series_radial_head<T, 2>(plan, stride, p, o, i, hd, nb, rt);
-  }
 }
 
 // A head's sample: r and the combination of its radial record with the
