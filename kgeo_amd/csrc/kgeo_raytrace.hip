@@ -155,8 +155,11 @@ __global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2)))
 
 // ---------------------------------------------------------------------------
 // Direct sample kernels (caller-given Mino times, ngeo <= 2): grid (pixel
-// blocks, sample chunks).  kg_theta writes theta and parks G_phi, G_t in ph,
-// t; kg_radial writes r and combines phi, t, sigma (kg_sample.hpp).
+// blocks, sample chunks), one wave per SIMD (held to two, kg_radial spills 273
+// registers: 0.23 for 0.18 ms on 150 x 140 pixels x 12 Mino times).  Bound by
+// the latency of one wave's chains, and by its first pass over the code.
+// kg_theta writes theta and parks G_phi, G_t in ph, t; kg_radial writes r and
+// combines phi, t, sigma (kg_sample.hpp).
 // ---------------------------------------------------------------------------
 struct SampleArgs {
   const double* plan;
@@ -167,21 +170,19 @@ struct SampleArgs {
 };
 
 template <bool DO_PHI_T>
-__global__ __launch_bounds__(kBlock) void kg_theta(DevParams p, SampleArgs a) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+__global__ __launch_bounds__(kPassBlock) void kg_theta(DevParams p, SampleArgs a) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
   if (i >= p.npix) return;
-  const int64_t j0 = chunk_start(p.ngeo, blockIdx.y, a.chunks);
-  const int64_t j1 = chunk_start(p.ngeo, blockIdx.y + 1, a.chunks);
+  const int64_t j0 = p.ngeo * blockIdx.y / a.chunks, j1 = p.ngeo * (blockIdx.y + 1) / a.chunks;
   const uint32_t st = theta_pixel<DO_PHI_T, double, false>(a.plan, p.npix, i, a.gflags[0], a.out, i, j0, j1);
   if (a.status && st) atomicOr(&a.status[i], st);
 }
 
 template <bool DO_PHI_T>
-__global__ __launch_bounds__(kBlock) void kg_radial(DevParams p, SampleArgs a) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+__global__ __launch_bounds__(kPassBlock) void kg_radial(DevParams p, SampleArgs a) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
   if (i >= p.npix) return;
-  const int64_t j0 = chunk_start(p.ngeo, blockIdx.y, a.chunks);
-  const int64_t j1 = chunk_start(p.ngeo, blockIdx.y + 1, a.chunks);
+  const int64_t j0 = p.ngeo * blockIdx.y / a.chunks, j1 = p.ngeo * (blockIdx.y + 1) / a.chunks;
   const uint32_t st = radial_pixel<DO_PHI_T, double, false>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, j0, j1);
   if (a.status && st) atomicOr(&a.status[i], st);
 }
@@ -331,18 +332,24 @@ __global__ __launch_bounds__(kBlock) void kg_turnings(DevParams p, const double*
   }
 }
 
-// Samples per lane chunking: split ngeo so that about 2^21 (pixel, chunk)
-// lanes exist (256 CUs x 128 waves of 64 over the kernels' lifetime: more
-// lanes than the chip holds at once lets waves that finish early be
-// replaced; measured at 512^2 x 500, 8 chunks run 2 % faster than 4 and as
-// fast as 15), keeping chunks >= 32 samples so the walk's per-chunk set-up
-// stays a few percent of the work.
+// Sample chunks per pixel of the direct loops (one lane each; the results do
+// not depend on it).  A sample costs thousands of instructions (three Carlson
+// R_J) and a lane's set-up about a hundred (its plan slots, the Landen
+// ladder), so few pixels take one sample per lane, until 2^19 lanes are there
+// (eight times the 1024 waves that kg_radial keeps resident); many pixels
+// chunks of at least 32 samples, up to 2^21 lanes.  150 x 140 pixels x 12
+// Mino times: kg_theta 94 and kg_radial 240 us with 1 chunk, 44 and 79 with
+// 12; the whole call 0.36, 0.19, 0.195, 0.184 and 0.178 ms with 1, 3, 4, 6
+// and 12.
 int pick_chunks(int64_t npix, int64_t ngeo) {
-  const int64_t target_lanes = 256LL * 128 * 64;
-  int64_t c = (target_lanes + npix - 1) / (npix > 0 ? npix : 1);
-  if (c < 1) c = 1;
+  const int64_t np = npix > 0 ? npix : 1;
+  int64_t c = (256LL * 128 * 64 + np - 1) / np;
   const int64_t max_c = ngeo / 32 > 0 ? ngeo / 32 : 1;
   if (c > max_c) c = max_c;
+  int64_t few = (1LL << 19) / np;
+  if (few > ngeo) few = ngeo;
+  if (few > c) c = few;
+  if (c < 1) c = 1;
   if (c > 65535) c = 65535;
   return static_cast<int>(c);
 }
@@ -552,13 +559,16 @@ int run_sample(const kgeo_ray_params* p, int64_t ngeo, const double* tau_in, dou
   if (!t || !ph) return fail_msg(KGEO_E_ARG, "t and ph outputs are required");
   const uint32_t* gflags = static_cast<const uint32_t*>(ws);
   const double* plan = reinterpret_cast<const double*>(static_cast<const char*>(ws) + kFlagBytes);
-  const unsigned nb = static_cast<unsigned>((d.npix + kBlock - 1) / kBlock);
+  const unsigned nb = static_cast<unsigned>((d.npix + kPassBlock - 1) / kPassBlock);
   const int chunks = kgeo_sample_chunks(d.npix, ngeo);
   dim3 grid(nb, static_cast<unsigned>(chunks));
   SampleArgs a{plan, gflags, SampleOut{tau_in, tau, t, r, th, ph, sig, d.npix, ngeo}, status, chunks};
   // the linspace grid takes the series (heads, series, fixup); caller-given
   // Mino times and grids of at most two samples are evaluated directly
   if (!tau_in && ngeo > 2) return run_series(d, a, ws, st);
+  hipLaunchKernelGGL(kg_theta<true>, grid, dim3(kPassBlock), 0, st, d, a);
+  int rc = check_launch("kg_theta");
+  if (rc) return rc;
   {
     // the plan's radial constants come from the side stream (run_plan)
     std::lock_guard<std::mutex> lock(g_side_mu);
@@ -566,10 +576,7 @@ int run_sample(const kgeo_ray_params* p, int64_t ngeo, const double* tau_in, dou
     if (ss && hipStreamWaitEvent(st, ss->planned, 0) != hipSuccess)
       return fail_msg(KGEO_E_HIP, "wait for the plan failed");
   }
-  hipLaunchKernelGGL(kg_theta<true>, grid, dim3(kBlock), 0, st, d, a);
-  int rc = check_launch("kg_theta");
-  if (rc) return rc;
-  hipLaunchKernelGGL(kg_radial<true>, grid, dim3(kBlock), 0, st, d, a);
+  hipLaunchKernelGGL(kg_radial<true>, grid, dim3(kPassBlock), 0, st, d, a);
   return check_launch("kg_radial");
 }
 
@@ -661,7 +668,7 @@ int kgeo_crossings(const kgeo_ray_params* p, const double* alpha, const double* 
   if (p->npix == 0 || ntau == 0) return KGEO_OK;
   if (!alpha || !beta || !tau) return fail_msg(KGEO_E_ARG, "NULL array");
   DevParams d = make_dev(p, ntau);
-  const unsigned nb = static_cast<unsigned>((d.npix + kBlock - 1) / kBlock);
+  const unsigned nb = static_cast<unsigned>((d.npix + kPassBlock - 1) / kPassBlock);
   hipLaunchKernelGGL(kg_counts, dim3(nb), dim3(kBlock), 0, static_cast<hipStream_t>(stream), d, alpha, beta, tau,
                      ntau, n_equatorial, n_poloidal);
   return check_launch("kg_counts");
@@ -677,7 +684,7 @@ int kgeo_turnings(const kgeo_ray_params* p, const double* alpha, const double* b
   if (p->npix == 0 || ntau == 0) return KGEO_OK;
   if (!alpha || !beta || !tau) return fail_msg(KGEO_E_ARG, "NULL array");
   DevParams d = make_dev(p, ntau);
-  const unsigned nb = static_cast<unsigned>((d.npix + kBlock - 1) / kBlock);
+  const unsigned nb = static_cast<unsigned>((d.npix + kPassBlock - 1) / kPassBlock);
   hipLaunchKernelGGL(kg_turnings, dim3(nb), dim3(kBlock), 0, static_cast<hipStream_t>(stream), d, alpha, beta, tau,
                      ntau, n_angular, turns_theta, turns_r);
   return check_launch("kg_turnings");
