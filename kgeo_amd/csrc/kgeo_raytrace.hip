@@ -285,33 +285,54 @@ __global__ __launch_bounds__(kBlock) void kg_ellip_pi(const double* __restrict__
   out[i] = (kfabs(phi[i]) <= 1.0e-10) ? phi[i] : ellip_pi_amp(L, nn, mm, Pc);
 }
 
+// Samples a count kernel's lane loads before it works on them.  One lane per
+// pixel leaves few waves (1024 for 256 x 256 pixels, one per SIMD), each with
+// the pixel's elliptic integrals ahead of its samples, so the loads in flight
+// are to hide the memory's latency: 256 x 256 pixels x 100 samples take 39 us
+// (kg_counts) and 49 us (kg_turnings), 80 and 94 with one load at a time
+// (157 and 137 MB: 31 and 27 us at the rate of a large copy).
+constexpr int kCountAhead = 8;
+
+// Calls f(offset, tau) for each sample of pixel i, kCountAhead loads at a time.
+template <class F>
+__device__ inline void count_samples(const double* __restrict__ tau, int64_t ntau, int64_t npix, int64_t i, F f) {
+  const double* __restrict__ t = tau + i;
+  int64_t j = 0;
+  for (; j + kCountAhead <= ntau; j += kCountAhead) {
+    double x[kCountAhead];
+#pragma unroll
+    for (int q = 0; q < kCountAhead; ++q) x[q] = t[(j + q) * npix];
+#pragma unroll
+    for (int q = 0; q < kCountAhead; ++q) f((j + q) * npix + i, x[q]);
+  }
+  for (; j < ntau; ++j) f(j * npix + i, t[j * npix]);
+}
+
 // Per-sample counts (kerr_raytracing_utils.py:551-684): equatorial crossings
 // and poloidal orbits, one lane per pixel (kg_counts.hpp).
-__global__ __launch_bounds__(kBlock) void kg_counts(DevParams p, const double* __restrict__ alpha,
-                                                    const double* __restrict__ beta, const double* __restrict__ tau,
-                                                    int64_t ntau, double* __restrict__ n_eq,
-                                                    double* __restrict__ n_pol) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+__global__ __launch_bounds__(kPassBlock) void kg_counts(DevParams p, const double* __restrict__ alpha,
+                                                        const double* __restrict__ beta,
+                                                        const double* __restrict__ tau, int64_t ntau,
+                                                        double* __restrict__ n_eq, double* __restrict__ n_pol) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
   if (i >= p.npix) return;
   const double be = beta[i];
   const CountConsts k = count_consts(p.c, alpha[i], be);
-  for (int64_t j = 0; j < ntau; ++j) {
-    const int64_t o = j * p.npix + i;
-    const double tj = tau[o];
+  count_samples(tau, ntau, p.npix, i, [&](int64_t o, double tj) {
     if (n_eq) n_eq[o] = n_equatorial_at(k, p.north != 0, be, tj);
     if (n_pol) n_pol[o] = n_poloidal_at(k, tj);
-  }
+  });
 }
 
 // Turning points passed by each Mino time (kerr_raytracing_utils.py:686-826),
 // one lane per pixel: the reference's fractional n_angular_turnings, its
 // floor (theta turning points) and the radial turning point (kg_counts.hpp).
-__global__ __launch_bounds__(kBlock) void kg_turnings(DevParams p, const double* __restrict__ alpha,
-                                                      const double* __restrict__ beta,
-                                                      const double* __restrict__ tau, int64_t ntau,
-                                                      double* __restrict__ n_ang, int32_t* __restrict__ turns_th,
-                                                      int8_t* __restrict__ turns_r) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+__global__ __launch_bounds__(kPassBlock) void kg_turnings(DevParams p, const double* __restrict__ alpha,
+                                                          const double* __restrict__ beta,
+                                                          const double* __restrict__ tau, int64_t ntau,
+                                                          double* __restrict__ n_ang, int32_t* __restrict__ turns_th,
+                                                          int8_t* __restrict__ turns_r) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
   if (i >= p.npix) return;
   const double al = alpha[i], be = beta[i];
   const bool ang = n_ang || turns_th;
@@ -319,9 +340,7 @@ __global__ __launch_bounds__(kBlock) void kg_turnings(DevParams p, const double*
   if (ang) k = count_consts(p.c, al, be);
   RadialTurn rt{false, 0.0};
   if (turns_r) rt = radial_turn_consts(p.c, al, be);
-  for (int64_t j = 0; j < ntau; ++j) {
-    const int64_t o = j * p.npix + i;
-    const double tj = tau[o];
+  count_samples(tau, ntau, p.npix, i, [&](int64_t o, double tj) {
     if (ang) {
       const double n = n_angular_at(k, be, tj);
       if (n_ang) n_ang[o] = n;
@@ -329,7 +348,7 @@ __global__ __launch_bounds__(kBlock) void kg_turnings(DevParams p, const double*
       if (turns_th) turns_th[o] = (n == n && kfabs(n) < 2.0e9) ? static_cast<int32_t>(kfloor(n)) : INT32_MIN;
     }
     if (turns_r) turns_r[o] = static_cast<int8_t>(radial_turns_at(rt, tj));
-  }
+  });
 }
 
 // Sample chunks per pixel of the direct loops (one lane each; the results do
@@ -669,7 +688,7 @@ int kgeo_crossings(const kgeo_ray_params* p, const double* alpha, const double* 
   if (!alpha || !beta || !tau) return fail_msg(KGEO_E_ARG, "NULL array");
   DevParams d = make_dev(p, ntau);
   const unsigned nb = static_cast<unsigned>((d.npix + kPassBlock - 1) / kPassBlock);
-  hipLaunchKernelGGL(kg_counts, dim3(nb), dim3(kBlock), 0, static_cast<hipStream_t>(stream), d, alpha, beta, tau,
+  hipLaunchKernelGGL(kg_counts, dim3(nb), dim3(kPassBlock), 0, static_cast<hipStream_t>(stream), d, alpha, beta, tau,
                      ntau, n_equatorial, n_poloidal);
   return check_launch("kg_counts");
 }
@@ -685,7 +704,7 @@ int kgeo_turnings(const kgeo_ray_params* p, const double* alpha, const double* b
   if (!alpha || !beta || !tau) return fail_msg(KGEO_E_ARG, "NULL array");
   DevParams d = make_dev(p, ntau);
   const unsigned nb = static_cast<unsigned>((d.npix + kPassBlock - 1) / kPassBlock);
-  hipLaunchKernelGGL(kg_turnings, dim3(nb), dim3(kBlock), 0, static_cast<hipStream_t>(stream), d, alpha, beta, tau,
+  hipLaunchKernelGGL(kg_turnings, dim3(nb), dim3(kPassBlock), 0, static_cast<hipStream_t>(stream), d, alpha, beta, tau,
                      ntau, n_angular, turns_theta, turns_r);
   return check_launch("kg_turnings");
 }
