@@ -10,14 +10,14 @@
 //                        straddles two images and the image-wide predicates
 //                        (any eta > 0, any zero grid step) are per-image
 //                        wave ballots.
-//   kg_batch_heads<P>    the theta, then the radial heads of the plain kernels
-//                        (kg_series_pass.hpp): a fixed grid of waves taking
-//                        work items (image, 64-pixel tile, head) from an
-//                        atomic counter until the pass is empty; every wave
-//                        leaves once the counter passes the pass's item
-//                        total, so the grid always drains;
-//   kg_batch_series      the rays' blocks, items (image, tile, block,
-//                        part), in the same way;
+//   kg_batch_*_heads     the theta, then the radial heads of the plain kernels
+//                        (kg_series_pass.hpp), items (image, 64-pixel tile,
+//                        head) in strides over a fixed grid of waves;
+//   kg_batch_series      the rays' blocks: a fixed grid of waves taking
+//                        items (image, tile, block, part) from an atomic
+//                        counter until the pass is empty; every wave leaves
+//                        once the counter passes the pass's item total, so
+//                        the grid always drains;
 //   kg_batch_fixup       the queued ranges of all images, one lane per
 //                        (range, sample), by direct evaluation (grid-stride).
 // Outputs go to caller arenas: image k's [ngeo_k][npix_k] block of r, theta,
@@ -61,8 +61,8 @@ size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 // pass kinds and their per-tile work units
 enum : int { K_HEAD = 0, K_SERIES = 1, K_N = 2 };
-// counters: theta heads, radial heads, series, then the fixup queue
-enum : int { CT_THETA = 0, CT_RADIAL, CT_SERIES, CT_QUEUE, kCounters };
+// counters: series items, the fixup queue
+enum : int { CT_SERIES = 0, CT_QUEUE, kCounters };
 
 struct BatchImage {
   RayScalars<double> c;
@@ -120,7 +120,9 @@ __global__ void kg_batch_clear(BatchDev d) {
   if (threadIdx.x < kCounters) d.counter[threadIdx.x] = 0u;
 }
 
-__global__ __launch_bounds__(kBlock) void kg_batch_setup(BatchDev d) {
+// Two waves per SIMD: 0.94 ms for a 16-image survey (1.4 million slots), with 73
+// spilled registers; 1.30 at one.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_batch_setup(BatchDev d) {
   const int64_t s = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   // total_slots is a multiple of 64: whole waves leave here together
   if (s >= d.total_slots) return;
@@ -173,38 +175,60 @@ __device__ inline Records image_records(const BatchDev& d, const BatchImage& B, 
   return Records{d.rec + (theta ? B.th_rec : B.r_rec), B.slots, B.slot_off};
 }
 
-// Items (image, tile, unit) of pass KIND from `counter` until none is left;
-// f(image, its index, its pixel on this lane, whether there is one, unit).
-template <int KIND, class F> __device__ inline void batch_items(const BatchDev& d, uint32_t* counter, F f) {
-  const int lane = __lane_id();
-  for (;;) {
-    const uint32_t item = fetch_item(counter, lane);
-    if (item >= d.total_items[KIND]) break;  // scalar branch: the whole wave leaves once the pass is empty
-    const int im = find_image(d.imgs, d.nimg, static_cast<int64_t>(item), KIND);
-    const BatchImage& B = d.imgs[im];
-    const int64_t li = static_cast<int64_t>(item) - B.item_off[KIND];
-    const int64_t units = B.units[KIND];
-    const int64_t i = (li / units) * kWave + lane;
-    const bool in = i < B.npix;
-    const uint32_t st = f(B, im, in ? i : B.npix - 1, in, li % units);
-    if (in && d.status && st) atomicOr(&d.status[B.pix_off + i], st);
-    atomicAdd(&d.done[im], lane == 0 ? 1u : 0u);
-  }
+// Item `item` (image, tile, unit) of pass KIND: f(image, its index, its pixel
+// on this lane, whether there is one, unit); returns the image's index.
+template <int KIND, class F> __device__ inline int batch_item(const BatchDev& d, uint32_t item, int lane, F f) {
+  const int im = find_image(d.imgs, d.nimg, static_cast<int64_t>(item), KIND);
+  const BatchImage& B = d.imgs[im];
+  const int64_t li = static_cast<int64_t>(item) - B.item_off[KIND];
+  const int64_t units = B.units[KIND];
+  const int64_t i = (li / units) * kWave + lane;
+  const bool in = i < B.npix;
+  const uint32_t st = f(B, im, in ? i : B.npix - 1, in, li % units);
+  if (in && d.status && st) atomicOr(&d.status[B.pix_off + i], st);
+  return im;
 }
 
-template <bool THETA> __global__ __launch_bounds__(kBlock) void kg_batch_heads(BatchDev d) {
-  batch_items<K_HEAD>(d, d.counter + (THETA ? CT_THETA : CT_RADIAL),
-                      [&](const BatchImage& B, int im, int64_t i, bool in, int64_t hd) {
-                        if (!in) return 0u;
-                        const int64_t s = B.slot_off + i;
-                        const SampleOut o = image_out(d, B);
-                        const Records rt = image_records(d, B, THETA);
-                        return THETA ? series_theta_head_pixel(d.plan, d.total_slots, s, d.flags[im], o, i, hd,
-                                                               B.units[K_HEAD], rt)
-                                     : series_radial_head_pixel(d.plan, d.total_slots, s, d.flags[im], o, i, hd,
-                                                                B.units[K_HEAD], B.c.r_o, rt);
-                      });
+// Heads cost alike, so the waves share them out in strides, without a counter:
+// the fetches and the progress counts are atomics on a few words that all
+// XCDs share, about 7 ns each, and with two per item they bounded the theta
+// heads of a 16-image survey (43520 items: 0.65 ms, 0.39 now; the radial ones
+// 0.85, 0.77 now).  A wave counts an image's items and adds them once.
+template <bool THETA> __device__ inline void batch_heads(const BatchDev& d) {
+  const int lane = __lane_id();
+  const uint32_t waves = gridDim.x * (kBlock / kWave);
+  uint32_t count = 0u;
+  int last = 0;
+  for (uint32_t item = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+           static_cast<int>(blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave)));
+       item < d.total_items[K_HEAD]; item += waves) {
+    const int im = batch_item<K_HEAD>(
+        d, item, lane, [&](const BatchImage& B, int k, int64_t i, bool in, int64_t hd) {
+          if (!in) return 0u;
+          const int64_t s = B.slot_off + i;
+          const SampleOut o = image_out(d, B);
+          const Records rt = image_records(d, B, THETA);
+          return THETA ? series_theta_head_pixel(d.plan, d.total_slots, s, d.flags[k], o, i, hd, B.units[K_HEAD], rt)
+                       : series_radial_head_pixel(d.plan, d.total_slots, s, d.flags[k], o, i, hd, B.units[K_HEAD],
+                                                  B.c.r_o, rt);
+        });
+    if (im != last && count) {
+      atomicAdd(&d.done[last], lane == 0 ? count : 0u);
+      count = 0u;
+    }
+    last = im;
+    ++count;
+  }
+  if (count) atomicAdd(&d.done[last], lane == 0 ? count : 0u);
 }
+
+// theta at two waves per SIMD (0.39 ms, 0.47 at one), r at one (0.77; with 110
+// spilled registers at two 0.93)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_batch_theta_heads(BatchDev d) {
+  batch_heads<true>(d);
+}
+
+__global__ __launch_bounds__(kBlock) void kg_batch_radial_heads(BatchDev d) { batch_heads<false>(d); }
 
 // kg_series (kgeo_raytrace.hip) over all images, two waves per SIMD as there.
 // A survey of 16 images (64 .. 512 pixels a side, 50 .. 400 samples; 58 million
@@ -212,14 +236,20 @@ template <bool THETA> __global__ __launch_bounds__(kBlock) void kg_batch_heads(B
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_batch_series(BatchDev d) {
   __shared__ double sl[kBlock / kWave][SERIES_SLOTS][kWave];
   LdsSlots slots{sl[threadIdx.x / kWave], static_cast<int>(threadIdx.x % kWave)};
-  batch_items<K_SERIES>(d, d.counter + CT_SERIES, [&](const BatchImage& B, int im, int64_t i, bool in, int64_t u) {
-    BatchPush push{d.queue, d.counter + CT_QUEUE, d.qcap, static_cast<unsigned long long>(im)};
-    const SampleOut o = image_out(d, B);
-    const Records rth = image_records(d, B, true), rr = image_records(d, B, false);
-    const int64_t nb = B.units[K_HEAD], parts = B.units[K_SERIES] / nb;
-    return series_block_pixel<false, false>(B.c, d.plan, d.total_slots, B.slot_off + i, d.flags[im], o, i, in, u % nb,
-                                            nb, parts - 1 - u / nb, parts, rth, rr, slots, push);
-  });
+  const int lane = __lane_id();
+  for (;;) {
+    const uint32_t item = fetch_item(d.counter + CT_SERIES, lane);
+    if (item >= d.total_items[K_SERIES]) break;  // scalar branch: the whole wave leaves once the pass is empty
+    const int im = batch_item<K_SERIES>(d, item, lane, [&](const BatchImage& B, int k, int64_t i, bool in, int64_t u) {
+      BatchPush push{d.queue, d.counter + CT_QUEUE, d.qcap, static_cast<unsigned long long>(k)};
+      const SampleOut o = image_out(d, B);
+      const Records rth = image_records(d, B, true), rr = image_records(d, B, false);
+      const int64_t nb = B.units[K_HEAD], parts = B.units[K_SERIES] / nb;
+      return series_block_pixel<false, false>(B.c, d.plan, d.total_slots, B.slot_off + i, d.flags[k], o, i, in, u % nb,
+                                              nb, parts - 1 - u / nb, parts, rth, rr, slots, push);
+    });
+    atomicAdd(&d.done[im], lane == 0 ? 1u : 0u);
+  }
 }
 
 // one lane per (queued range, sample of the range) (grid-stride), each
@@ -469,8 +499,8 @@ int kgeo_batch_plan(const kgeo_ray_params* imgs, int32_t nimg, const kgeo_batch_
   }
   hipLaunchKernelGGL(kg_batch_clear, dim3(1), dim3(kBlock), 0, st, d);
   hipLaunchKernelGGL(kg_batch_setup, dim3(setup_blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL(kg_batch_heads<true>, dim3(blocks), dim3(kBlock), 0, st, d);
-  hipLaunchKernelGGL(kg_batch_heads<false>, dim3(blocks), dim3(kBlock), 0, st, d);
+  hipLaunchKernelGGL(kg_batch_theta_heads, dim3(blocks), dim3(kBlock), 0, st, d);
+  hipLaunchKernelGGL(kg_batch_radial_heads, dim3(blocks), dim3(kBlock), 0, st, d);
   hipLaunchKernelGGL(kg_batch_series, dim3(blocks), dim3(kBlock), 0, st, d);
   hipLaunchKernelGGL(kg_batch_fixup, dim3(blocks), dim3(kBlock), 0, st, d);
   const int lrc = blaunch("batch kernel launch (capture)");
