@@ -882,7 +882,8 @@ struct StokesArrays {
 KG_INLINE void stokes_pixel(const RayScalars<double>& c, bool north, const kgeo_emission_model& M, double alpha,
                             double beta, int nsub, double bsq0, int64_t i, const StokesArrays& o) {
   EqRay<double> e;
-  eq_ray(c, alpha, beta, e);
+  JacobiLadder<double> lad;
+  eq_ray(c, alpha, beta, e, lad);
   if (o.nmax_eq) o.nmax_eq[i] = e.vort ? -2.0 : e.N;
   if (o.n_poloidal) {
     CountConsts k;
@@ -899,7 +900,7 @@ KG_INLINE void stokes_pixel(const RayScalars<double>& c, bool north, const kgeo_
     double Ir = -1.0, rs = -1.0;
     bool zero = true;
     if (!e.vort) {
-      eq_subring(c, beta, e, m, Ir, rs);
+      eq_subring(c, beta, e, lad, m, Ir, rs);
       zero = (e.N < m) || (e.N == -1.0) || (rs <= rh) || (em.emiscut_in > 0.0 && rs < em.emiscut_in) ||
              (em.emiscut_out > 0.0 && rs > em.emiscut_out);
     }

@@ -21,7 +21,8 @@ KG_INLINE double r_equatorial2(const RayScalars<double>& c, double rho, double c
   const double alpha = cphi * rho;
   const double beta = sphi * rho;
   EqRay<double> e;
-  eq_ray(c, alpha, beta, e);
+  JacobiLadder<double> lad;
+  eq_ray(c, alpha, beta, e, lad);
   double r;
   bool outside;
   if (e.vort) {
@@ -36,7 +37,7 @@ KG_INLINE double r_equatorial2(const RayScalars<double>& c, double rho, double c
     }
   } else {
     double Ir;
-    eq_subring(c, beta, e, mbar, Ir, r);
+    eq_subring(c, beta, e, lad, mbar, Ir, r);
     outside = e.outside;
   }
   if (r <= 0.0 && outside) return kLensInf;

@@ -54,20 +54,24 @@ struct EqOut {
   uint8_t* zero_mask;
 };
 
+// Bound by FP64 issue (5500 vector instructions per wave, up to 7 complete and
+// incomplete integrals of the first kind per pixel).  The subrings' values go
+// straight to memory: in arrays indexed by the subring they lay in scratch
+// (1024 x 1024 pixels, 3 subrings: 0.24 ms, 0.21 now).
 __global__ __launch_bounds__(kLaneBlock) void kg_eq_image(EqParams p, const double* __restrict__ alpha,
                                                       const double* __restrict__ beta, EqOut o) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kLaneBlock + threadIdx.x;
   if (i >= p.npix) return;
-  EqPixel<double> e;
-  equatorial_pixel(p.c, alpha[i], beta[i], p.p_emis, p.ri, p.mbar_max, e);
+  EqLabels<double> e;
+  equatorial_pixel(p.c, alpha[i], beta[i], p.p_emis, p.ri, p.mbar_max, e,
+                   [&](int m, double I, double g, double rs, double Ir) {
+                     const int64_t q = static_cast<int64_t>(m) * p.npix + i;
+                     if (o.I) o.I[q] = I;
+                     if (o.g) o.g[q] = g;
+                     if (o.r_s) o.r_s[q] = rs;
+                     if (o.Ir) o.Ir[q] = Ir;
+                   });
   if (o.image) o.image[i] = e.image;
-  for (int m = 0; m <= p.mbar_max; ++m) {
-    const int64_t q = static_cast<int64_t>(m) * p.npix + i;
-    if (o.I) o.I[q] = e.I[m];
-    if (o.g) o.g[q] = e.g[m];
-    if (o.r_s) o.r_s[q] = e.r_s[m];
-    if (o.Ir) o.Ir[q] = e.Ir[m];
-  }
   if (o.Imax) o.Imax[i] = e.Imax;
   if (o.Nmax) o.Nmax[i] = e.Nmax;
   if (o.zero_mask) o.zero_mask[i] = static_cast<uint8_t>(e.zero_mask);
@@ -92,8 +96,9 @@ __global__ __launch_bounds__(kBlock) void kg_eq_tangent(TanParams p, const doubl
     const Dual3 pe = Dual3::seed(p.p_emis, 2);
     RayScalars<Dual3> c = make_scalars(a, th, p.r_o, 1.0);
     const Dual3 ri = r_isco(a);
-    EqPixel<Dual3> e;
-    equatorial_pixel(c, Dual3(alpha[i]), Dual3(beta[i]), pe, ri, p.mbar_max, e);
+    EqLabels<Dual3> e;
+    equatorial_pixel(c, Dual3(alpha[i]), Dual3(beta[i]), pe, ri, p.mbar_max, e,
+                     [](int, const Dual3&, const Dual3&, const Dual3&, const Dual3&) {});
     if (jac) {
       jac[i] = e.image.d[0];
       jac[p.npix + i] = e.image.d[1];
