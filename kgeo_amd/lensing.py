@@ -34,13 +34,18 @@ def default_varphis():
 
 def _curve_params(spins, incs):
     """A device array of kgeo_ray_params, one per (spin, inclination) curve,
-    with numpy's derived scalars and the observer at infinity."""
-    n = len(spins)
-    arr = (_lib.RayParams * n)()
-    for k in range(n):
-        arr[k] = _lib.make_params(float(spins[k]), R0, float(incs[k]), 1, 1, 1.0)
-    raw = np.frombuffer(bytes(arr), dtype=np.uint8).copy()
-    return torch.from_numpy(raw).to(_device())
+    with numpy's derived scalars and the observer at infinity (as
+    _lib.make_params, over arrays: 144 curves took 0.4 ms one by one)."""
+    p = np.zeros(len(spins), dtype=np.dtype(_lib.RayParams))
+    spins, incs = np.asarray(spins, np.float64), np.asarray(incs, np.float64)
+    p["a"], p["r_o"], p["th_o"], p["maxtaufrac"] = spins, R0, incs, 1.0
+    a2 = np.array([a ** 2 for a in spins.tolist()])
+    root = np.sqrt(1 - a2)
+    p["a2"], p["rplus"], p["rminus"] = a2, 1 + root, 1 - root
+    p["sin_th"], p["cos_th"] = np.sin(incs), np.cos(incs)
+    p["cos2_th"] = [c ** 2 for c in p["cos_th"]]  # scalar powers, as there (an array squares)
+    p["npix"], p["ngeo"], p["flags"] = 1, 1, _lib.KGEO_DO_PHI_T
+    return torch.from_numpy(p.view(np.uint8)).to(_device())
 
 
 def rho_of_req_device(spins, incs, reqs, mbars, varphis):
