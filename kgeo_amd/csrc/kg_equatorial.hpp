@@ -125,6 +125,7 @@ KG_INLINE void eq_ray(const RayScalars<T>& c, const T& alpha, const T& beta, EqR
   e.N = -2.0;
   if (e.vort) return;
   T up, um, ratio, a2um;
+  ObserverIntegrals<T> obs;
   {
 #if defined(__clang__)
 #pragma clang fp contract(off)
@@ -140,7 +141,7 @@ KG_INLINE void eq_ray(const RayScalars<T>& c, const T& alpha, const T& beta, EqR
     e.K = ellip_K(ratio);
     e.Fo = legendre_F(legendre_base(amp_from_sin(c.cos_th / ksqrt(up)), ratio), e.K);
     radial_roots(c, lam, eta, px);
-    e.Im = mino_total(c, px);
+    e.Im = mino_total(c, px, &obs);
     e.w = ksqrt(-a2um);
     const double x = val(e.Im) * val(e.w);
     const double Fo = val(e.Fo), K = val(e.K);
@@ -150,7 +151,7 @@ KG_INLINE void eq_ray(const RayScalars<T>& c, const T& alpha, const T& beta, EqR
       e.N = (val(beta) >= 0.0) ? kfloor((x + Fo) / (2.0 * K)) : kfloor((x - Fo) / (2.0 * K)) - 1.0;
     }
   }
-  radial_consts(c, px, false, e.rc);
+  radial_consts(c, px, false, e.rc, &obs);
   jacobi_ladder(e.rc.v[R_k], lad);
   e.outside = (val(px.ri[3]) == 0.0) && (val(px.rr[3]) > val(c.rplus)) && !(val(eta) < 0.0);
 }

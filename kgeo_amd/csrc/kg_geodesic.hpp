@@ -653,13 +653,25 @@ template <class T> KG_INLINE void atan_sum_sc(const T& x, const T& g, bool x_inf
   cb = (1.0 - x * g) / d;
 }
 
+// The first-kind integrals at the observer, which mino_total and radial_consts
+// both need: K(k) and the Legendre base at the observer's amplitude.
+template <class T> struct ObserverIntegrals {
+  T K;
+  LegendreBase<T> L;
+  int rcase = 0;  // the radial case they hold for, 0 for none
+};
+
 // The radial constants, in three stages: each case's modulus, amplitude and
 // characteristics; the elliptic integrals of all cases in one place; what each
 // case makes of them.  (A wave holds rays of all cases: with the integrals
 // inside the cases it ran them three times, and the kernels' first pass over
 // that code, fetched cold by every CU, was most of a small image's set-up.)
+// obs: mino_total's integrals, used where they are this case's (two of the seven
+// first-kind integrals of an equatorial pixel: 1024 x 1024 pixels 0.212 ms
+// without, 0.187 with; 144 x 360 lensed curve points 0.84 and 0.70).
 template <class T>
-KG_INLINE void radial_consts(const RayScalars<T>& c, const PixelSetup<T>& px, bool do_phi_t, RadialConsts<T>& rc) {
+KG_INLINE void radial_consts(const RayScalars<T>& c, const PixelSetup<T>& px, bool do_phi_t, RadialConsts<T>& rc,
+                             const ObserverIntegrals<T>* obs = nullptr) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
@@ -734,8 +746,15 @@ KG_INLINE void radial_consts(const RayScalars<T>& c, const PixelSetup<T>& px, bo
     nm = (rrm3 * rr41) / (rrm4 * rr31);
   }
   // the integrals at the observer's amplitude, and the complete ones
-  const T K = ellip_K(k);
-  const LegendreBase<T> Lb = legendre_base(amp_from_sc(sb, cb), k);
+  T K;
+  LegendreBase<T> Lb;
+  if (obs && obs->rcase == px.rcase) {
+    K = obs->K;
+    Lb = obs->L;
+  } else {
+    K = ellip_K(k);
+    Lb = legendre_base(amp_from_sc(sb, cb), k);
+  }
   const T Fb = legendre_F(Lb, K);
   const T s2b = ksqrt(1.0 - k * (sb * sb));
   v[R_k] = k;
@@ -1099,7 +1118,8 @@ KG_INLINE RadialOut<T> radial_eval(const RadialConsts<T>& rc, const JacobiLadder
 // the reference's order so overlapping masks resolve the same way.
 // ---------------------------------------------------------------------------
 // The integrals of all cases in one place, as in radial_consts.
-template <class T> KG_INLINE T mino_total(const RayScalars<T>& c, const PixelSetup<T>& px) {
+template <class T>
+KG_INLINE T mino_total(const RayScalars<T>& c, const PixelSetup<T>& px, ObserverIntegrals<T>* obs = nullptr) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
@@ -1155,7 +1175,13 @@ template <class T> KG_INLINE T mino_total(const RayScalars<T>& c, const PixelSet
     Ao = amp_from_sc(ksqrt((1.0 - x3ro) * (1.0 + x3ro)), x3ro);
   }
   const T K = ellip_K(k);
-  const T Iobs = pref * legendre_F(legendre_base(Ao, k), K);
+  const LegendreBase<T> Lo = legendre_base(Ao, k);
+  if (obs) {
+    obs->K = K;
+    obs->L = Lo;
+    obs->rcase = (reg2 || reg1) ? 2 : (iv ? 4 : 3);
+  }
+  const T Iobs = pref * legendre_F(Lo, K);
   if (reg1) return 2.0 * Iobs;
   return Iobs - pref * legendre_F(legendre_base(Ah, k), K);
 }

@@ -54,10 +54,10 @@ struct EqOut {
   uint8_t* zero_mask;
 };
 
-// Bound by FP64 issue (5500 vector instructions per wave, up to 7 complete and
+// Bound by FP64 issue (5500 vector instructions per wave, 5 complete and
 // incomplete integrals of the first kind per pixel).  The subrings' values go
 // straight to memory: in arrays indexed by the subring they lay in scratch
-// (1024 x 1024 pixels, 3 subrings: 0.24 ms, 0.21 now).
+// (1024 x 1024 pixels, 3 subrings: 0.24 ms, 0.21 without).
 __global__ __launch_bounds__(kLaneBlock) void kg_eq_image(EqParams p, const double* __restrict__ alpha,
                                                       const double* __restrict__ beta, EqOut o) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kLaneBlock + threadIdx.x;
