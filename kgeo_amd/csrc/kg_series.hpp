@@ -10,8 +10,8 @@
 // Taylor coefficients at any point follow from the ones before by the
 // Cauchy products w^2, w^3, c^2, c^3.  The integrands of t, phi and sigma
 // are rational in w and c; their series are the products' quotients,
-// integrated term by term.  One expansion (about 3.5 P^2 multiply-adds for
-// order P) replaces the elliptic functions and integrals of every sample in
+// integrated term by term.  One expansion (about 5 P^2 multiply-adds for
+// order P, on both sides of its centre) replaces the elliptic functions and integrals of every sample in
 // its step, and a sample costs one polynomial per coordinate: the
 // Gralla-Lupsasca formulas (kerr_raytracing_ana.py:126-683) are evaluated
 // only at the rays' anchors (kg_sample.hpp).  w is regular at infinity,
@@ -49,11 +49,16 @@ namespace kg {
 
 // A lane holds five coefficient arrays of kSeriesOrder + 1 doubles while it
 // samples: at order 14 two waves per SIMD fit without spills (247 of 256
-// registers; with sigma 24 values spill), at order 16 14 spill.  Measured on
-// 512 x 512 x 500 and 217 x 301 x 333 samples: order 13 2.33 and 0.83 ms, 14
-// 2.27 and 0.84, 16 2.23 and 0.88; 64 x 64 x 100 0.37, 0.365, 0.362.
+// registers; with sigma 14 values spill).  Measured at orders 12, 14 and 16
+// (ms): 512 x 512 x 500 samples 2.14, 2.08, 2.11; 217 x 301 x 333 0.70, 0.69,
+// 0.76; 64 x 64 x 100 0.31, 0.28, 0.26; a 16-image survey 8.0, 7.7, 7.8.
 constexpr int kSeriesOrder = 14;
-constexpr float kSeriesTolLog2 = -49.828921f;  // log2(1e-15)
+// Truncation: 1e-14 (of w, and in phi and t relative to 10 and 100), 3e-15 in
+// cos(theta), whose error arccos magnifies next to the axis.  Against direct
+// evaluation r and theta then agree to 1.4e-13 and 1.5e-14 or better at 99 % of the
+// samples, phi to 2e-14 (the walk by addition theorems: 2.5e-13, 3e-14, 1.6e-13).
+constexpr float kSeriesTolLog2 = -46.506993f;     // log2(1e-14)
+constexpr float kSeriesTolPolarLog2 = -48.243958f;  // log2(3e-15)
 
 // The fits' coefficients.  In the sample loops the number of instructions
 // counts, not a chain's length (two waves per SIMD and several independent
@@ -197,6 +202,8 @@ enum SeriesSlot : int {
   SF_sg,                      // y = 1 - sg c
   SF_ax,                      // -2 l sg/h
   SF_af, SF_wrap,             // the angle's factor in phi, and 2 pi of it past a pass
+  SE_w, SE_v, SE_c, SE_u,     // the state where the last expansion ended
+  SE_t, SE_f, SE_s,
   SERIES_SLOTS
 };
 
@@ -369,8 +376,9 @@ template <class T, class Slots> KG_INLINE T series_angle(const Slots& k, const T
   return atan2_fast(k(SF_ax) * u, d);
 }
 
-// The expansion at st; returns the step (in grid units) over which the
-// truncated terms stay below the tolerances.
+// The expansion about st, without the integrals' constants (series_match);
+// returns the distance (in grid units, to both sides) over which the truncated
+// terms stay below the tolerances.
 template <class T, int P, bool SIG, class Slots>
 KG_INLINE float series_expand(const RayScalars<T>& g, Slots& k, const SeriesState<T>& st, Series<T, P, SIG>& S) {
   const T &rp = g.rplus, &a2 = g.a2;
@@ -505,26 +513,13 @@ KG_INLINE float series_expand(const RayScalars<T>& g, Slots& k, const SeriesStat
     S.f[n] = S.f[n] * f;
     if (SIG) S.s[n] = S.s[n] * f;
   }
-  // constants: the integrals so far less the closed forms at the start
-  {
-    const T iy = 1.0 / ((st.w - b) * st.w);
-    const T r = (st.w - b) * iy;
-    const T lg = series_log(k, st.w, S.w[1], st.w * iy);
-    const T an = series_angle(k, st.c, S.c[1]);
-    const T af = k(SF_af);
-    S.t[0] = st.t + st.v * r - k(SF_kt) * lg;
-    S.f[0] = st.f - k(SF_kf) * lg - af * an;
-    if (SIG) S.s[0] = st.s + st.v * r;
-    // approaching (an < 0): a later angle > 0 is past the pass, a turn further on
-    k.set(SF_wrap, val(an) < 0.0 ? 2.0 * kPi * af : T(0.0));
-  }
   // step: |coefficient| x^n at the two last orders below the tolerances
   constexpr float lt = kSeriesTolLog2;
   const float lw = lt + series_log2(kmax(kfabs(val(S.w[0])), kfabs(val(S.w[1]))));
   float x = series_step<P - 1>(S.w[P - 1], lw);
   const float xs[7] = {series_step<P>(S.w[P], lw),
-                       series_step<P - 1>(S.c[P - 1], lt),
-                       series_step<P>(S.c[P], lt),
+                       series_step<P - 1>(S.c[P - 1], kSeriesTolPolarLog2),
+                       series_step<P>(S.c[P], kSeriesTolPolarLog2),
                        series_step<P - 1>(S.t[P - 1], lt + 6.64386f),   // 100 times
                        series_step<P>(S.t[P], lt + 6.64386f),
                        series_step<P - 1>(S.f[P - 1], lt + 3.32193f),   // 10 times
@@ -535,9 +530,9 @@ KG_INLINE float series_expand(const RayScalars<T>& g, Slots& k, const SeriesStat
 }
 
 // The state at offset x of the expansion (FULL: with v and u per unit of Mino
-// time; otherwise a sample's values).
+// time; otherwise a sample's values); an: the axis angle there.
 template <class T, int P, bool SIG, bool FULL, class Slots>
-KG_INLINE void series_at(const Slots& k, const Series<T, P, SIG>& S, const T& x, SeriesState<T>& o, T& r) {
+KG_INLINE void series_at(const Slots& k, const Series<T, P, SIG>& S, const T& x, SeriesState<T>& o, T& r, T& an) {
   T w = S.w[P], c = S.c[P], t = S.t[P], f = S.f[P], s = S.s[SIG ? P : 0];
   T v = w, u = c;
 #pragma unroll
@@ -561,7 +556,7 @@ KG_INLINE void series_at(const Slots& k, const Series<T, P, SIG>& S, const T& x,
   o.t = t - vr + k(SF_kt) * lg;
   o.f = f + k(SF_kf) * lg;
   if (SIG) o.s = s - vr;
-  const T an = series_angle(k, c, u);
+  an = series_angle(k, c, u);
   o.f = o.f + (k(SF_af) * an - (val(an) > 0.0 ? k(SF_wrap) : T(0.0)));
   o.w = w;
   o.c = c;
@@ -569,6 +564,61 @@ KG_INLINE void series_at(const Slots& k, const Series<T, P, SIG>& S, const T& x,
     o.v = v * ih;
     o.u = u * ih;
   }
+}
+
+// The integrals' constants of a new expansion: t0, f0, s0 at its left end, the
+// offset x (where the last one ended).
+template <class T, int P, bool SIG, class Slots>
+KG_INLINE void series_match(Slots& k, Series<T, P, SIG>& S, const T& x, const T& t0, const T& f0, const T& s0) {
+  S.t[0] = T(0.0);
+  S.f[0] = T(0.0);
+  S.s[0] = T(0.0);
+  k.set(SF_wrap, T(0.0));
+  SeriesState<T> o;
+  T r, an;
+  series_at<T, P, SIG, false>(k, S, x, o, r, an);
+  S.t[0] = t0 - o.t;
+  S.f[0] = f0 - o.f;
+  if (SIG) S.s[0] = s0 - o.s;
+  // approaching (an < 0): a later angle > 0 is past the pass, a turn further on
+  k.set(SF_wrap, val(an) < 0.0 ? 2.0 * kPi * k(SF_af) : T(0.0));
+}
+
+// y and dy/dx at x of the motion y'' = q1 y + q2 y^2 + q3 y^3 from y, dy at 0.
+template <class T, int P> KG_INLINE void series_motion(const T& q1, const T& q2, const T& q3, const T& x, T& y, T& dy) {
+  T a[P + 1], a2[P];
+  a[0] = y;
+  a[1] = dy;
+#pragma unroll
+  for (int n = 0; n + 2 <= P; ++n) {
+    a2[n] = series_square<T, P>(a, n);
+    a[n + 2] = (q1 * a[n] + q2 * a2[n] + q3 * series_cube<T, P>(a, a2, n)) * (1.0 / ((n + 1) * (n + 2)));
+  }
+  T p = a[P], d = a[P];
+#pragma unroll
+  for (int n = P - 1; n >= 0; --n) {
+    if (n < P - 1) d = p + x * d;
+    p = a[n] + x * p;
+  }
+  y = p;
+  dy = d;
+}
+
+// The motion x further on from the state kept in the SE slots, by its own
+// series: a third of an expansion's work, where the integrals' series is then
+// centred.
+template <class T, class Slots> KG_INLINE void series_advance(const Slots& k, const T& x, SeriesState<T>& st) {
+  constexpr int P = kSeriesOrder;
+  const T h = k(SR_h), ih = k(SR_ih);
+  const T h2 = h * h;
+  st.c = k(SE_c);
+  st.u = k(SE_u) * h;
+  series_motion<T, P>(-(h2 * k(SR_E)), T(0.0), h2 * (2.0 * k(SR_Q)), x, st.c, st.u);
+  st.u = st.u * ih;
+  st.w = k(SE_w);
+  st.v = k(SE_v) * h;
+  series_motion<T, P>(h2 * k(SR_A), h2 * (1.5 * k(SR_B)), h2 * (2.0 * k(SR_C)), x, st.w, st.v);
+  st.v = st.v * ih;
 }
 
 }  // namespace kg

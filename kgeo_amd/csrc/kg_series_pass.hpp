@@ -24,6 +24,9 @@
 // fewer expansions per lane, but more anchors, and would let near-critical
 // rays change by 1e-9 with the number of pixels.)
 //
+// An expansion covers the samples on both sides of its centre, to which the
+// motion alone is carried first (series_advance).
+//
 // The lanes of a wave take their steps together (the smallest any lane
 // needs), so a sample index is uniform across the wave and every store is
 // one contiguous row; a lane that would hold the others to steps below
@@ -40,6 +43,11 @@ namespace kg {
 constexpr int kSeriesBlocks = 2;
 constexpr int kSeriesMaxParts = 8;
 constexpr double kSeriesMinStep = 128.0;
+// An expansion holds for the same distance x on both sides of its centre, so
+// the next is centred ahead of where the last ended, by this part of its x:
+// the distance to the nearest singularity (about 10 x) shrinks by at most the
+// distance moved, so the new x is at least 1 - 1.8 / 10 of the old.
+constexpr float kSeriesAhead = 0.8f;
 
 #if defined(__HIPCC__)
 // A lane's column of its wave's LDS (LocalSlots).  fresh() keeps the loads
@@ -73,10 +81,10 @@ KG_INLINE int64_t series_part(int64_t js, int64_t je, int64_t q, int64_t parts) 
 // Parts per block for npix rays (all images') sampled together on grids of
 // ngeo samples: enough that 2^17 (ray, part) lanes fill the chip's 2048 places
 // at two waves per SIMD.  More cost their expansions again.  Measured with 1,
-// 2, 4 and 8 parts (ms): 1000 rays x 250 samples 0.477, 0.409, 0.374, 0.361;
-// 64 x 64 x 100 0.456, 0.430, 0.425, 0.420; 217 x 301 x 333 0.94, 0.81, 0.86,
-// 1.04; 512 x 512 x 500 2.28, 2.44, 2.97, 3.97; a survey of 16 images of
-// 192 x 192 rays and 128 .. 512 samples 9.7, 10.4, 10.4, 10.4.
+// 2, 4 and 8 parts (ms): 1000 rays x 250 samples 0.361, 0.303, 0.272, 0.257;
+// 64 x 64 x 100 0.316, 0.292, 0.286, 0.280; 217 x 301 x 333 0.81, 0.69, 0.72,
+// 0.85; 512 x 512 x 500 2.03, 2.19, 2.51, 3.18; a survey of 16 images (64 .. 512
+// pixels a side, 50 .. 400 samples) 7.6, 8.1, 8.1, 8.1.
 inline int64_t pick_parts(int64_t npix, int64_t ngeo) {
   int64_t want = npix > 0 ? (1LL << 17) / npix : 1;
   const int64_t most = ngeo / series_blocks(ngeo) / kFixupSpan;
@@ -360,8 +368,12 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
     }
   }
   const float floor_x = static_cast<float>(je - js) / static_cast<float>(kSeriesMinStep);
-  // the position, in samples from js (exact: steps end on multiples of 2^-10)
-  double x0 = 0.0;
+  k.set(SE_t, st.t);
+  k.set(SE_f, st.f);
+  k.set(SE_s, st.s);
+  // in samples from js, multiples of 2^-10 (exact): x0, up to where the
+  // samples are done, and the expansion's centre x0 + d
+  double x0 = 0.0, d = 0.0;
   int64_t j = js + 1;
   const double xe = static_cast<double>(je - js);
   while (j < pe) {
@@ -375,18 +387,26 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
     if (!live) x = 1.0e30f;
     x = wave_min(x);
     if (x == 1.0e30f) break;  // no lane is left
-    double x1 = x0 + static_cast<double>(x);
+    if (static_cast<double>(x) < d) {
+      // it does not reach back to x0: centre it nearer
+      d = kfloor(static_cast<double>(kSeriesAhead * x) * 1024.0) * (1.0 / 1024.0);
+      series_advance<T>(k, T(d), st);
+      continue;
+    }
+    series_match<T, P, SIG>(k, S, T(-d), k(SE_t), k(SE_f), k(SE_s));
+    const double xc = x0 + d;
+    double x1 = xc + static_cast<double>(x);
     if (x1 > xe) x1 = xe;
     x1 = kfloor(x1 * 1024.0) * (1.0 / 1024.0);
     const int64_t jn = js + static_cast<int64_t>(kfloor(x1)) + 1;  // the first sample after the step
     const int64_t jm = jn < pe ? jn : pe;
     if (j < ps) j = ps < jm ? ps : jm;
-    double xj = static_cast<double>(j - js) - x0;
+    double xj = static_cast<double>(j - js) - xc;
     for (; j < jm; ++j) {
       SeriesState<T> s;
-      T r;
+      T r, an;
       k.fresh();
-      series_at<T, P, SIG, false>(k, S, T(xj), s, r);
+      series_at<T, P, SIG, false>(k, S, T(xj), s, r, an);
       xj += 1.0;
       const T th = acos_fast(s.c);
       if (live) {
@@ -401,11 +421,23 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
       }
     }
     if (j >= pe) break;
-    SeriesState<T> e;
-    T r;
-    series_at<T, P, SIG, true>(k, S, T(x1 - x0), e, r);
-    st = e;
+    {
+      SeriesState<T> e;
+      T r, an;
+      series_at<T, P, SIG, true>(k, S, T(x1 - xc), e, r, an);
+      k.set(SE_w, e.w);
+      k.set(SE_v, e.v);
+      k.set(SE_c, e.c);
+      k.set(SE_u, e.u);
+      k.set(SE_t, e.t);
+      k.set(SE_f, e.f);
+      if (SIG) k.set(SE_s, e.s);
+    }
     x0 = x1;
+    d = static_cast<double>(kSeriesAhead * x);
+    if (d > 0.5 * (xe - x0)) d = 0.5 * (xe - x0);
+    d = kfloor(d * 1024.0) * (1.0 / 1024.0);
+    series_advance<T>(k, T(d), st);
   }
   return bad ? ST_NONFINITE : 0u;
 }

@@ -71,7 +71,7 @@ constexpr size_t kFlagBytes = 256;
 // waves are to start first.  Workgroups go to the chip's 8 XCDs in turn and
 // an image is often a multiple of 8 tiles wide, so each group of 8 is turned
 // by one more place, lest an XCD hold the same columns of every row.  (512 x 512 x 500 samples:
-// 2.28 ms, 2.35 in the order of the pixels.)
+// 3 % less time than in the order of the pixels.)
 __device__ inline int64_t tile_of(unsigned b, unsigned n) {
   const unsigned g = b >> 3;
   const unsigned k = (g << 3) + 8 <= n ? (g << 3) + ((b + g) & 7u) : b;
@@ -231,15 +231,16 @@ __global__ __launch_bounds__(kPassBlock) void kg_radial_heads(DevParams p, Sampl
 
 // grid (pixel blocks, parts): one wave per workgroup, 64 neighbouring pixels
 // at one part of block b of their grids (the last part, the longest, first).
-// Bound by FP64 issue: a sample takes 235 vector instructions (84
+// Bound by FP64 issue: a sample takes about 200 vector instructions (84
 // multiply-adds of six polynomials, a logarithm, an arctangent, an arccosine,
-// a reciprocal), an expansion about 2300, and a ray about 12 of them.  At 512 x
-// 512 x 500 samples (t, r, theta, phi written) one block of all rays takes
-// 1.14 ms at 65 % VALU busy; the whole call 2.28 ms, where the walk by
-// addition theorems (up to three Carlson R_J per sample) took 4.95; 217 x 301 x
-// 333 0.82 for 1.29, 64 x 64 x 100 0.42 for 0.54, 1000 x 250 0.36 for 0.55.
-// Two waves per SIMD: one alone (512 registers) is slower from 217 x 301 on
-// (0.98 and 3.0 ms).
+// a reciprocal), an expansion with its share of the motion ahead about 2600,
+// and a ray about 15 of them (a wave's rays take the smallest of their
+// steps).  At 512 x 512 x 500 samples (t, r, theta, phi written) one block of
+// all rays takes 1.02 ms; the whole call 2.03 ms, where the walk by addition
+// theorems (up to three Carlson R_J per sample) took 4.95; 217 x 301 x 333
+// 0.69 for 1.29, 64 x 64 x 100 0.28 for 0.55, 1000 x 250 0.26 for 0.55.
+// (Expansions about the left end of their samples: 2.23, 0.77, 0.345 and 0.316.)
+// Two waves per SIMD: one alone (512 registers) was slower from 217 x 301 on.
 template <bool SIG, bool EARLY>
 __global__ __launch_bounds__(kPassBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_series(
     DevParams p, SampleArgs a, Records rth, Records rr, int64_t b, int64_t nb, FixupQueue q) {
