@@ -11,8 +11,8 @@
 // Cauchy products w^2, w^3, c^2, c^3.  The integrands of t, phi and sigma
 // are rational in w and c; their series are the products' quotients,
 // integrated term by term.  One expansion (about 5 P^2 multiply-adds for
-// order P, on both sides of its centre) replaces the elliptic functions and integrals of every sample in
-// its step, and a sample costs one polynomial per coordinate: the
+// order P) replaces the elliptic functions and integrals of every sample on
+// both sides of it, and a sample costs one polynomial per coordinate: the
 // Gralla-Lupsasca formulas (kerr_raytracing_ana.py:126-683) are evaluated
 // only at the rays' anchors (kg_sample.hpp).  w is regular at infinity,
 // where r is not, and the poles of the integrands that the ray reaches or
@@ -275,7 +275,7 @@ template <class T> struct SeriesState {
   T t, f, s;
 };
 
-// One expansion: polynomials in the grid index about its start.
+// One expansion: polynomials in the grid index about its centre.
 template <class T, int P, bool SIG> struct Series {
   T w[P + 1], c[P + 1], t[P + 1], f[P + 1], s[SIG ? P + 1 : 1];
 };
