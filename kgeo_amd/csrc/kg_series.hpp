@@ -131,8 +131,9 @@ KG_INLINE double sqrt_fast(double x) {
 KG_INLINE double acos_fast(double x) {
   const double ax = kfabs(x);
   const bool small = ax < 0.5;  // false for NaN
-  const double z = small ? x * x : 0.5 - 0.5 * ax;
-  const double s = small ? ax : sqrt_fast(z);  // NaN for |x| > 1
+  // |x| an ulp above 1 (a sample on the axis) counts as 1
+  const double z = small ? x * x : __builtin_fmax(0.5 - 0.5 * ax, 0.0);
+  const double s = small ? ax : sqrt_fast(z);
   const double r = s + s * (z * horner<kAcosTerms>(fits() + kAcosFit, z));  // asin s
   // acos |x|: pi/2 - r, or 2 r; of x < 0: pi less that
   const double q = small ? kHalfPi - (r - 6.123233995736766e-17) : r + r;

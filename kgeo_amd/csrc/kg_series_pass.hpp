@@ -384,7 +384,7 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
       if (live) push_range(push, i, j < ps ? ps : j, pe, last);
       live = false;
     }
-    if (!live) x = 1.0e30f;
+    x = live ? (x < 1.0e29f ? x : 1.0e29f) : 1.0e30f;  // all coefficients 0: no bound
     x = wave_min(x);
     if (x == 1.0e30f) break;  // no lane is left
     if (static_cast<double>(x) < d) {
