@@ -8,7 +8,7 @@ plus all 131,072,000 samples with r, theta, phi, t written to HBM
 (kgeo_sample).  Inputs are resident in HBM before the timed region.
 
 Prints ONE JSON line with the metric, the roofline of the sample passes
-(the heads, far, walk and fixup kernels of theta and r, FP64 vector ALU;
+(the heads, series and fixup kernels, FP64 vector ALU;
 timed with HIP events on the launch stream; algorithmic FLOPs op-counted on
 the kernels' own code) and the CPU
 baseline (the oracle, i.e. the reference algorithm in NumPy/SciPy, on a

@@ -409,7 +409,7 @@ int kgeo_equatorial_image_vjp_noalloc(const kgeo_ray_params* p, const double* al
  * from unfinished ones.
  */
 typedef struct kgeo_batch_tuning {
-  int32_t samples_per_item; /* Mino-time samples per work item (rounded up to a multiple of 16); an item is 64 pixels x this */
+  int32_t samples_per_item; /* Mino-time samples per work item asked for (rounded up to whole segments); an item is 64 pixels x a part of a block */
   int32_t waves_per_cu;     /* persistent grid: CUs x this waves (1..64) */
   int32_t reserved[2];
 } kgeo_batch_tuning;

@@ -4,9 +4,9 @@ The reference traces one image per ``raytrace_ana`` call
 (kerr_raytracing_ana.py:46-122); a survey over spins, inclinations,
 resolutions and ngeo is a Python loop of such calls.  ``BatchSurvey`` runs
 the whole survey as one HIP graph: a setup kernel over every pixel of every
-image, then for theta and r the plain path's passes (direct heads, long
-steps, walk, fixups) as persistent kernels whose waves pull (image, 64-pixel
-tile, unit) work items from one atomic queue per pass (kgeo_batch.hip).
+image, then the plain path's passes (direct heads of theta and r, Taylor
+series, fixups) as persistent kernels whose waves share out (image, 64-pixel
+tile, unit) work items (kgeo_batch.hip).
 Each image's results equal a plain ``raytrace_ana_device`` call on that
 image to the last bits.
 

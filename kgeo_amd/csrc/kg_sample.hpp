@@ -7,17 +7,18 @@
 // radial_pixel: loads the radial slots, builds the radial ladder, writes r and
 //   combines phi = I_phi + lambda G_phi, t = I_t + a^2 G_t,
 //   sigma = I_sigma + a^2 G_t (kerr_raytracing_ana.py:186-188).
-// Each runs one loop specialised at compile time for the pixel's motion class
-// or radial case, so a wave only keeps its own case's constants live.  The
-// plan is slot-major: slot s of pixel p is plan[s * stride + p].
+// The plan is slot-major: slot s of pixel p is plan[s * stride + p].
 //
-// On the linspace grid the loops walk: each sample's state follows from the
-// previous one by the addition theorems (kg_step.hpp), with a direct
-// evaluation at the chunk's first sample, at every multiple of the anchor
-// interval (kg_step.hpp),
-// at the last grid sample (tau = stop exactly) and wherever a step is not
-// well conditioned.  With caller-given Mino times (tau_in) every sample is direct.
-// Host-compilable (KG_INLINE), so the CPU test build runs the same loops.
+// The kernels run these loops with every sample evaluated directly (WALK =
+// false: caller-given Mino times, short grids and the fixup pass; one body for
+// all motions and cases).  The linspace grid goes by Taylor series
+// (kg_series_pass.hpp).
+//
+// The walk of the linspace grid by the addition theorems (kg_step.hpp: the
+// loops with WALK = true, and the passes below) is run by the CPU build only:
+// a second, independent way from the same plan to the same samples, which the
+// tests hold against the series and the direct evaluation.
+// Host-compilable (KG_INLINE), so the CPU test build runs the same code.
 
 #pragma once
 
@@ -397,10 +398,7 @@ KG_INLINE uint32_t radial_pixel(const RayScalars<T>& c, const double* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// The walk in passes, each its own kernel, so the walking loop is not held
-// to the register budget of the direct evaluation (Landen ladder, Carlson
-// duplication for three characteristics), which it needs only where it
-// restarts:
+// The walk in passes (CPU build):
 //   heads   one lane per (pixel, head): the direct evaluation at the grid
 //           step h and at the segment length L h (records 0 and 1), at the
 //           last grid sample and at the first sample of each block of
