@@ -900,7 +900,7 @@ KG_INLINE void stokes_pixel(const RayScalars<double>& c, bool north, const kgeo_
     double Ir = -1.0, rs = -1.0;
     bool zero = true;
     if (!e.vort) {
-      eq_subring(c, beta, e, lad, m, Ir, rs);
+      eq_subring<true>(c, beta, e, lad, m, Ir, rs);
       zero = (e.N < m) || (e.N == -1.0) || (rs <= rh) || (em.emiscut_in > 0.0 && rs < em.emiscut_in) ||
              (em.emiscut_out > 0.0 && rs > em.emiscut_out);
     }

@@ -157,8 +157,8 @@ KG_INLINE void eq_ray(const RayScalars<T>& c, const T& alpha, const T& beta, EqR
 }
 
 // I_r and r_s of subring m (equatorial_lensing.py:158-188): r_s = 0 where
-// N_max < m.  Needs a non-vortical ray.
-template <class T>
+// N_max < m.  Needs a non-vortical ray.  PIN: case3_numerator's.
+template <bool PIN = false, class T>
 KG_INLINE void eq_subring(const RayScalars<T>& c, const T& beta, const EqRay<T>& e, const JacobiLadder<T>& lad, int m, T& Ir,
                           T& rs) {
   {
@@ -174,7 +174,7 @@ KG_INLINE void eq_subring(const RayScalars<T>& c, const T& beta, const EqRay<T>&
       Ir = (val(beta) >= 0.0) ? (2.0 * msub * e.K - e.Fo) / e.w : (2.0 * msub * e.K + e.Fo) / e.w;
     }
   }
-  rs = radial_eval(e.rc, lad, Ir, false).r;
+  rs = radial_eval<T, -1, PIN>(e.rc, lad, Ir, false).r;
   if (e.N < m) rs = T(0.0);
 }
 

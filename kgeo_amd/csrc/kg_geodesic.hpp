@@ -1016,9 +1016,29 @@ KG_INLINE void radial_state(const RadialConsts<T>& rc, const JacobiLadder<T>& la
   }
 }
 
+// The numerator (BB r2 - AA r1) + (BB r2 + AA r1) cn of case 3's r.  Which of
+// the products are fused is the compiler's choice, and differs between the
+// kernels that inline it by up to a few ulp of r.  PIN fixes it, for the polarized image:
+// its models (the four-velocity and the metric's Delta, whose terms cancel at
+// the horizon) magnify an ulp of r by about 1/(r - r_+)^2, up to 2e-5 of
+// sin(theta_B) at a pixel next to it, so its r must not follow the code around it.
+template <bool PIN, class T>
+KG_INLINE T case3_numerator(const T& AA, const T& BB, const T& rr1, const T& rr2, const T& cn) {
+  if constexpr (PIN) {
+#if defined(__clang__)
+#pragma clang fp contract(off)
+#endif
+    const T q = AA * rr1;
+    const T n0 = __builtin_fma(BB, rr2, -q), n1 = __builtin_fma(BB, rr2, q);
+    return __builtin_fma(n1, cn, n0);
+  } else {
+    return (BB * rr2 - AA * rr1) + (BB * rr2 + AA * rr1) * cn;
+  }
+}
+
 // r(tau) and, with do_phi_t, the building blocks I_+, I_-, I_1, I_2
 // CASE = 2, 3, 4 fixes the radial case at compile time; CASE = -1 reads rc.rcase.
-template <class T, int CASE = -1>
+template <class T, int CASE = -1, bool PIN = false>
 KG_INLINE RadialOut<T> radial_out(const RadialConsts<T>& rc, const T& tau, const RState<T>& st, bool do_phi_t) {
   RadialOut<T> o;
   const T* v = rc.v;
@@ -1054,7 +1074,7 @@ KG_INLINE RadialOut<T> radial_out(const RadialConsts<T>& rc, const T& tau, const
     const T& BB = v[C3_BB];
     const T& rr1 = v[C3_rr1];
     const T& rr2 = v[C3_rr2];
-    T num = (BB * rr2 - AA * rr1) + (BB * rr2 + AA * rr1) * cn;
+    T num = case3_numerator<PIN>(AA, BB, rr1, rr2, cn);
     T den = (BB - AA) + (BB + AA) * cn;
     o.r = num / den;
     if (!do_phi_t) return o;
@@ -1103,14 +1123,14 @@ KG_INLINE RadialOut<T> radial_out(const RadialConsts<T>& rc, const T& tau, const
   return o;
 }
 
-template <class T, int CASE = -1>
+template <class T, int CASE = -1, bool PIN = false>
 KG_INLINE RadialOut<T> radial_eval(const RadialConsts<T>& rc, const JacobiLadder<T>& lad, const T& tau,
                                    bool do_phi_t) {
   const T dv = rc.v[R_Xs] * tau;
   const T X = rc.v[R_U0] - dv;
   RState<T> st;
   radial_state<T, CASE>(rc, lad, X, dv, do_phi_t, st);
-  return radial_out<T, CASE>(rc, tau, st, do_phi_t);
+  return radial_out<T, CASE, PIN>(rc, tau, st, do_phi_t);
 }
 
 // ---------------------------------------------------------------------------
