@@ -66,7 +66,7 @@ void three_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, c
     bool w;
     unpack_host_item(e, i, j, w);
     for (int64_t sg = 0; sg < kFixupSpan; ++sg)
-      st[i] |= theta_fixup_sample<DO_PHI_T, T>(plan, npix, i, gflags, o, i, j, w, sg);
+      st[i] |= theta_fixup_sample<DO_PHI_T, T>(plan, npix, i, gflags, o, i, j, fixup_end(j, G, w), sg);
   }
   items.clear();
   for (int64_t i = 0; i < npix; ++i)
@@ -95,7 +95,7 @@ void three_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, c
     bool w;
     unpack_host_item(e, i, j, w);
     for (int64_t sg = 0; sg < kFixupSpan; ++sg)
-      st[i] |= radial_fixup_sample<DO_PHI_T, T>(c, plan, npix, i, gflags, o, i, j, w, sg);
+      st[i] |= radial_fixup_sample<DO_PHI_T, T>(c, plan, npix, i, gflags, o, i, j, fixup_end(j, G, w), sg);
   }
 }
 
@@ -122,7 +122,7 @@ void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, 
       st[i] |= o.sig ? series_block_pixel<true, false, LocalSlots<T>, HostPush, T>(c, plan, npix, i, gflags, o, i, true, b, nb, q, parts, rth, rr, slots, push)
                      : series_block_pixel<false, false, LocalSlots<T>, HostPush, T>(c, plan, npix, i, gflags, o, i, true, b, nb, q, parts, rth, rr, slots, push);
     }
-  const size_t cap = static_cast<size_t>(npix) * static_cast<size_t>(fixup_items(G));
+  const size_t cap = static_cast<size_t>(npix) * static_cast<size_t>(series_items(G));
   nfix[0] = items.size() <= cap ? static_cast<int64_t>(items.size()) : -1;
   nfix[1] = nfix[0];
   nfix[2] = 0;
@@ -131,9 +131,10 @@ void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, 
       int64_t i, j;
       bool w;
       unpack_host_item(e, i, j, w);
+      const int64_t end = series_fixup_end(j, G, w);
       for (int64_t sg = 0; sg < kFixupSpan; ++sg)
-        st[i] |= part == 0 ? theta_fixup_sample<true, T>(plan, npix, i, gflags, o, i, j, w, sg)
-                           : radial_fixup_sample<true, T>(c, plan, npix, i, gflags, o, i, j, w, sg);
+        st[i] |= part == 0 ? theta_fixup_sample<true, T>(plan, npix, i, gflags, o, i, j, end, sg)
+                           : radial_fixup_sample<true, T>(c, plan, npix, i, gflags, o, i, j, end, sg);
     }
 }
 

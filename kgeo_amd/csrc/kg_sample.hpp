@@ -1000,15 +1000,15 @@ KG_INLINE int64_t fixup_end(int64_t j, int64_t ngeo, bool walked) {
   return je < lim ? je : lim;
 }
 
-// Queued theta sample j + s (0 <= s < kFixupSpan) of the range j .. fixup_end,
+// Queued theta sample j + s (0 <= s < kFixupSpan) of the range j .. end - 1,
 // by direct evaluation, if it lies in the range: the fixup pass with one
 // sample per lane, whose lanes are independent (the pass is latency-bound:
 // few items, each a chain of dependent evaluations when walked).
 template <bool DO_PHI_T, class T = double>
 KG_INLINE uint32_t theta_fixup_sample(const double* __restrict__ plan, int64_t stride, int64_t p, uint32_t gflags,
-                                      const SampleOut& o, int64_t i, int64_t j, bool walked, int64_t s) {
+                                      const SampleOut& o, int64_t i, int64_t j, int64_t end, int64_t s) {
   const int64_t js = j + s;
-  if (js >= fixup_end(j, o.ngeo, walked)) return 0u;
+  if (js >= end) return 0u;
   return theta_pixel<DO_PHI_T, T, false>(plan, stride, p, gflags, o, i, js, js + 1);
 }
 
@@ -1129,13 +1129,13 @@ KG_INLINE uint32_t radial_walk_pixel(const RayScalars<T>& c, const double* __res
   return bad ? ST_NONFINITE : 0u;
 }
 
-// Queued radial sample j + s of the range j .. fixup_end (as theta_fixup_sample).
+// Queued radial sample j + s of the range j .. end - 1 (as theta_fixup_sample).
 template <bool DO_PHI_T, class T = double>
 KG_INLINE uint32_t radial_fixup_sample(const RayScalars<T>& c, const double* __restrict__ plan, int64_t stride,
                                        int64_t p, uint32_t gflags, const SampleOut& o, int64_t i, int64_t j,
-                                       bool walked, int64_t s) {
+                                       int64_t end, int64_t s) {
   const int64_t js = j + s;
-  if (js >= fixup_end(j, o.ngeo, walked)) return 0u;
+  if (js >= end) return 0u;
   return radial_pixel<DO_PHI_T, T, false>(c, plan, stride, p, gflags, o, i, js, js + 1);
 }
 

@@ -31,7 +31,7 @@
 // needs), so a sample index is uniform across the wave and every store is
 // one contiguous row; a lane that would hold the others to steps below
 // 1/kSeriesMinStep of its block leaves the rest of it to the fixup pass.
-// Blocks start at multiples of kFixupSpan, so a queued range lies in one.
+// A queued range ends with its block (series_fixup_end).
 
 #pragma once
 
@@ -65,17 +65,42 @@ struct LdsSlots {
 // First sample of block b of nb (nb: the end, the last grid sample).
 KG_INLINE int64_t series_start(int64_t ngeo, int64_t b, int64_t nb) {
   const int64_t last = ngeo - 1;
-  return b >= nb ? last : last * b / nb / kFixupSpan * kFixupSpan;
+  return b >= nb ? last : (last * b + nb - 1) / nb;
 }
 
-// Blocks per ray: two, as long as each holds kFixupSpan samples.  (One block
-// over a whole ray near the critical curve: 1.2e-10 of r at 0.94, 17 deg, 500
-// samples, against 6e-12 in two.)
-KG_INLINE int64_t series_blocks(int64_t ngeo) { return ngeo - 1 >= kSeriesBlocks * kFixupSpan ? kSeriesBlocks : 1; }
+// Blocks per ray: two, so that no sample is more than half a ray from its
+// block's start (of 3 samples the middle one is not in any case).  Against direct
+// evaluation, rays near the critical curve (four observers, 240 x 240 pixels,
+// grids of 4 .. 16 samples) are off by up to 4e-9 of r in one block over the
+// whole ray; in two of which the second started at a multiple of 8 samples
+// (0.7 of the ray for grids of 32) by 2.5e-11; in two halves by 5e-12.
+KG_INLINE int64_t series_blocks(int64_t ngeo) { return ngeo - 1 > kSeriesBlocks ? kSeriesBlocks : 1; }
 
-// First sample of part q of `parts` of a block's samples js .. je - 1.
+// First sample of part q of `parts` of a block's samples js .. je - 1: inside
+// the block a multiple of kFixupSpan, so that a queued range lies in one part.
 KG_INLINE int64_t series_part(int64_t js, int64_t je, int64_t q, int64_t parts) {
-  return q <= 0 ? js : (q >= parts ? je : (js + (je - js) * q / parts) / kFixupSpan * kFixupSpan);
+  if (q <= 0) return js;
+  if (q >= parts) return je;
+  const int64_t s = (js + (je - js) * q / parts) / kFixupSpan * kFixupSpan;
+  return s > js ? s : js;
+}
+
+// End of the queued range that starts at sample j: fixup_end, or the end of
+// j's block before it.
+KG_INLINE int64_t series_fixup_end(int64_t j, int64_t ngeo, bool walked) {
+  const int64_t e = fixup_end(j, ngeo, walked), nb = series_blocks(ngeo);
+  const int64_t s = nb > 1 ? series_start(ngeo, 1, nb) : 0;
+  return (j < s && s < e) ? s : e;
+}
+
+// Queued ranges per pixel at most: one per window of kFixupSpan samples, and
+// one more for the window that the second block starts in.
+KG_INLINE int64_t series_items(int64_t ngeo) { return fixup_items(ngeo) + (series_blocks(ngeo) - 1); }
+
+// Queue samples j .. e - 1 of a block: from j to the next window, then one
+// item per window.  walked: the last grid sample is a head's.
+template <class Push> KG_INLINE void push_windows(Push& push, int64_t i, int64_t j, int64_t e, bool walked) {
+  for (; j < e; j = (j / kFixupSpan + 1) * kFixupSpan) push(i, j, walked);
 }
 
 // Parts per block for npix rays (all images') sampled together on grids of
@@ -270,7 +295,7 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
   constexpr int P = kSeriesOrder;
   const int64_t last = o.ngeo - 1;
   const int64_t js = series_start(o.ngeo, b, nb), je = series_start(o.ngeo, b + 1, nb);
-  if (js >= je) {  // a grid of one sample; series_blocks gives blocks of others kFixupSpan samples
+  if (js >= je) {  // a grid of one sample
     if (in && q + 1 == parts) push(i, js, false);
     return 0u;
   }
@@ -291,7 +316,7 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
         tp.walk && (EARLY || radial_walks(o, gflags, plan[static_cast<int64_t>(PL_R + R_k) * stride + p]));
     if (live && !walks) {
       // no heads for this pixel either: every sample, the last included
-      for (int64_t j = ps; j < (ends ? o.ngeo : pe); j += kFixupSpan) push(i, j, false);
+      push_windows(push, i, ps, ends ? o.ngeo : pe, false);
       live = false;
     }
     const T h = T(stop / static_cast<double>(o.ngeo - 1));
@@ -345,7 +370,7 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
                     kfinite(val(st.t)) & kfinite(val(st.f)) & (val(k(SR_l2)) > 0.0) & (val(lam) != 0.0) &
                     (val(st.w) > 0.0) & kfinite(val(k(SR_E))) & kfinite(val(h));
     if (live && !ok) {
-      push_range(push, i, ps, pe, last);
+      push_windows(push, i, ps, pe, true);
       live = false;
     }
     if (live && ps == js) {
@@ -381,7 +406,7 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
     k.fresh();
     float x = series_expand<T, P, SIG>(c, k, st, S);
     if (!(x >= floor_x)) {  // also NaN
-      if (live) push_range(push, i, j < ps ? ps : j, pe, last);
+      if (live) push_windows(push, i, j < ps ? ps : j, pe, true);
       live = false;
     }
     x = live ? (x < 1.0e29f ? x : 1.0e29f) : 1.0e30f;  // all coefficients 0: no bound

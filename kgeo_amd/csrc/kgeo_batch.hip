@@ -269,8 +269,9 @@ __global__ __launch_bounds__(kBlock) void kg_batch_fixup(BatchDev d) {
     const int64_t s = B.slot_off + i;
     const uint32_t fl = d.flags[im];
     const SampleOut o = image_out(d, B);
-    uint32_t st = theta_fixup_sample<true>(d.plan, d.total_slots, s, fl, o, i, j, walked, sg);
-    st |= radial_fixup_sample<true>(B.c, d.plan, d.total_slots, s, fl, o, i, j, walked, sg);
+    const int64_t end = series_fixup_end(j, B.ngeo, walked);
+    uint32_t st = theta_fixup_sample<true>(d.plan, d.total_slots, s, fl, o, i, j, end, sg);
+    st |= radial_fixup_sample<true>(B.c, d.plan, d.total_slots, s, fl, o, i, j, end, sg);
     if (d.status && st) atomicOr(&d.status[B.pix_off + i], st);
   }
 }
@@ -308,19 +309,14 @@ int64_t total_slots_of(const kgeo_ray_params* imgs, int32_t nimg) {
   return s;
 }
 
-// Elements of image k's theta and radial record tables (a walked grid needs
-// ngeo > 2; smaller images keep none) and its fixup-queue share.  The sizes
-// are the interface's; the anchor records take a part of each table.
-int64_t theta_rec_elems(const kgeo_ray_params& p) {
-  return p.ngeo > 2 ? theta_records(p.ngeo) * kThFields * slots_of(p) : 0;
-}
-int64_t radial_rec_elems(const kgeo_ray_params& p) {
-  return p.ngeo > 2 ? radial_records(p.ngeo) * kRFields * slots_of(p) : 0;
-}
-static_assert(kSeriesBlocks * kThSFields <= 4 * kThFields && kSeriesBlocks * kRSFields <= 4 * kRFields,
-              "the records fit the smallest tables");
-int64_t queue_elems(const kgeo_ray_params& p) { return fixup_items(p.ngeo) * slots_of(p); }
+// Elements of image k's theta and radial anchor records (a grid of the series
+// has ngeo > 2; smaller images keep none) and of its fixup-queue share.
+int64_t theta_rec_elems(const kgeo_ray_params& p) { return p.ngeo > 2 ? kSeriesBlocks * kThSFields * slots_of(p) : 0; }
+int64_t radial_rec_elems(const kgeo_ray_params& p) { return p.ngeo > 2 ? kSeriesBlocks * kRSFields * slots_of(p) : 0; }
+int64_t queue_elems(const kgeo_ray_params& p) { return series_items(p.ngeo) * slots_of(p); }
 
+// Elements of the plan, and of the interface's record tables and queue (the
+// workspace's size): the records and the queue above take a part of them.
 struct BatchSizes {
   int64_t slots, rec, queue;
 };
@@ -328,12 +324,17 @@ struct BatchSizes {
 BatchSizes sizes_of(const kgeo_ray_params* imgs, int32_t nimg) {
   BatchSizes z{0, 0, 0};
   for (int32_t k = 0; k < nimg; ++k) {
-    z.slots += slots_of(imgs[k]);
-    z.rec += theta_rec_elems(imgs[k]) + radial_rec_elems(imgs[k]);
-    z.queue += queue_elems(imgs[k]);
+    const kgeo_ray_params& p = imgs[k];
+    z.slots += slots_of(p);
+    if (p.ngeo > 2)
+      z.rec += (theta_records(p.ngeo) * kThFields + radial_records(p.ngeo) * kRFields) * slots_of(p);
+    z.queue += fixup_items(p.ngeo) * slots_of(p);
   }
   return z;
 }
+// per slot; a whole wave's slots cover the records' alignment too
+static_assert(1 + kSeriesBlocks * (kThSFields + kRSFields) + 1 <= 4 * kThFields + 4 * kRFields,
+              "the records and the queue's extra item fit the smallest tables");
 
 }  // namespace
 
@@ -395,7 +396,7 @@ int kgeo_batch_plan(const kgeo_ray_params* imgs, int32_t nimg, const kgeo_batch_
 
   std::vector<BatchImage> host(nimg);
   std::vector<uint32_t> per(nimg);
-  int64_t pix = 0, slots = 0, outo = 0, rec = 0;
+  int64_t pix = 0, slots = 0, outo = 0, rec = 0, queue = 0;
   int64_t items[K_N] = {0, 0};
   // the survey's size as its caller cut it: an item holds samples_per_item
   // samples, rounded up to whole segments
@@ -424,6 +425,7 @@ int kgeo_batch_plan(const kgeo_ray_params* imgs, int32_t nimg, const kgeo_batch_
     rec += theta_rec_elems(p);
     B.r_rec = rec;
     rec += radial_rec_elems(p);
+    queue += queue_elems(p);
     B.do_phi_t = 1;  // required by check_images
     const int64_t tiles = B.slots / kWave;
     int64_t mine = 0;
@@ -457,7 +459,7 @@ int kgeo_batch_plan(const kgeo_ray_params* imgs, int32_t nimg, const kgeo_batch_
   d.rec = reinterpret_cast<double*>(w);
   w += align256(static_cast<size_t>(rec) * sizeof(double));
   d.queue = reinterpret_cast<unsigned long long*>(w);
-  d.qcap = static_cast<unsigned long long>(sizes_of(imgs, nimg).queue);
+  d.qcap = static_cast<unsigned long long>(queue);
   d.nimg = nimg;
   d.total_slots = slots;
   for (int q = 0; q < K_N; ++q) d.total_items[q] = static_cast<uint32_t>(items[q]);

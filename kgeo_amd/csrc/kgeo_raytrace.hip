@@ -266,8 +266,9 @@ __global__ __launch_bounds__(kPassBlock) void kg_fixup(DevParams p, SampleArgs a
     bool walked;
     unpack_item(q.items[e / kFixupSpan], i, j, walked);
     const int64_t sg = static_cast<int64_t>(e % kFixupSpan);
-    uint32_t st = theta_fixup_sample<true>(a.plan, p.npix, i, a.gflags[0], a.out, i, j, walked, sg);
-    st |= radial_fixup_sample<true>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, j, walked, sg);
+    const int64_t end = series_fixup_end(j, p.ngeo, walked);
+    uint32_t st = theta_fixup_sample<true>(a.plan, p.npix, i, a.gflags[0], a.out, i, j, end, sg);
+    st |= radial_fixup_sample<true>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, j, end, sg);
     if (a.status && st) atomicOr(&a.status[i], st);
   }
 }
@@ -380,10 +381,9 @@ int env_chunks() {
 }
 
 // Workspace: the flag page, the plan [PL_N][npix] and, for a grid of more
-// than two samples, the theta and radial anchor records and the fixup queue
-// (one item per kFixupSpan samples and pixel bounds the series' pushes).  The
-// size is the interface's (kgeo.h), of which the records take a part: per
-// pixel at least 76 doubles, of which they take 2 (kThSFields + kRSFields).
+// than two samples, the fixup queue (series_items per pixel bounds the series'
+// pushes) and the theta and radial anchor records.  The size is the
+// interface's (kgeo.h), of which queue and records take a part.
 struct WsLayout {
   size_t plan, threc, rrec, queue, total;
   unsigned long long qcap;
@@ -397,7 +397,7 @@ WsLayout ws_layout(int64_t npix, int64_t ngeo) {
   if (ngeo > 2) {
     const size_t tables = static_cast<size_t>(theta_records(ngeo)) * kThFields +
                           static_cast<size_t>(radial_records(ngeo)) * kRFields;
-    L.qcap = static_cast<unsigned long long>(np) * static_cast<unsigned long long>(fixup_items(ngeo));
+    L.qcap = static_cast<unsigned long long>(np) * static_cast<unsigned long long>(series_items(ngeo));
     L.queue = off;
     L.threc = off + static_cast<size_t>(L.qcap) * sizeof(unsigned long long);
     L.rrec = L.threc + static_cast<size_t>(kSeriesBlocks) * kThSFields * np * sizeof(double);
@@ -406,8 +406,8 @@ WsLayout ws_layout(int64_t npix, int64_t ngeo) {
   L.total = off;
   return L;
 }
-static_assert(kSeriesBlocks * (kThSFields + kRSFields) <= 4 * kThFields + 4 * kRFields,
-              "the records fit the tables' part of the workspace");
+static_assert(1 + kSeriesBlocks * (kThSFields + kRSFields) <= 4 * kThFields + 4 * kRFields,
+              "the records and the queue's extra item fit the tables' part of the workspace");
 
 // The kernels always sample t, phi and sigma (as the reference's
 // raytrace_ana does, kerr_raytracing_ana.py:97): the theta pass parks G_phi,
@@ -421,8 +421,9 @@ int require_phi_t(const kgeo_ray_params* p) {
 }
 
 // Sizes one call handles: a fixup item packs the pixel in 32 bits and the
-// sample in 31, and the queue counters are 32-bit (a pass queues at most
-// npix * ceil(ngeo / 8) items).  Larger jobs are split over pixels.
+// sample in 31, and the queue counter is 32-bit (a call queues at most
+// npix * series_items(ngeo) items; the bound leaves out the one item more, whose
+// t and phi alone would take 512 GiB at it).  Larger jobs are split over pixels.
 int size_limit(int64_t npix, int64_t ngeo) {
   if (npix > 0x7fffffffLL) return fail(KGEO_E_ARG, "npix above 2^31 - 1%s (%lld): split the pixels", "", npix);
   if (ngeo > 0x7fffffffLL) return fail(KGEO_E_ARG, "ngeo above 2^31 - 1%s (%lld)", "", ngeo);
