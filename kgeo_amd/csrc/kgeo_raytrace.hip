@@ -493,6 +493,19 @@ SideStream* side_stream(hipStream_t st) {
   return s.side ? &s : nullptr;
 }
 
+// The caller's stream waits for the radial plan constants (run_plan).
+int wait_planned(hipStream_t st) {
+  std::lock_guard<std::mutex> lock(g_side_mu);
+  SideStream* ss = side_stream(st);
+  if (ss && hipStreamWaitEvent(st, ss->planned, 0) != hipSuccess)
+    return fail_msg(KGEO_E_HIP, "wait for the plan failed");
+  return KGEO_OK;
+}
+
+// The plan.  Its radial constants are left to the side stream: what follows on
+// the caller's must wait for them (wait_planned) or for a pass that follows
+// them there (run_series' join) before the call returns, whatever becomes of
+// it, since the kernel reads alpha and beta and writes the workspace.
 int run_plan(const kgeo_ray_params* p, const double* alpha, const double* beta, int8_t* rclass, int8_t* thclass,
              int32_t* nmax_eq, double* tau_tot, uint32_t* status, void* ws, hipStream_t st) {
   DevParams d = make_dev(p, p->ngeo);
@@ -511,18 +524,16 @@ int run_plan(const kgeo_ray_params* p, const double* alpha, const double* beta, 
     return check_launch("kg_setup");
   }
   // the radial constants on the side stream, after everything enqueued so
-  // far on the caller's (an earlier sample pass may still read the plan);
-  // kgeo_sample's radial passes follow them there, and its direct path
-  // waits for `planned`
+  // far on the caller's (an earlier sample pass may still read the plan)
   if (hipEventRecord(ss->fork, st) != hipSuccess || hipStreamWaitEvent(ss->side, ss->fork, 0) != hipSuccess)
     return fail_msg(KGEO_E_HIP, "fork to the side stream failed");
   hipLaunchKernelGGL(kg_setup_theta, dim3(nb), dim3(kPassBlock), 0, st, d, alpha, beta, plan, gflags, rclass, thclass,
                      nmax_eq, tau_tot, status);
   if ((rc = check_launch("kg_setup_theta"))) return rc;
   hipLaunchKernelGGL(kg_setup_radial, dim3(nb), dim3(kPassBlock), 0, ss->side, d, alpha, beta, plan);
-  if ((rc = check_launch("kg_setup_radial"))) return rc;
-  if (hipEventRecord(ss->planned, ss->side) != hipSuccess) return fail_msg(KGEO_E_HIP, "plan event failed");
-  return KGEO_OK;
+  rc = check_launch("kg_setup_radial");
+  if (hipEventRecord(ss->planned, ss->side) != hipSuccess) rc = fail_msg(KGEO_E_HIP, "plan event failed");
+  return rc;
 }
 
 int run_series(const DevParams& d, const SampleArgs& a, void* ws, hipStream_t st) {
@@ -559,25 +570,29 @@ int run_series(const DevParams& d, const SampleArgs& a, void* ws, hipStream_t st
     }
     // the heads and the blocks that start from them, beside block 0
     hipLaunchKernelGGL(kg_theta_heads, dim3(np, nbu), dim3(kPassBlock), 0, rs, d, a, rth, nb);
-    if ((rc = check_launch("kg_theta_heads"))) return rc;
-    hipLaunchKernelGGL(kg_radial_heads, dim3(np, nbu), dim3(kPassBlock), 0, rs, d, a, rr, nb);
-    if ((rc = check_launch("kg_radial_heads"))) return rc;
-    for (int64_t b = early ? 1 : 0; b < nb; ++b)
-      if ((rc = a.out.sig ? series(kg_series<true, false>, rs, b) : series(kg_series<false, false>, rs, b))) return rc;
-    if (ss && hipEventRecord(ss->join, rs) != hipSuccess) return fail_msg(KGEO_E_HIP, "join event failed");
-    if (early && (rc = a.out.sig ? series(kg_series<true, true>, st, 0) : series(kg_series<false, true>, st, 0)))
-      return rc;
-    if (ss && hipStreamWaitEvent(st, ss->join, 0) != hipSuccess) return fail_msg(KGEO_E_HIP, "join failed");
+    rc = check_launch("kg_theta_heads");
+    if (!rc) {
+      hipLaunchKernelGGL(kg_radial_heads, dim3(np, nbu), dim3(kPassBlock), 0, rs, d, a, rr, nb);
+      rc = check_launch("kg_radial_heads");
+    }
+    for (int64_t b = early ? 1 : 0; b < nb && !rc; ++b)
+      rc = a.out.sig ? series(kg_series<true, false>, rs, b) : series(kg_series<false, false>, rs, b);
+    const bool marked = !ss || hipEventRecord(ss->join, rs) == hipSuccess;
+    if (early && !rc) rc = a.out.sig ? series(kg_series<true, true>, st, 0) : series(kg_series<false, true>, st, 0);
+    // joined also where a launch failed: what was enqueued uses the caller's buffers
+    if (ss && (!marked || hipStreamWaitEvent(st, ss->join, 0) != hipSuccess))
+      return fail_msg(KGEO_E_HIP, "join failed");
+    if (rc) return rc;
   }
   hipLaunchKernelGGL(kg_fixup, fgrid, dim3(kPassBlock), 0, st, d, a, q);
   return check_launch("kg_fixup");
 }
 
+// pending: run_plan's radial constants are not yet waited for on st.
 int run_sample(const kgeo_ray_params* p, int64_t ngeo, const double* tau_in, double* tau, double* t, double* r,
-               double* th, double* ph, double* sig, uint32_t* status, void* ws, hipStream_t st) {
+               double* th, double* ph, double* sig, uint32_t* status, void* ws, hipStream_t st, bool pending) {
   DevParams d = make_dev(p, ngeo);
   if (d.npix == 0 || ngeo <= 0) return KGEO_OK;
-  if (!t || !ph) return fail_msg(KGEO_E_ARG, "t and ph outputs are required");
   const uint32_t* gflags = static_cast<const uint32_t*>(ws);
   const double* plan = reinterpret_cast<const double*>(static_cast<const char*>(ws) + kFlagBytes);
   const unsigned nb = static_cast<unsigned>((d.npix + kPassBlock - 1) / kPassBlock);
@@ -589,16 +604,29 @@ int run_sample(const kgeo_ray_params* p, int64_t ngeo, const double* tau_in, dou
   if (!tau_in && ngeo > 2) return run_series(d, a, ws, st);
   hipLaunchKernelGGL(kg_theta<true>, grid, dim3(kPassBlock), 0, st, d, a);
   int rc = check_launch("kg_theta");
-  if (rc) return rc;
-  {
-    // the plan's radial constants come from the side stream (run_plan)
-    std::lock_guard<std::mutex> lock(g_side_mu);
-    SideStream* ss = side_stream(st);
-    if (ss && hipStreamWaitEvent(st, ss->planned, 0) != hipSuccess)
-      return fail_msg(KGEO_E_HIP, "wait for the plan failed");
-  }
+  if (rc || (pending && (rc = wait_planned(st)))) return rc;
   hipLaunchKernelGGL(kg_radial<true>, grid, dim3(kPassBlock), 0, st, d, a);
   return check_launch("kg_radial");
+}
+
+int require_outputs(int64_t npix, int64_t ngeo, const double* t, const double* ph) {
+  if (npix > 0 && ngeo > 0 && (!t || !ph)) return fail_msg(KGEO_E_ARG, "t and ph outputs are required");
+  return KGEO_OK;
+}
+
+// A plan and its samples in one call.  Where no sample pass ran to its end,
+// the caller's stream waits for the plan here.
+int plan_and_sample(const kgeo_ray_params* p, const double* alpha, const double* beta, int64_t ngeo,
+                    const double* tau_in, double* tau, double* t, double* r, double* th, double* ph, double* sig,
+                    int8_t* rclass, int8_t* thclass, int32_t* nmax_eq, double* tau_tot, uint32_t* status, void* ws,
+                    hipStream_t st) {
+  int rc = run_plan(p, alpha, beta, rclass, thclass, nmax_eq, tau_tot, status, ws, st);
+  if (!rc) rc = run_sample(p, ngeo, tau_in, tau, t, r, th, ph, sig, status, ws, st, true);
+  if (p->npix > 0 && (rc || ngeo <= 0)) {
+    const int wrc = wait_planned(st);
+    if (!rc) rc = wrc;
+  }
+  return rc;
 }
 
 }  // namespace
@@ -638,8 +666,10 @@ int kgeo_plan(const kgeo_ray_params* p, const double* alpha, const double* beta,
               void* stream) {
   int rc = validate(p, alpha, beta, workspace, workspace_bytes, 0);
   if (rc) return rc;
-  return run_plan(p, alpha, beta, rclass, thclass, nmax_eq, tau_tot, status, workspace,
-                  static_cast<hipStream_t>(stream));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  rc = run_plan(p, alpha, beta, rclass, thclass, nmax_eq, tau_tot, status, workspace, st);
+  const int wrc = p->npix > 0 ? wait_planned(st) : KGEO_OK;
+  return rc ? rc : wrc;
 }
 
 int kgeo_sample(const kgeo_ray_params* p, const double* tau_in, int64_t ntau, double* tau, double* t, double* r,
@@ -653,7 +683,8 @@ int kgeo_sample(const kgeo_ray_params* p, const double* tau_in, int64_t ntau, do
   const size_t need = kgeo_workspace_bytes(p->npix, tau_in ? 0 : ntau);
   if (workspace_bytes < need)
     return fail(KGEO_E_WORKSPACE, "workspace too small%s: need %lld bytes", "", static_cast<long long>(need));
-  return run_sample(p, ntau, tau_in, tau, t, r, th, ph, sig, status, workspace, static_cast<hipStream_t>(stream));
+  if (require_outputs(p->npix, ntau, t, ph)) return KGEO_E_ARG;
+  return run_sample(p, ntau, tau_in, tau, t, r, th, ph, sig, status, workspace, static_cast<hipStream_t>(stream), false);
 }
 
 int kgeo_raytrace_ana(const kgeo_ray_params* p, const double* alpha, const double* beta, double* tau, double* t,
@@ -663,10 +694,9 @@ int kgeo_raytrace_ana(const kgeo_ray_params* p, const double* alpha, const doubl
   int rc = validate(p, alpha, beta, workspace, workspace_bytes, p ? p->ngeo : 0);
   if (rc) return rc;
   if (p->ngeo < 1) return fail(KGEO_E_ARG, "ngeo < 1%s (%lld)", "", p->ngeo);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  rc = run_plan(p, alpha, beta, rclass, thclass, nmax_eq, tau_tot, status, workspace, st);
-  if (rc) return rc;
-  return run_sample(p, p->ngeo, nullptr, tau, t, r, th, ph, sig, status, workspace, st);
+  if (require_outputs(p->npix, p->ngeo, t, ph)) return KGEO_E_ARG;
+  return plan_and_sample(p, alpha, beta, p->ngeo, nullptr, tau, t, r, th, ph, sig, rclass, thclass, nmax_eq, tau_tot,
+                         status, workspace, static_cast<hipStream_t>(stream));
 }
 
 int kgeo_coords_at_tau(const kgeo_ray_params* p, const double* alpha, const double* beta, const double* tau_in,
@@ -676,10 +706,9 @@ int kgeo_coords_at_tau(const kgeo_ray_params* p, const double* alpha, const doub
   if (rc) return rc;
   if (ntau < 0) return fail(KGEO_E_ARG, "ntau < 0%s (%lld)", "", ntau);
   if (ntau > 0 && p->npix > 0 && !tau_in) return fail_msg(KGEO_E_ARG, "tau_in is NULL");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  rc = run_plan(p, alpha, beta, nullptr, nullptr, nullptr, nullptr, status, workspace, st);
-  if (rc) return rc;
-  return run_sample(p, ntau, tau_in, nullptr, t, r, th, ph, sig, status, workspace, st);
+  if (require_outputs(p->npix, ntau, t, ph)) return KGEO_E_ARG;
+  return plan_and_sample(p, alpha, beta, ntau, tau_in, nullptr, t, r, th, ph, sig, nullptr, nullptr, nullptr, nullptr,
+                         status, workspace, static_cast<hipStream_t>(stream));
 }
 
 int kgeo_crossings(const kgeo_ray_params* p, const double* alpha, const double* beta, const double* tau,
