@@ -1297,6 +1297,7 @@ enum PlanSlot : int {
   PL_QB,
   PL_QC,
   PL_U0,     // d cos(theta)/dtau at the observer
+  PL_RWALK,  // the radial modulus is below 1 (radial_modulus)
   PL_N
 };
 
@@ -1324,6 +1325,29 @@ template <class T> KG_INLINE void radial_quartic(const PixelSetup<T>& px, T& A, 
   C = p * q;
 }
 
+// The radial modulus of the roots, as radial_consts has it (whose slots the
+// first block of a ray must not read yet, kg_series_pass.hpp).
+template <class T> KG_INLINE T radial_modulus(const PixelSetup<T>& px) {
+#if defined(__clang__)
+#pragma clang fp contract(off)
+#endif
+  if (px.rcase == 4) {
+    const T a1 = px.ri[3], b1 = px.rr[3], a2 = px.ri[1], b2 = px.rr[1];
+    const T CC = ksqrt(sq(a1 - a2) + sq(b1 - b2));
+    const T DD = ksqrt(sq(a1 + a2) + sq(b1 - b2));
+    return (4.0 * CC * DD) / sq(CC + DD);
+  }
+  if (px.rcase == 3) {
+    const T a1 = px.ri[3], b1 = px.rr[3], rr1 = px.rr[0], rr2 = px.rr[1];
+    const T rr21 = rr2 - rr1;
+    const T AA = ksqrt(a1 * a1 + sq(b1 - rr2));
+    const T BB = ksqrt(a1 * a1 + sq(b1 - rr1));
+    return (sq(AA + BB) - rr21 * rr21) / (4.0 * AA * BB);
+  }
+  const T rr1 = px.rr[0], rr2 = px.rr[1], rr3 = px.rr[2], rr4 = px.rr[3];
+  return ((rr3 - rr2) * (rr4 - rr1)) / ((rr3 - rr1) * (rr4 - rr2));
+}
+
 // The plan in two parts: theta, lambda and the grid stop; the radial
 // constants (PL_R .. PL_R + R_NSLOT - 1 and PL_RCASE).
 KG_INLINE void plan_pack_theta(const ThetaConsts<double>& tc, const PixelSetup<double>& px, double stop,
@@ -1332,6 +1356,7 @@ KG_INLINE void plan_pack_theta(const ThetaConsts<double>& tc, const PixelSetup<d
   plan[PL_LAM] = px.lam;
   radial_quartic(px, plan[PL_QA], plan[PL_QB], plan[PL_QC]);
   plan[PL_U0] = tc.u0;
+  plan[PL_RWALK] = radial_modulus(px) < 1.0 ? 1.0 : 0.0;
   plan[PL_STOP] = stop;
   plan[PL_THK] = static_cast<double>(tc.kind);
   plan[PL_ETA0] = static_cast<double>(tc.eta_zero);

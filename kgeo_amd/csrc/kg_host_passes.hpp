@@ -7,6 +7,7 @@
 #pragma once
 
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "kg_sample.hpp"
@@ -101,10 +102,11 @@ void three_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, c
 
 // The series passes over all pixels, in the kernels' order: heads of both
 // coordinates, the blocks in `parts` parts each, then the fixups of theta and r over one queue.
+// early: block 0 as the plain kernels run it above MINSPIN, reading no radial constant and no record.
 // nfix[0] receives the queue's length (-1 past the kernels' capacity).
 template <class T>
 void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, const SampleOut& o, int64_t parts,
-                   uint32_t* st, int64_t* nfix) {
+                   bool early, uint32_t* st, int64_t* nfix) {
   const int64_t npix = o.npix, G = o.ngeo, nb = series_blocks(G);
   std::vector<double> trec(static_cast<size_t>(nb) * kThSFields * npix), rrec(static_cast<size_t>(nb) * kRSFields * npix);
   const Records rth{trec.data(), npix, 0}, rr{rrec.data(), npix, 0};
@@ -113,14 +115,20 @@ void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, 
   for (int64_t i = 0; i < npix; ++i)
     for (int64_t hd = 0; hd < nb; ++hd) {
       st[i] |= series_theta_head_pixel<T>(plan, npix, i, gflags, o, i, hd, nb, rth);
-      st[i] |= series_radial_head_pixel<T>(plan, npix, i, gflags, o, i, hd, nb, val(c.r_o), rr);
+      st[i] |= series_radial_head_pixel<T>(plan, npix, i, gflags, o, i, hd, nb, rr);
     }
   for (int64_t i = 0; i < npix; ++i)
     for (int64_t u = 0; u < nb * parts; ++u) {
       const int64_t b = u / parts, q = u % parts;
       LocalSlots<T> slots;
-      st[i] |= o.sig ? series_block_pixel<true, false, LocalSlots<T>, HostPush, T>(c, plan, npix, i, gflags, o, i, true, b, nb, q, parts, rth, rr, slots, push)
-                     : series_block_pixel<false, false, LocalSlots<T>, HostPush, T>(c, plan, npix, i, gflags, o, i, true, b, nb, q, parts, rth, rr, slots, push);
+      auto block = [&](auto sig, auto early0) {
+        return series_block_pixel<decltype(sig)::value, decltype(early0)::value, LocalSlots<T>, HostPush, T>(
+            c, plan, npix, i, gflags, o, i, true, b, nb, q, parts, rth, rr, slots, push);
+      };
+      const std::true_type yes;
+      const std::false_type no;
+      if (early && b == 0 && nb > 1 && !c.minspin) st[i] |= o.sig ? block(yes, yes) : block(no, yes);
+      else st[i] |= o.sig ? block(yes, no) : block(no, no);
     }
   const size_t cap = static_cast<size_t>(npix) * static_cast<size_t>(series_items(G));
   nfix[0] = items.size() <= cap ? static_cast<int64_t>(items.size()) : -1;

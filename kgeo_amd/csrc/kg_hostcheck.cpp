@@ -115,6 +115,8 @@ void kgh_setup(const double* sc, const double* alpha, const double* beta, int64_
 //   passes = 4: the heads / series / fixup passes with each block in `chunks` parts,
 //               per ray (the kernels' path for the linspace grid with ngeo >
 //               2); nfix (optional) receives the fixup queue's length;
+//   passes = 5: the same with block 0 as the plain kernels run it above
+//               MINSPIN, which read no radial constant and no record there;
 //   passes = 3: the anchor / walk / fixup passes (the same samples by the
 //               addition theorems); nfix[3] (optional) receives the
 //               theta and radial fixup-queue lengths and the radial repair
@@ -150,9 +152,9 @@ void kgh_raytrace_passes(const double* sc, const double* alpha, const double* be
     o.t = nullptr;
     o.ph = nullptr;
   }
-  if ((passes == 3 || (passes == 4 && do_phi_t)) && !tau_in && G > 2) {
+  if ((passes == 3 || (passes >= 4 && do_phi_t)) && !tau_in && G > 2) {
     int64_t nf[3] = {0, 0, 0};
-    if (passes == 4) series_passes<double>(c, plan.data(), gflags, o, chunks, st.data(), nf);
+    if (passes >= 4) series_passes<double>(c, plan.data(), gflags, o, chunks, passes == 5, st.data(), nf);
     else if (do_phi_t) three_passes<true, double>(c, plan.data(), gflags, o, chunks, st.data(), nf);
     else three_passes<false, double>(c, plan.data(), gflags, o, chunks, st.data(), nf);
     if (nfix) {

@@ -170,6 +170,13 @@ template <class T> KG_INLINE T radial_motion(const RadialConsts<T>& rc, const RS
   return 2.0 * Xs * v[C2_rr41] * v[C2_rr31] * v[C2_rr43] * (st.s * st.c * st.d) / (num * num);
 }
 
+// Whether the heads and the series serve a pixel: its motion and its radial
+// modulus (theta_pick's walk, PL_RWALK).  The same in every pass, block 0's
+// included; the fixup pass takes the other pixels whole.
+KG_INLINE bool series_serves(const double* __restrict__ plan, int64_t stride, int64_t p, const ThetaPick& tp) {
+  return tp.walk && plan[static_cast<int64_t>(PL_RWALK) * stride + p] != 0.0;
+}
+
 // Theta head hd (0 the last sample, b the anchor of block b) of output pixel
 // i: theta and the parked G_phi, G_t of its sample, and an anchor's motion.
 template <class T = double>
@@ -177,7 +184,7 @@ KG_INLINE uint32_t series_theta_head_pixel(const double* __restrict__ plan, int6
                                            const SampleOut& o, int64_t i, int64_t hd, int64_t nb, const Records& rt) {
   ThetaConsts<T> tc;
   const ThetaPick tp = theta_pick(plan, stride, p, gflags, o, tc);
-  if (!tp.walk) return 0u;
+  if (!series_serves(plan, stride, p, tp)) return 0u;
   tc.kind = tp.kind;
   JacobiLadder<T> lad;
   jacobi_ladder(tc.v[TH_mp], lad);
@@ -212,13 +219,9 @@ KG_INLINE uint32_t series_theta_head_pixel(const double* __restrict__ plan, int6
 template <class T = double>
 KG_INLINE uint32_t series_radial_head_pixel(const double* __restrict__ plan, int64_t stride, int64_t p,
                                             uint32_t gflags, const SampleOut& o, int64_t i, int64_t hd, int64_t nb,
-                                            double r_o, const Records& rt) {
-  if (!radial_walks(o, gflags, plan[static_cast<int64_t>(PL_R + R_k) * stride + p])) {
-    // its blocks leave every sample to the fixup pass, but an early block 0
-    // (series_block_pixel), which cannot know, still writes its own
-    if (hd == 0 && o.r) o.r[i] = r_o;
+                                            const Records& rt) {
+  if (!walk_ok(o, (gflags & GF_ANY_STEP_ZERO) != 0) || plan[static_cast<int64_t>(PL_RWALK) * stride + p] == 0.0)
     return 0u;
-  }
   RadialConsts<T> rc;
   T lam;
   double stop;
@@ -311,10 +314,7 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
     const ThetaPick tp = theta_pick(plan, stride, p, gflags, o, tc);
     stop = tp.stop;
     const T lam = T(plan[static_cast<int64_t>(PL_LAM) * stride + p]);
-    // EARLY: the plan's radial constants may still be being written
-    const bool walks =
-        tp.walk && (EARLY || radial_walks(o, gflags, plan[static_cast<int64_t>(PL_R + R_k) * stride + p]));
-    if (live && !walks) {
+    if (live && !series_serves(plan, stride, p, tp)) {
       // no heads for this pixel either: every sample, the last included
       push_windows(push, i, ps, ends ? o.ngeo : pe, false);
       live = false;

@@ -209,8 +209,7 @@ template <bool THETA> __device__ inline void batch_heads(const BatchDev& d) {
           const SampleOut o = image_out(d, B);
           const Records rt = image_records(d, B, THETA);
           return THETA ? series_theta_head_pixel(d.plan, d.total_slots, s, d.flags[k], o, i, hd, B.units[K_HEAD], rt)
-                       : series_radial_head_pixel(d.plan, d.total_slots, s, d.flags[k], o, i, hd, B.units[K_HEAD],
-                                                  B.c.r_o, rt);
+                       : series_radial_head_pixel(d.plan, d.total_slots, s, d.flags[k], o, i, hd, B.units[K_HEAD], rt);
         });
     if (im != last && count) {
       atomicAdd(&d.done[last], lane == 0 ? count : 0u);

@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kPassBlock) void kg_theta_heads(DevParams p, Sample
 __global__ __launch_bounds__(kPassBlock) void kg_radial_heads(DevParams p, SampleArgs a, Records rt, int64_t nb) {
   const int64_t i = tile_of(blockIdx.x, gridDim.x) * kPassBlock + threadIdx.x;
   if (i >= p.npix) return;
-  const uint32_t st = series_radial_head_pixel(a.plan, p.npix, i, a.gflags[0], a.out, i, blockIdx.y, nb, p.c.r_o, rt);
+  const uint32_t st = series_radial_head_pixel(a.plan, p.npix, i, a.gflags[0], a.out, i, blockIdx.y, nb, rt);
   if (a.status && st) atomicOr(&a.status[i], st);
 }
 
