@@ -1297,7 +1297,7 @@ enum PlanSlot : int {
   PL_QB,
   PL_QC,
   PL_U0,     // d cos(theta)/dtau at the observer
-  PL_RWALK,  // the radial modulus is below 1 (radial_modulus)
+  PL_SERVED, // the series may serve the ray (series_may_serve)
   PL_N
 };
 
@@ -1348,16 +1348,27 @@ template <class T> KG_INLINE T radial_modulus(const PixelSetup<T>& px) {
   return ((rr3 - rr2) * (rr4 - rr1)) / ((rr3 - rr1) * (rr4 - rr2));
 }
 
+// Rays that the series may serve: of radial modulus below 1, and sampled from
+// the observer on, up to at most half their length past their end
+// (kSeriesPast).  Further out, through the horizon or infinity more than once,
+// a sample is too far from an anchor: r is off by up to 1e-10 at twice the
+// length and 2e-8 at three times it (3e-12 at 1.5), and half the samples are
+// refused.  Backwards (maxtaufrac < 0) the axis angle would turn the wrong way.
+constexpr double kSeriesPast = 1.5;
+template <class T> KG_INLINE bool series_may_serve(const PixelSetup<T>& px, double maxtaufrac) {
+  return val(radial_modulus(px)) < 1.0 && maxtaufrac > 0.0 && maxtaufrac <= kSeriesPast;
+}
+
 // The plan in two parts: theta, lambda and the grid stop; the radial
 // constants (PL_R .. PL_R + R_NSLOT - 1 and PL_RCASE).
-KG_INLINE void plan_pack_theta(const ThetaConsts<double>& tc, const PixelSetup<double>& px, double stop,
+KG_INLINE void plan_pack_theta(const ThetaConsts<double>& tc, const PixelSetup<double>& px, double maxtaufrac,
                                double* plan) {
   for (int i = 0; i < TH_NSLOT; ++i) plan[PL_TH + i] = tc.v[i];
   plan[PL_LAM] = px.lam;
   radial_quartic(px, plan[PL_QA], plan[PL_QB], plan[PL_QC]);
   plan[PL_U0] = tc.u0;
-  plan[PL_RWALK] = radial_modulus(px) < 1.0 ? 1.0 : 0.0;
-  plan[PL_STOP] = stop;
+  plan[PL_SERVED] = series_may_serve(px, maxtaufrac) ? 1.0 : 0.0;
+  plan[PL_STOP] = maxtaufrac * px.tau_tot;
   plan[PL_THK] = static_cast<double>(tc.kind);
   plan[PL_ETA0] = static_cast<double>(tc.eta_zero);
 }
@@ -1370,8 +1381,8 @@ KG_INLINE void plan_pack_radial(const RadialConsts<double>& rc, double* plan) {
 KG_INLINE bool plan_slot_radial(int s) { return (s >= PL_R && s < PL_R + R_NSLOT) || s == PL_RCASE; }
 
 KG_INLINE void plan_pack(const ThetaConsts<double>& tc, const RadialConsts<double>& rc, const PixelSetup<double>& px,
-                         double stop, double* plan) {
-  plan_pack_theta(tc, px, stop, plan);
+                         double maxtaufrac, double* plan) {
+  plan_pack_theta(tc, px, maxtaufrac, plan);
   plan_pack_radial(rc, plan);
 }
 
@@ -1415,7 +1426,7 @@ KG_INLINE PixelSetup<double> plan_pixel(const RayScalars<double>& c, double alph
   RadialConsts<double> rc;
   theta_consts(c, px, do_phi_t, tc);
   radial_consts(c, px, do_phi_t, rc);
-  plan_pack(tc, rc, px, c.maxtaufrac * px.tau_tot, plan);
+  plan_pack(tc, rc, px, c.maxtaufrac, plan);
   return px;
 }
 
@@ -1426,7 +1437,7 @@ KG_INLINE PixelSetup<double> plan_pixel_theta(const RayScalars<double>& c, doubl
   pixel_setup(c, alpha, beta, px);
   ThetaConsts<double> tc;
   theta_consts(c, px, do_phi_t, tc);
-  plan_pack_theta(tc, px, c.maxtaufrac * px.tau_tot, plan);
+  plan_pack_theta(tc, px, c.maxtaufrac, plan);
   return px;
 }
 

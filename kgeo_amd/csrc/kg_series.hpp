@@ -205,6 +205,7 @@ enum SeriesSlot : int {
   SF_af, SF_wrap,             // the angle's factor in phi, and 2 pi of it past a pass
   SE_w, SE_v, SE_c, SE_u,     // the state where the last expansion ended
   SE_t, SE_f, SE_s,
+  SE_q,                       // samples before this one (from the block's first) are queued
   SERIES_SLOTS
 };
 

@@ -43,6 +43,9 @@ namespace kg {
 constexpr int kSeriesBlocks = 2;
 constexpr int kSeriesMaxParts = 8;
 constexpr double kSeriesMinStep = 128.0;
+// Rays followed past their end: |r - r_+|, and |r|/r_o on the way out, beyond
+// which the closed forms are not used.
+constexpr double kSeriesHorizon = 1.0e-3, kSeriesFar = 0.1;
 // An expansion holds for the same distance x on both sides of its centre, so
 // the next is centred ahead of where the last ended, by this part of its x:
 // the distance to the nearest singularity (about 10 x) shrinks by at most the
@@ -170,11 +173,11 @@ template <class T> KG_INLINE T radial_motion(const RadialConsts<T>& rc, const RS
   return 2.0 * Xs * v[C2_rr41] * v[C2_rr31] * v[C2_rr43] * (st.s * st.c * st.d) / (num * num);
 }
 
-// Whether the heads and the series serve a pixel: its motion and its radial
-// modulus (theta_pick's walk, PL_RWALK).  The same in every pass, block 0's
-// included; the fixup pass takes the other pixels whole.
+// Whether the heads and the series serve a pixel: its motion (theta_pick's
+// walk) and PL_SERVED.  The same in every pass, block 0's included; the fixup
+// pass takes the other pixels whole.
 KG_INLINE bool series_serves(const double* __restrict__ plan, int64_t stride, int64_t p, const ThetaPick& tp) {
-  return tp.walk && plan[static_cast<int64_t>(PL_RWALK) * stride + p] != 0.0;
+  return tp.walk && plan[static_cast<int64_t>(PL_SERVED) * stride + p] != 0.0;
 }
 
 // Theta head hd (0 the last sample, b the anchor of block b) of output pixel
@@ -220,7 +223,7 @@ template <class T = double>
 KG_INLINE uint32_t series_radial_head_pixel(const double* __restrict__ plan, int64_t stride, int64_t p,
                                             uint32_t gflags, const SampleOut& o, int64_t i, int64_t hd, int64_t nb,
                                             const Records& rt) {
-  if (!walk_ok(o, (gflags & GF_ANY_STEP_ZERO) != 0) || plan[static_cast<int64_t>(PL_RWALK) * stride + p] == 0.0)
+  if (!walk_ok(o, (gflags & GF_ANY_STEP_ZERO) != 0) || plan[static_cast<int64_t>(PL_SERVED) * stride + p] == 0.0)
     return 0u;
   RadialConsts<T> rc;
   T lam;
@@ -396,6 +399,8 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
   k.set(SE_t, st.t);
   k.set(SE_f, st.f);
   k.set(SE_s, st.s);
+  k.set(SE_q, T(0.0));
+  const bool past = c.maxtaufrac > 1.0;
   // in samples from js, multiples of 2^-10 (exact): x0, up to where the
   // samples are done, and the expansion's centre x0 + d
   double x0 = 0.0, d = 0.0;
@@ -406,7 +411,10 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
     k.fresh();
     float x = series_expand<T, P, SIG>(c, k, st, S);
     if (!(x >= floor_x)) {  // also NaN
-      if (live) push_windows(push, i, j < ps ? ps : j, pe, true);
+      if (live) {
+        const int64_t from = j < ps ? ps : j, queued = js + static_cast<int64_t>(val(k(SE_q)));
+        push_windows(push, i, from < queued ? queued : from, pe, true);
+      }
       live = false;
     }
     x = live ? (x < 1.0e29f ? x : 1.0e29f) : 1.0e30f;  // all coefficients 0: no bound
@@ -442,7 +450,16 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
         o.t[idx] = val(-s.t);
         o.ph[idx] = val(-s.f);
         if (SIG) o.sig[idx] = val(-s.s);
-        bad = bad | !(kfabs(val(r)) + kfabs(val(th)) + kfabs(val(s.t)) + kfabs(val(s.f)) < INFINITY);
+        // a sample at a pole that the closed forms take out (0 times infinity) or,
+        // of rays followed past their end, next to the horizon, where only the
+        // direct formulas reproduce the reference's rounding: to the fixup
+        // pass, with the rest of its window
+        const bool odd = !(kfabs(val(r)) + kfabs(val(th)) + kfabs(val(s.t)) + kfabs(val(s.f)) < INFINITY) ||
+                         (past && kfabs(val(r) - val(c.rplus)) < kSeriesHorizon);
+        if (odd && j - js >= static_cast<int64_t>(val(k(SE_q)))) {
+          push(i, j, true);
+          k.set(SE_q, T(static_cast<double>(series_fixup_end(j, o.ngeo, true) - js)));
+        }
       }
     }
     if (j >= pe) break;
@@ -450,7 +467,13 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
       SeriesState<T> e;
       T r, an;
       series_at<T, P, SIG, true>(k, S, T(x1 - xc), e, r, an);
-      k.set(SE_w, e.w);
+      // past the end of the ray the state may be handed on next to the horizon
+      // or on the way through infinity, where the closed forms' terms have lost
+      // the integrals' digits (an error of w by 1e-15 is one of r by 1e-15 r^2):
+      // the rest is refused
+      const bool lost = past && (kfabs(val(r) - val(c.rplus)) < kSeriesHorizon ||
+                                 (val(e.v) < 0.0 && kfabs(val(r)) > kSeriesFar * c.r_o));
+      k.set(SE_w, lost ? T(NAN) : e.w);
       k.set(SE_v, e.v);
       k.set(SE_c, e.c);
       k.set(SE_u, e.u);
