@@ -127,7 +127,7 @@ void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, 
       };
       const std::true_type yes;
       const std::false_type no;
-      if (early && b == 0 && nb > 1 && !c.minspin) st[i] |= o.sig ? block(yes, yes) : block(no, yes);
+      if (early && b == 0 && nb > 1 && !c.minspin && !c.r_o_inf) st[i] |= o.sig ? block(yes, yes) : block(no, yes);
       else st[i] |= o.sig ? block(yes, no) : block(no, no);
     }
   const size_t cap = static_cast<size_t>(npix) * static_cast<size_t>(series_items(G));
@@ -139,7 +139,7 @@ void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, 
       int64_t i, j;
       bool w;
       unpack_host_item(e, i, j, w);
-      const int64_t end = series_fixup_end(j, G, w);
+      const int64_t end = series_fixup_end(j, G, w, c.r_o_inf != 0);
       for (int64_t sg = 0; sg < kFixupSpan; ++sg)
         st[i] |= part == 0 ? theta_fixup_sample<true, T>(plan, npix, i, gflags, o, i, j, end, sg)
                            : radial_fixup_sample<true, T>(c, plan, npix, i, gflags, o, i, j, end, sg);

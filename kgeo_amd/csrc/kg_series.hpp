@@ -569,9 +569,12 @@ KG_INLINE void series_at(const Slots& k, const Series<T, P, SIG>& S, const T& x,
 }
 
 // The integrals' constants of a new expansion: t0, f0, s0 at its left end, the
-// offset x (where the last one ended).
+// offset x (where the last one ended).  far (an observer at infinity): t0 and
+// s0 are the reference's constants of the ray, infinite, NaN or about 1e16, of
+// which the terms at the left end, infinite too, are a part already.
 template <class T, int P, bool SIG, class Slots>
-KG_INLINE void series_match(Slots& k, Series<T, P, SIG>& S, const T& x, const T& t0, const T& f0, const T& s0) {
+KG_INLINE void series_match(Slots& k, Series<T, P, SIG>& S, const T& x, const T& t0, const T& f0, const T& s0,
+                            bool far) {
   S.t[0] = T(0.0);
   S.f[0] = T(0.0);
   S.s[0] = T(0.0);
@@ -579,9 +582,9 @@ KG_INLINE void series_match(Slots& k, Series<T, P, SIG>& S, const T& x, const T&
   SeriesState<T> o;
   T r, an;
   series_at<T, P, SIG, false>(k, S, x, o, r, an);
-  S.t[0] = t0 - o.t;
+  S.t[0] = far ? t0 : t0 - o.t;
   S.f[0] = f0 - o.f;
-  if (SIG) S.s[0] = s0 - o.s;
+  if (SIG) S.s[0] = far ? s0 : s0 - o.s;
   // approaching (an < 0): a later angle > 0 is past the pass, a turn further on
   k.set(SF_wrap, val(an) < 0.0 ? 2.0 * kPi * k(SF_af) : T(0.0));
 }

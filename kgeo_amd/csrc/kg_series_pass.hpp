@@ -89,16 +89,22 @@ KG_INLINE int64_t series_part(int64_t js, int64_t je, int64_t q, int64_t parts) 
 }
 
 // End of the queued range that starts at sample j: fixup_end, or the end of
-// j's block before it.
-KG_INLINE int64_t series_fixup_end(int64_t j, int64_t ngeo, bool walked) {
+// j's block before it.  far (an observer at infinity): sample 0 of the served
+// rays is a range of its own.
+KG_INLINE int64_t series_fixup_end(int64_t j, int64_t ngeo, bool walked, bool far) {
   const int64_t e = fixup_end(j, ngeo, walked), nb = series_blocks(ngeo);
+  if (far && walked && j == 0) return 1;
   const int64_t s = nb > 1 ? series_start(ngeo, 1, nb) : 0;
   return (j < s && s < e) ? s : e;
 }
 
-// Queued ranges per pixel at most: one per window of kFixupSpan samples, and
-// one more for the window that the second block starts in.
-KG_INLINE int64_t series_items(int64_t ngeo) { return fixup_items(ngeo) + (series_blocks(ngeo) - 1); }
+// Queued ranges per pixel at most: one per window of kFixupSpan samples, one
+// more for the window that the second block starts in and one for the sample 0
+// of an observer at infinity.
+constexpr int64_t kSeriesMoreItems = 2;
+KG_INLINE int64_t series_items(int64_t ngeo) {
+  return fixup_items(ngeo) + (series_blocks(ngeo) > 1 ? kSeriesMoreItems : 1);
+}
 
 // Queue samples j .. e - 1 of a block: from j to the next window, then one
 // item per window.  walked: the last grid sample is a head's.
@@ -292,7 +298,8 @@ KG_INLINE bool series_head_store(const SampleOut& o, const CombineConsts<T>& cmb
 // series.  All lanes of a wave call together; `in` is false for a lane without a pixel
 // (its i and p must be valid).  EARLY: block 0 of several, which reads nothing
 // of the plan's radial constants (kg_setup_radial may still be writing them)
-// and no record; not below MINSPIN.  Returns the status bits.
+// and no record; not below MINSPIN, and for no observer at infinity, whose t
+// and sigma start from the anchor's.  Returns the status bits.
 template <bool SIG, bool EARLY, class Slots, class Push, class T = double>
 KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __restrict__ plan, int64_t stride,
                                       int64_t p, uint32_t gflags, const SampleOut& o, int64_t i, bool in, int64_t b,
@@ -310,6 +317,7 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
   if (ps >= pe) return 0u;  // never the block's last part
   SeriesState<T> st;
   double stop;
+  const bool far = !EARLY && c.r_o_inf;
   bool live = in;
   bool bad = false;
   {
@@ -338,42 +346,50 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
     const CombineConsts<T> cmb = combine_consts(c, lam);
     if (!EARLY && live && ends) bad = series_head_store<T>(o, cmb, last * o.npix + i, stop, rr, 0, p) || bad;
     const int64_t idx = js * o.npix + i;
+    st.t = T(0.0);
+    st.f = T(0.0);
+    st.s = T(0.0);
     if (EARLY || b == 0) {
-      const T w0 = 1.0 / T(c.r_o);
+      // from infinity: 1/w and 1/w^2 finite, w as good as 0
+      const T w0 = far ? T(1.0e-30) : 1.0 / T(c.r_o);
       st.w = w0;
       st.v = ksqrt(1.0 + w0 * w0 * (k(SR_A) + w0 * (k(SR_B) + w0 * k(SR_C))));
       st.c = c.cos_th;
       st.u = T(plan[static_cast<int64_t>(PL_U0) * stride + p]);
-      st.t = T(0.0);
-      st.f = T(0.0);
-      st.s = T(0.0);
     } else {
-      const double tau = mino_tau(js, o.ngeo, stop, false);
       st.c = T(*rth.at(b, kThSFields, 0, p));
       st.u = T(*rth.at(b, kThSFields, 1, p));
       st.w = 1.0 / T(*rr.at(b, kRSFields, 0, p));
       st.v = T(*rr.at(b, kRSFields, 5, p));
-      if (live) {
-        RadialOut<T> ro;
-        ro.r = T(*rr.at(b, kRSFields, 0, p));
-        ro.Ip = T(*rr.at(b, kRSFields, 1, p));
-        ro.Im = T(*rr.at(b, kRSFields, 2, p));
-        ro.I1 = T(*rr.at(b, kRSFields, 3, p));
-        ro.I2 = T(*rr.at(b, kRSFields, 4, p));
-        Sample<T> s;
-        combine(cmb, T(tau), ro, T(0.0), T(*rth.at(b, kThSFields, 2, p)), T(*rth.at(b, kThSFields, 3, p)), s);
-        st.t = -s.t;
-        st.f = -s.ph;
-        st.s = -s.sig;
-      }
     }
-    // the series needs a pole at the axis (lam != 0), a bounded observer and
-    // a finite start
+    if (!EARLY && live && nb > 1 && (b > 0 || far)) {
+      const int64_t hd = b > 0 ? b : 1;
+      RadialOut<T> ro;
+      ro.r = T(*rr.at(hd, kRSFields, 0, p));
+      ro.Ip = T(*rr.at(hd, kRSFields, 1, p));
+      ro.Im = T(*rr.at(hd, kRSFields, 2, p));
+      ro.I1 = T(*rr.at(hd, kRSFields, 3, p));
+      ro.I2 = T(*rr.at(hd, kRSFields, 4, p));
+      Sample<T> s;
+      combine(cmb, T(mino_tau(series_start(o.ngeo, hd, nb), o.ngeo, stop, false)), ro, T(0.0),
+              T(*rth.at(hd, kThSFields, 2, p)), T(*rth.at(hd, kThSFields, 3, p)), s);
+      st.t = -s.t;
+      st.s = -s.sig;
+      if (b > 0) st.f = -s.ph;
+    }
+    // the series needs a pole at the axis (lam != 0) and a finite start; t and
+    // sigma of an observer at infinity are what the anchor's are
+    const bool fin = kfinite(val(st.t)) && kfinite(val(st.s));
     const bool ok = kfinite(val(st.w)) & kfinite(val(st.v)) & kfinite(val(st.c)) & kfinite(val(st.u)) &
-                    kfinite(val(st.t)) & kfinite(val(st.f)) & (val(k(SR_l2)) > 0.0) & (val(lam) != 0.0) &
+                    (far ? nb > 1 : fin) & kfinite(val(st.f)) & (val(k(SR_l2)) > 0.0) & (val(lam) != 0.0) &
                     (val(st.w) > 0.0) & kfinite(val(k(SR_E))) & kfinite(val(h));
+    bad = bad || (live && ok && !fin);
+    // at infinity itself t and sigma are the difference of two infinite terms:
+    // as the reference has it
+    const int64_t first = far && b == 0 ? 1 : 0;
+    if (live && ps < first) push(i, 0, true);
     if (live && !ok) {
-      push_windows(push, i, ps, pe, true);
+      push_windows(push, i, ps < first ? first : ps, pe, true);
       live = false;
     }
     if (live && ps == js) {
@@ -426,7 +442,7 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
       series_advance<T>(k, T(d), st);
       continue;
     }
-    series_match<T, P, SIG>(k, S, T(-d), k(SE_t), k(SE_f), k(SE_s));
+    series_match<T, P, SIG>(k, S, T(-d), k(SE_t), k(SE_f), k(SE_s), far);
     const double xc = x0 + d;
     double x1 = xc + static_cast<double>(x);
     if (x1 > xe) x1 = xe;
@@ -454,11 +470,12 @@ KG_INLINE uint32_t series_block_pixel(const RayScalars<T>& c, const double* __re
         // of rays followed past their end, next to the horizon, where only the
         // direct formulas reproduce the reference's rounding: to the fixup
         // pass, with the rest of its window
-        const bool odd = !(kfabs(val(r)) + kfabs(val(th)) + kfabs(val(s.t)) + kfabs(val(s.f)) < INFINITY) ||
+        // (t has the same terms as r and phi)
+        const bool odd = !(kfabs(val(r)) + kfabs(val(th)) + kfabs(val(s.f)) < INFINITY) ||
                          (past && kfabs(val(r) - val(c.rplus)) < kSeriesHorizon);
         if (odd && j - js >= static_cast<int64_t>(val(k(SE_q)))) {
           push(i, j, true);
-          k.set(SE_q, T(static_cast<double>(series_fixup_end(j, o.ngeo, true) - js)));
+          k.set(SE_q, T(static_cast<double>(series_fixup_end(j, o.ngeo, true, false) - js)));
         }
       }
     }

@@ -268,7 +268,7 @@ __global__ __launch_bounds__(kBlock) void kg_batch_fixup(BatchDev d) {
     const int64_t s = B.slot_off + i;
     const uint32_t fl = d.flags[im];
     const SampleOut o = image_out(d, B);
-    const int64_t end = series_fixup_end(j, B.ngeo, walked);
+    const int64_t end = series_fixup_end(j, B.ngeo, walked, B.c.r_o_inf != 0);
     uint32_t st = theta_fixup_sample<true>(d.plan, d.total_slots, s, fl, o, i, j, end, sg);
     st |= radial_fixup_sample<true>(B.c, d.plan, d.total_slots, s, fl, o, i, j, end, sg);
     if (d.status && st) atomicOr(&d.status[B.pix_off + i], st);
@@ -332,8 +332,8 @@ BatchSizes sizes_of(const kgeo_ray_params* imgs, int32_t nimg) {
   return z;
 }
 // per slot; a whole wave's slots cover the records' alignment too
-static_assert(1 + kSeriesBlocks * (kThSFields + kRSFields) + 1 <= 4 * kThFields + 4 * kRFields,
-              "the records and the queue's extra item fit the smallest tables");
+static_assert(kSeriesMoreItems + kSeriesBlocks * (kThSFields + kRSFields) + 1 <= 4 * kThFields + 4 * kRFields,
+              "the records and the queue's further items fit the smallest tables");
 
 }  // namespace
 

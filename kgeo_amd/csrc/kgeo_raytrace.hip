@@ -266,7 +266,7 @@ __global__ __launch_bounds__(kPassBlock) void kg_fixup(DevParams p, SampleArgs a
     bool walked;
     unpack_item(q.items[e / kFixupSpan], i, j, walked);
     const int64_t sg = static_cast<int64_t>(e % kFixupSpan);
-    const int64_t end = series_fixup_end(j, p.ngeo, walked);
+    const int64_t end = series_fixup_end(j, p.ngeo, walked, p.c.r_o_inf != 0);
     uint32_t st = theta_fixup_sample<true>(a.plan, p.npix, i, a.gflags[0], a.out, i, j, end, sg);
     st |= radial_fixup_sample<true>(p.c, a.plan, p.npix, i, a.gflags[0], a.out, i, j, end, sg);
     if (a.status && st) atomicOr(&a.status[i], st);
@@ -406,8 +406,8 @@ WsLayout ws_layout(int64_t npix, int64_t ngeo) {
   L.total = off;
   return L;
 }
-static_assert(1 + kSeriesBlocks * (kThSFields + kRSFields) <= 4 * kThFields + 4 * kRFields,
-              "the records and the queue's extra item fit the tables' part of the workspace");
+static_assert(kSeriesMoreItems + kSeriesBlocks * (kThSFields + kRSFields) <= 4 * kThFields + 4 * kRFields,
+              "the records and the queue's further items fit the tables' part of the workspace");
 
 // The kernels always sample t, phi and sigma (as the reference's
 // raytrace_ana does, kerr_raytracing_ana.py:97): the theta pass parks G_phi,
@@ -422,8 +422,9 @@ int require_phi_t(const kgeo_ray_params* p) {
 
 // Sizes one call handles: a fixup item packs the pixel in 32 bits and the
 // sample in 31, and the queue counter is 32-bit (a call queues at most
-// npix * series_items(ngeo) items; the bound leaves out the one item more, whose
-// t and phi alone would take 512 GiB at it).  Larger jobs are split over pixels.
+// npix * series_items(ngeo) items; the bound leaves out the one or two more per
+// pixel: at it the plan, t and phi take more memory than the GPU has).  Larger
+// jobs are split over pixels.
 int size_limit(int64_t npix, int64_t ngeo) {
   if (npix > 0x7fffffffLL) return fail(KGEO_E_ARG, "npix above 2^31 - 1%s (%lld): split the pixels", "", npix);
   if (ngeo > 0x7fffffffLL) return fail(KGEO_E_ARG, "ngeo above 2^31 - 1%s (%lld)", "", ngeo);
@@ -551,8 +552,9 @@ int run_series(const DevParams& d, const SampleArgs& a, void* ws, hipStream_t st
   const unsigned long long fb = (L.qcap * kFixupSpan + kPassBlock - 1) / kPassBlock;
   const dim3 fgrid(static_cast<unsigned>(fb < 4096ull ? fb : 4096ull));
   // block 0 starts from the observer: with further blocks (which take the
-  // last sample) it waits for no head, nor, above MINSPIN, for the radial plan
-  const bool early = nb > 1 && !d.c.minspin;
+  // last sample) it waits for no head, nor, above MINSPIN, for the radial plan;
+  // t and sigma of an observer at infinity start from the second block's head
+  const bool early = nb > 1 && !d.c.minspin && !d.c.r_o_inf;
   auto series = [&](auto kernel, hipStream_t on, int64_t b) {
     hipLaunchKernelGGL(kernel, dim3(np, parts), dim3(kPassBlock), 0, on, d, a, rth, rr, b, nb, q);
     return check_launch("kg_series");
