@@ -103,7 +103,8 @@ void three_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, c
 // The series passes over all pixels, in the kernels' order: heads of both
 // coordinates, the blocks in `parts` parts each, then the fixups of theta and r over one queue.
 // early: block 0 as the plain kernels run it above MINSPIN, reading no radial constant and no record.
-// nfix[0] receives the queue's length (-1 past the kernels' capacity).
+// nfix[0] receives the queue's length (-1 past the kernels' capacity, -2 if a sample is queued
+// twice: the fixup lanes would race for its parked G_phi, G_t).
 template <class T>
 void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, const SampleOut& o, int64_t parts,
                    bool early, uint32_t* st, int64_t* nfix) {
@@ -132,6 +133,16 @@ void series_passes(const RayScalars<T>& c, const double* plan, uint32_t gflags, 
     }
   const size_t cap = static_cast<size_t>(npix) * static_cast<size_t>(series_items(G));
   nfix[0] = items.size() <= cap ? static_cast<int64_t>(items.size()) : -1;
+  std::vector<bool> queued(static_cast<size_t>(npix) * static_cast<size_t>(G), false);
+  for (uint64_t e : items) {
+    int64_t i, j;
+    bool w;
+    unpack_host_item(e, i, j, w);
+    for (const int64_t end = series_fixup_end(j, G, w, c.r_o_inf != 0); j < end; ++j) {
+      if (queued[static_cast<size_t>(j * npix + i)]) nfix[0] = -2;
+      queued[static_cast<size_t>(j * npix + i)] = true;
+    }
+  }
   nfix[1] = nfix[0];
   nfix[2] = 0;
   for (int part = 0; part < 2; ++part)

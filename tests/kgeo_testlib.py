@@ -219,9 +219,11 @@ class Host:
     def raytrace_loops(self, a, r_o, th_o, alpha, beta, ngeo, tau_in=None, chunks=1, passes=3, do_phi_t=1):
         """The kernels' per-pixel sample code on the CPU, with ngeo split into
         `chunks` ranges as the kernels' grid does; adds the status bits.
-        passes=3: the anchor / walk / fixup passes (the kernels' path on the
-        linspace grid; adds the theta and radial fixup-queue lengths and the
-        radial repair items as "nfix"); passes=1: one
+        passes=4: the heads / series / fixup passes (the kernels' path on the
+        linspace grid; adds the fixup queue's length as "nfix"), passes=5 with
+        block 0 early as the plain kernels run it; passes=3: the anchor / walk /
+        fixup passes (the CPU build's second way; "nfix" then holds the theta
+        and radial queue lengths and the radial repair items); passes=1: one
         combined loop per coordinate.  do_phi_t=0 runs the passes without t
         and phi (NULL outputs), which only the CPU build keeps."""
         n = len(alpha)
