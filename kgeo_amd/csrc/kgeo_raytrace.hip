@@ -503,12 +503,13 @@ int wait_planned(hipStream_t st) {
   return KGEO_OK;
 }
 
-// The plan.  Its radial constants are left to the side stream: what follows on
-// the caller's must wait for them (wait_planned) or for a pass that follows
-// them there (run_series' join) before the call returns, whatever becomes of
-// it, since the kernel reads alpha and beta and writes the workspace.
+// The plan.  Its radial constants are left to the side stream; unless joined
+// here, what follows on the caller's must wait for them (wait_planned) or for
+// a pass that follows them there (run_series' join) before the call returns,
+// whatever becomes of it, since the kernel reads alpha and beta and writes the
+// workspace.
 int run_plan(const kgeo_ray_params* p, const double* alpha, const double* beta, int8_t* rclass, int8_t* thclass,
-             int32_t* nmax_eq, double* tau_tot, uint32_t* status, void* ws, hipStream_t st) {
+             int32_t* nmax_eq, double* tau_tot, uint32_t* status, void* ws, hipStream_t st, bool join) {
   DevParams d = make_dev(p, p->ngeo);
   if (d.npix == 0) return KGEO_OK;
   uint32_t* gflags = static_cast<uint32_t*>(ws);
@@ -534,6 +535,8 @@ int run_plan(const kgeo_ray_params* p, const double* alpha, const double* beta, 
   hipLaunchKernelGGL(kg_setup_radial, dim3(nb), dim3(kPassBlock), 0, ss->side, d, alpha, beta, plan);
   rc = check_launch("kg_setup_radial");
   if (hipEventRecord(ss->planned, ss->side) != hipSuccess) rc = fail_msg(KGEO_E_HIP, "plan event failed");
+  else if (join && hipStreamWaitEvent(st, ss->planned, 0) != hipSuccess)
+    rc = fail_msg(KGEO_E_HIP, "wait for the plan failed");
   return rc;
 }
 
@@ -622,12 +625,9 @@ int plan_and_sample(const kgeo_ray_params* p, const double* alpha, const double*
                     const double* tau_in, double* tau, double* t, double* r, double* th, double* ph, double* sig,
                     int8_t* rclass, int8_t* thclass, int32_t* nmax_eq, double* tau_tot, uint32_t* status, void* ws,
                     hipStream_t st) {
-  int rc = run_plan(p, alpha, beta, rclass, thclass, nmax_eq, tau_tot, status, ws, st);
+  int rc = run_plan(p, alpha, beta, rclass, thclass, nmax_eq, tau_tot, status, ws, st, ngeo <= 0);
   if (!rc) rc = run_sample(p, ngeo, tau_in, tau, t, r, th, ph, sig, status, ws, st, true);
-  if (p->npix > 0 && (rc || ngeo <= 0)) {
-    const int wrc = wait_planned(st);
-    if (!rc) rc = wrc;
-  }
+  if (rc && p->npix > 0) (void)wait_planned(st);
   return rc;
 }
 
@@ -668,10 +668,8 @@ int kgeo_plan(const kgeo_ray_params* p, const double* alpha, const double* beta,
               void* stream) {
   int rc = validate(p, alpha, beta, workspace, workspace_bytes, 0);
   if (rc) return rc;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  rc = run_plan(p, alpha, beta, rclass, thclass, nmax_eq, tau_tot, status, workspace, st);
-  const int wrc = p->npix > 0 ? wait_planned(st) : KGEO_OK;
-  return rc ? rc : wrc;
+  return run_plan(p, alpha, beta, rclass, thclass, nmax_eq, tau_tot, status, workspace,
+                  static_cast<hipStream_t>(stream), true);
 }
 
 int kgeo_sample(const kgeo_ray_params* p, const double* tau_in, int64_t ntau, double* tau, double* t, double* r,
