@@ -19,10 +19,10 @@
 //
 // Where the rays are too few to fill the chip, the samples of a block are
 // split into parts, one lane each, which all run the block's expansions up to
-// their own samples' end: the results do not depend on the parts, nor on how
-// many rays are sampled together.  (More blocks instead of parts would run
-// fewer expansions per lane, but more anchors, and would let near-critical
-// rays change by 1e-9 with the number of pixels.)
+// their own samples' end: the results do not depend on the parts.  (More
+// blocks instead of parts would run fewer expansions per lane, but more
+// anchors, and would let near-critical rays change by 1e-9 with the number of
+// pixels.)
 //
 // An expansion covers the samples on both sides of its centre, to which the
 // motion alone is carried first (series_advance).
@@ -30,7 +30,10 @@
 // The lanes of a wave take their steps together (the smallest any lane
 // needs), so a sample index is uniform across the wave and every store is
 // one contiguous row; a lane that would hold the others to steps below
-// 1/kSeriesMinStep of its block leaves the rest of it to the fixup pass.
+// 1/kSeriesMinStep of its block leaves the rest of it to the fixup pass.  So a
+// ray's last bits depend on the 64 rays of its wave: the same neighbours give
+// the same bits for any number of pixels and parts, others (a ragged tail, a
+// crop that moves the tiles) the same samples to the truncation.
 // A queued range ends with its block (series_fixup_end).
 
 #pragma once

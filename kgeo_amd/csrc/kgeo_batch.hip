@@ -230,8 +230,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 __global__ __launch_bounds__(kBlock) void kg_batch_radial_heads(BatchDev d) { batch_heads<false>(d); }
 
 // kg_series (kgeo_raytrace.hip) over all images, two waves per SIMD as there.
-// A survey of 16 images (64 .. 512 pixels a side, 50 .. 400 samples; 58 million
-// samples) takes 7.6 ms, where the walk by addition theorems took 21.
+// A survey of 16 images (64 .. 512 pixels a side, 50 .. 400 samples; 327 million
+// samples, 10.5 GB) takes 7.6 ms, where the walk by addition theorems took 21.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void kg_batch_series(BatchDev d) {
   __shared__ double sl[kBlock / kWave][SERIES_SLOTS][kWave];
   LdsSlots slots{sl[threadIdx.x / kWave], static_cast<int>(threadIdx.x % kWave)};
